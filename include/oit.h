@@ -54,8 +54,8 @@ enum oit_algorithm {
 #define OIT_VARIANT_LL_APPEND_8      0x4u /* Linked List: fused append takes 8 chunks per wave (default 4) */
 #define OIT_VARIANT_LL_KEYS_ONLY     0x8u /* Linked List: resolve keeps sort keys only and reloads colours by node
                                              (always at 32 layers) */
-#define OIT_VARIANT_STORE_CHUNKS_1   0x10u /* Loop64: store one fragment per lane (default: two 64-fragment chunks per wave) */
-#define OIT_VARIANT_STORE_CHUNKS_4   0x20u /* Loop64: store four 64-fragment chunks per wave */
+#define OIT_VARIANT_STORE_CHUNKS_1   0x10u /* accepted, no effect (Loop64 has one schedule) */
+#define OIT_VARIANT_STORE_CHUNKS_4   0x20u /* likewise */
 
 /* Status codes. */
 enum oit_status {
@@ -156,10 +156,8 @@ int oit_clear(oit_ctx* ctx, void* stream);
  * 313-322, 358-368, 384-414) running oitSimple/oitLinkedList/oitLoop64/
  * oitSpinlock/oitWeighted.frag.glsl with PASS == PASS_COLOR. The fragment
  * buffers must stay valid until oit_resolve has been enqueued when the
- * algorithm is OIT_LOOP64 or OIT_LOOP: Loop64 counts each pixel's fragments
- * here and stores them in the resolve, once every append of the frame is
- * counted (a pixel of at most K fragments keeps them all and needs no
- * atomicMin chain); Loop32 runs its second geometry pass there. */
+ * algorithm is OIT_LOOP64 or OIT_LOOP: the append lists the fragments per
+ * tile of 64 targets, and the resolve reads their depths and colours there. */
 int oit_append(oit_ctx* ctx, const oit_fragments* frags, void* stream);
 /* Composite pass: writes the final premultiplied RGBA per target
  * (composite over tail-blended colour buffer over background) to
@@ -231,7 +229,7 @@ const char* oit_status_string(int status);
 /* ---- Stage timing (replaces the reference's per-pass GPU timer sections,
  * e.g. "LinkedListColor" / "LinkedListComposite", oitRender.cpp:223,235).
  * Stages: 0 clear, 1 store (colour pass), 2 link (LL head insertion),
- * 3 classify (Loop64 tail classification), 4 tail link, 5 resolve. ---- */
+ * 3 classify (unused: Loop64 and Loop32 find their tails in the resolve), 4 tail link, 5 resolve. ---- */
 #define OIT_PROFILE_STAGES 6
 typedef struct oit_profile {
   double   ms[OIT_PROFILE_STAGES];

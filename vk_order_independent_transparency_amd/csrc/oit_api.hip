@@ -108,13 +108,17 @@ struct oit_ctx {
   uint32_t* kb_col = nullptr;
   uint32_t* kb_key = nullptr;
   uint32_t* kb_id = nullptr;
-  // Loop64
-  uint64_t* l64 = nullptr;
-  uint32_t* l64_cnt = nullptr;  // [T] the frame's fragments per target (0 = clean)
-  uint64_t* l64_big = nullptr;  // per 64-fragment chunk of the frame: lanes whose pixel holds more than K
-  bool l64_clean = false;  // every slot empty and every count 0 (a fill, or the last frame's composite)
+  // tile path (Loop32, Loop64): runs of fragments per tile of 64 targets
+  uint32_t* tile_cnt = nullptr;
+  uint64_t* tile_run = nullptr;
+  uint32_t* tile_more = nullptr;
+  uint32_t* tile_deep = nullptr;
+  uint32_t* tile_ctl = nullptr;
+  uint64_t* tile_link = nullptr;   // [cap_tile_link] links of the runs past a tile's slots, by first id
+  oit::TileSeg* tile_segs = nullptr;
+  uint64_t cap_tiles = 0, cap_tile_ctl = 0, cap_tile_link = 0, cap_tile_segs = 0;
+  bool tile_clean = false;  // run counts and lists at their clear values (a fill, or the last composite)
   bool kb_clean = false;   // Simple / Spinlock: counts, lock words and bounds at their clear values, likewise
-  bool l32_clean = false;  // Loop32: likewise for the depth and colour slots
   bool wb_clean = false;   // WBOIT: accumulators at the clear values (a fill, or the last composite)
   // WBOIT
   float4* wb_accum = nullptr;
@@ -142,13 +146,11 @@ struct oit_ctx {
   // frame sizes stops allocating once it has seen the largest
   uint64_t cap_ll_head = 0, ll_alloc = 0;
   uint64_t cap_kb_count = 0, cap_kb_lock = 0, cap_kb_depth = 0, cap_kb_filled = 0, cap_kb_elems = 0;
-  uint64_t cap_l64 = 0, cap_l64_cnt = 0, cap_l64_big = 0, cap_wb = 0, cap_tl_head = 0;
+  uint64_t cap_wb = 0, cap_tl_head = 0;
   // coverage shading: sample masks of nodes, k-buffer slots and tail entries
   uint32_t* ll_mask = nullptr;
   float4* il_full = nullptr;   // ordered interlock: shaded colour per node [ll_alloc]
-  uint32_t* l32_z = nullptr;   // Loop32 depth slots [K][T]
-  uint64_t* l32_c = nullptr;   // Loop32 colour slots [K][T]: (id + 1) << 32 | colour
-  uint64_t cap_il_full = 0, cap_l32 = 0;
+  uint64_t cap_il_full = 0;
   uint32_t* kb_mask = nullptr;
   uint32_t* tl_mask = nullptr;
   uint64_t cap_ll_mask = 0, cap_kb_mask = 0, cap_tl_mask = 0;
@@ -243,14 +245,11 @@ void free_frame_buffers(oit_ctx* c) {
   wait_idle(c);
   c->cap_ll_head = c->ll_alloc = 0;
   c->cap_kb_count = c->cap_kb_lock = c->cap_kb_depth = c->cap_kb_filled = c->cap_kb_elems = 0;
-  c->cap_l64 = c->cap_l64_cnt = c->cap_l64_big = c->cap_wb = c->cap_tl_head = 0;
+  c->cap_wb = c->cap_tl_head = 0;
   c->cap_ll_mask = c->cap_kb_mask = c->cap_tl_mask = 0;
   dev_free(&c->ll_mask);
   dev_free(&c->il_full);
-  dev_free(&c->l32_z);
-  dev_free(&c->l32_c);
-  c->l32_clean = false;
-  c->cap_il_full = c->cap_l32 = 0;
+  c->cap_il_full = 0;
   dev_free(&c->kb_mask);
   dev_free(&c->tl_mask);
   dev_free(&c->opq_z);
@@ -267,10 +266,15 @@ void free_frame_buffers(oit_ctx* c) {
   dev_free(&c->kb_col);
   dev_free(&c->kb_key);
   dev_free(&c->kb_id);
-  dev_free(&c->l64);
-  dev_free(&c->l64_cnt);
-  dev_free(&c->l64_big);
-  c->l64_clean = false;
+  dev_free(&c->tile_cnt);
+  dev_free(&c->tile_run);
+  dev_free(&c->tile_more);
+  dev_free(&c->tile_deep);
+  dev_free(&c->tile_ctl);
+  dev_free(&c->tile_link);
+  dev_free(&c->tile_segs);
+  c->cap_tiles = c->cap_tile_ctl = c->cap_tile_link = c->cap_tile_segs = 0;
+  c->tile_clean = false;
   c->kb_clean = false;
   dev_free(&c->wb_accum);
   dev_free(&c->wb_reveal);
@@ -358,9 +362,55 @@ oit::TailBuf tail_of(const oit_ctx* c) {
 // The Linked List and the ordered interlock keep fragments in the node pool.
 bool pooled(uint32_t alg) { return alg == OIT_LINKEDLIST || alg == OIT_INTERLOCK; }
 
-// The ordered interlock blends its tail in the resolve, in primitive order.
+// Loop32 and Loop64 list their fragments per tile of targets.
+bool tiled(uint32_t alg) { return alg == OIT_LOOP || alg == OIT_LOOP64; }
+
+// The ordered interlock blends its tail in the resolve, in primitive order,
+// and the tile path's composite finds the tail in the tile's fragments.
 bool uses_tail_lists(const oit_ctx* c) {
-  return c->cfg.tail_blend && c->cfg.algorithm != OIT_WEIGHTED && c->cfg.algorithm != OIT_INTERLOCK;
+  return c->cfg.tail_blend && c->cfg.algorithm != OIT_WEIGHTED && c->cfg.algorithm != OIT_INTERLOCK &&
+         !tiled(c->cfg.algorithm);
+}
+
+oit::TileBuf tiles_of(const oit_ctx* c) {
+  oit::TileBuf t;
+  t.cnt = c->tile_cnt;
+  t.run = c->tile_run;
+  t.more = c->tile_more;
+  t.link = c->tile_link;
+  t.deep = c->tile_deep;
+  t.ctl = c->tile_ctl;
+  return t;
+}
+
+// Makes the tile path's links hold `need` fragments, keeping this frame's
+// (a stream-ordered copy; the old buffer is freed once the stream has
+// drained). With tail blending, max_fragments bounds a frame as it does for
+// the algorithms that keep tail lists.
+int ensure_tile_link(oit_ctx* c, uint64_t need, hipStream_t s) {
+  if (need <= c->cap_tile_link) return OIT_OK;
+  uint64_t cap = c->cap_tile_link ? c->cap_tile_link : 1024;
+  while (cap < need) cap *= 2;
+  if (c->cfg.tail_blend && c->cfg.max_fragments && cap > c->cfg.max_fragments) cap = c->cfg.max_fragments;
+  if (cap < need) return OIT_ERR_CAPACITY;
+  if (cap > kMaxFrameFragments) cap = kMaxFrameFragments;
+  uint64_t* n = nullptr;
+  const int rc = dev_alloc(&n, cap);
+  if (rc) return rc;
+  hipError_t e = hipSuccess;
+  if (c->frame_frags) {
+    e = hipMemcpyAsync(n, c->tile_link, c->frame_frags * sizeof(uint64_t), hipMemcpyDeviceToDevice, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+  }
+  if (e != hipSuccess) {
+    dev_free(&n);
+    return status_of(e);
+  }
+  wait_idle(c);
+  dev_free(&c->tile_link);
+  c->tile_link = n;
+  c->cap_tile_link = cap;
+  return OIT_OK;
 }
 
 // Makes the per-fragment tail arrays hold `need` fragments, keeping this
@@ -610,16 +660,16 @@ int oit_configure(oit_ctx* c, const oit_config* cfg) {
   }
   if (!pooled(alg)) release(c, &c->ll_mask, &c->cap_ll_mask);
   if (alg != OIT_INTERLOCK) release(c, &c->il_full, &c->cap_il_full);
-  if (alg != OIT_LOOP) {
-    uint64_t d = c->cap_l32;
-    release(c, &c->l32_z, &d);
-    release(c, &c->l32_c, &c->cap_l32);
-  }
   if (alg != OIT_SIMPLE && alg != OIT_SPINLOCK) release(c, &c->kb_mask, &c->cap_kb_mask);
-  if (alg != OIT_LOOP64) {
-    release(c, &c->l64, &c->cap_l64);
-    release(c, &c->l64_cnt, &c->cap_l64_cnt);
-    release(c, &c->l64_big, &c->cap_l64_big);
+  if (!tiled(alg)) {
+    uint64_t d1 = c->cap_tiles, d2 = c->cap_tiles, d3 = c->cap_tiles;
+    release(c, &c->tile_cnt, &d1);
+    release(c, &c->tile_run, &d2);
+    release(c, &c->tile_more, &d3);
+    release(c, &c->tile_deep, &c->cap_tiles);
+    release(c, &c->tile_ctl, &c->cap_tile_ctl);
+    release(c, &c->tile_link, &c->cap_tile_link);
+    release(c, &c->tile_segs, &c->cap_tile_segs);
   }
   if (alg != OIT_WEIGHTED) {
     uint64_t d = c->cap_wb;
@@ -645,16 +695,6 @@ int oit_configure(oit_ctx* c, const oit_config* cfg) {
       c->bytes_aux = T * 4u;
       break;
     }
-    case OIT_LOOP: {  // oit.cpp:127-133: depth and colour planes
-      if (T * K > c->cap_l32) {
-        uint64_t d = c->cap_l32;
-        rc = reserve(c, &c->l32_z, &d, T * K);
-        if (!rc) rc = reserve(c, &c->l32_c, &c->cap_l32, T * K);
-      }
-      c->bytes_abuf = T * K * 12u;
-      c->bytes_aux = 0;
-      break;
-    }
     case OIT_SIMPLE:
     case OIT_SPINLOCK: {  // oit.cpp:102-118 (the Spinlock's count lives in its lock word)
       if (alg == OIT_SIMPLE) rc = reserve(c, &c->kb_count, &c->cap_kb_count, T);
@@ -674,11 +714,22 @@ int oit_configure(oit_ctx* c, const oit_config* cfg) {
       c->bytes_aux = T * (alg == OIT_SPINLOCK ? 12u : 4u);
       break;
     }
-    case OIT_LOOP64: {  // oit.cpp:134-140
-      rc = reserve(c, &c->l64, &c->cap_l64, T * K);
-      if (!rc) rc = reserve(c, &c->l64_cnt, &c->cap_l64_cnt, T);
-      c->bytes_abuf = T * K * 8u;
-      c->bytes_aux = T * 4u;
+    case OIT_LOOP:
+    case OIT_LOOP64: {  // in place of the slot planes of oit.cpp:127-140: runs of fragments per tile
+      const uint64_t tiles = oit::tile_count(T);
+      if (tiles > c->cap_tiles) {
+        uint64_t d1 = c->cap_tiles, d2 = c->cap_tiles * oit::kTileRuns, d3 = d2;
+        rc = reserve(c, &c->tile_cnt, &d1, tiles);
+        if (!rc) rc = reserve(c, &c->tile_run, &d2, tiles * oit::kTileRuns);
+        if (!rc) rc = reserve(c, &c->tile_more, &d3, tiles * oit::kTileRuns);
+        if (!rc) rc = reserve(c, &c->tile_deep, &c->cap_tiles, tiles);
+      }
+      if (!rc) rc = reserve(c, &c->tile_ctl, &c->cap_tile_ctl, oit::kTileCtlAll);
+      if (!rc && cfg->tail_blend && cfg->max_fragments)
+        rc = reserve(c, &c->tile_link, &c->cap_tile_link,
+                     cfg->max_fragments < kMaxFrameFragments ? cfg->max_fragments : kMaxFrameFragments);
+      c->bytes_abuf = tiles * oit::kTileRuns * 12u;
+      c->bytes_aux = tiles * 8u;
       break;
     }
     case OIT_WEIGHTED: {  // oit.h:234-235 (binary32 here)
@@ -721,8 +772,7 @@ int oit_configure(oit_ctx* c, const oit_config* cfg) {
   }
   c->tl_head_valid = false;
   c->tl_clean = false;
-  c->l64_clean = false;  // slots beyond the last frame's T x K may hold an older frame's keys
-  c->l32_clean = false;
+  c->tile_clean = false;
   c->wb_clean = false;
   c->kb_clean = false;
   if (pooled(alg) && ll_grown) {
@@ -763,7 +813,7 @@ int oit_query_sizes(const oit_ctx* c, oit_sizes* out) {
   std::memset(out, 0, sizeof *out);
   out->abuffer_bytes = c->bytes_abuf;
   out->aux_bytes = c->bytes_aux + (c->tl_head ? (uint64_t)c->T * 4u : 0u);
-  out->tail_bytes = (uint64_t)c->tl_cap * (4u + 16u + 8u) + oit::tail_regions(c->tl_cap) * 4u;
+  out->tail_bytes = (uint64_t)c->tl_cap * (4u + 16u + 8u) + oit::tail_regions(c->tl_cap) * 4u + c->cap_tile_link * 8u;
   out->total_bytes = out->abuffer_bytes + out->aux_bytes + out->tail_bytes;
   out->ll_capacity = c->ll_cap;
   switch (c->cfg.algorithm) {
@@ -777,10 +827,12 @@ int oit_query_sizes(const oit_ctx* c, oit_sizes* out) {
   }
   out->targets = c->T;
   out->resident_bytes = c->cap_ll_head * 4u + c->ll_alloc * 12u + c->cap_kb_count * 4u + c->cap_kb_lock * 4u +
-                        c->cap_kb_depth * 4u + c->cap_kb_filled * 4u + c->cap_kb_elems * 12u + c->cap_l64 * 8u + c->cap_l64_cnt * 4u + c->cap_l64_big * 8u + c->cap_wb * 20u +
+                        c->cap_kb_depth * 4u + c->cap_kb_filled * 4u + c->cap_kb_elems * 12u +
+                        c->cap_tiles * (8u + oit::kTileRuns * 12u) + c->cap_tile_ctl * 4u + c->cap_tile_link * 8u +
+                        c->cap_tile_segs * sizeof(oit::TileSeg) + c->cap_wb * 20u +
                         c->cap_tl_head * 4u + (uint64_t)c->tl_cap * (4u + 16u + 8u) + oit::tail_regions(c->tl_cap) * 4u +
                         (c->cap_ll_mask + c->cap_kb_mask + c->cap_tl_mask) * 4u + c->cap_il_full * 16u +
-                        c->cap_l32 * 12u + c->cap_opq * 8u + c->cap_opq_rgba * 16u;
+                        c->cap_opq * 8u + c->cap_opq_rgba * 16u;
   return OIT_OK;
 }
 
@@ -789,7 +841,7 @@ int oit_clear(oit_ctx* c, void* stream) {
   if (!c->configured) return OIT_ERR_STATE;
   DeviceGuard g(c->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const uint64_t T = c->T, K = c->cfg.layers;
+  const uint64_t T = c->T;
   const bool ll = pooled(c->cfg.algorithm);
   const bool need_ll_fill = ll && !c->ll_clean;
   // only the Linked List's kernels write the frame counters (its resolve
@@ -808,15 +860,8 @@ int oit_clear(oit_ctx* c, void* stream) {
   int nf = 0;
   auto fill = [&](void* p, uint64_t n, uint32_t v) { fr[nf++] = oit::FillRange{static_cast<uint32_t*>(p), n, v}; };
   if (need_counters) fill(c->d_counters, 16, 0u);
-  bool l64_fill = false, l32_fill = false, wb_fill = false, kb_fill = false;
+  bool tile_fill = false, wb_fill = false, kb_fill = false;
   switch (c->cfg.algorithm) {
-    case OIT_LOOP:  // depths to all ones (oitRender.cpp:242-265), colour slots to 0; the composite leaves them so
-      l32_fill = !c->l32_clean;
-      if (l32_fill) {
-        fill(c->l32_z, T * K, kEmpty);
-        fill(c->l32_c, 2 * T * K, 0u);
-      }
-      break;
     case OIT_INTERLOCK:
     case OIT_LINKEDLIST:  // head and counter to 0, oitRender.cpp:206-212; links of a dirty range to kUnset
       // every allocated head: a larger earlier frame may have left some
@@ -837,11 +882,13 @@ int oit_clear(oit_ctx* c, void* stream) {
         fill(c->kb_filled, T, 0u);
       }
       break;
-    case OIT_LOOP64:  // every byte to 0xFF, oitRender.cpp:307; the composite leaves its slots empty
-      l64_fill = !c->l64_clean;
-      if (l64_fill) {
-        fill(c->l64, 2 * T * K, kEmpty);
-        fill(c->l64_cnt, T, 0u);
+    case OIT_LOOP:
+    case OIT_LOOP64:  // no runs (the slot clears of oitRender.cpp:242-265,307); the composite leaves it so
+      tile_fill = !c->tile_clean;
+      if (tile_fill) {
+        fill(c->tile_cnt, oit::tile_count(T), 0u);
+        fill(c->tile_more, oit::tile_count(T) * oit::kTileRuns, 0u);
+        fill(c->tile_ctl + oit::kTileShares, oit::kSharedTiles, 0u);
       }
       break;
     case OIT_WEIGHTED:  // accum 0, reveal 1 (log2 0), oitRender.cpp:394-397; the composite leaves them so
@@ -858,8 +905,7 @@ int oit_clear(oit_ctx* c, void* stream) {
   }
   hipError_t e = hipSuccess;
   if (nf > 0) e = staged(c, kStClear, s, [&]() -> hipError_t { return oit::launch_fill_ranges(fr, nf, s); });
-  if (e == hipSuccess && l64_fill) c->l64_clean = true;
-  if (e == hipSuccess && l32_fill) c->l32_clean = true;
+  if (e == hipSuccess && tile_fill) c->tile_clean = true;
   if (e == hipSuccess && wb_fill) c->wb_clean = true;
   if (e == hipSuccess && kb_fill) c->kb_clean = true;
   if (e == hipSuccess) c->counters_clean = true;
@@ -982,9 +1028,17 @@ int oit_append(oit_ctx* c, const oit_fragments* f, void* stream) {
       e = staged(c, kStStore, s, [&] { return oit::launch_ll_append(k, v, ll, none, 4, s); });
       break;
     }
-    case OIT_LOOP: {  // depth pass now; the colour pass runs over the recorded batches at resolve
-      c->l32_clean = false;
-      e = staged(c, kStStore, s, [&] { return oit::launch_loop32_depth(k, v, c->l32_z, s); });
+    case OIT_LOOP:
+    case OIT_LOOP64: {  // runs per tile now; the composite reads the recorded batches at resolve
+      int rc = ensure_tile_link(c, end, s);
+      if (!rc && !c->segments.empty()) {
+        uint64_t want = c->cap_tile_segs ? c->cap_tile_segs : oit::kSegArgs;
+        while (want < c->segments.size() + 1) want *= 2;
+        rc = reserve(c, &c->tile_segs, &c->cap_tile_segs, want);
+      }
+      if (rc) return rc;
+      c->tile_clean = false;
+      e = staged(c, kStStore, s, [&] { return oit::launch_tile_link(k, v, tiles_of(c), s); });
       c->segments.push_back(v);
       break;
     }
@@ -1003,12 +1057,6 @@ int oit_append(oit_ctx* c, const oit_fragments* f, void* stream) {
       kb.filled = c->kb_filled;
       kb.mask = coverage(c) ? c->kb_mask : nullptr;
       e = staged(c, kStStore, s, [&] { return oit::launch_spin_store(k, v, kb, tb, s); });
-      break;
-    }
-    case OIT_LOOP64: {  // counted now; stored at resolve, once every pixel's count is known
-      c->l64_clean = false;
-      e = staged(c, kStStore, s, [&] { return oit::launch_loop64_count(k, v, c->l64_cnt, s); });
-      c->segments.push_back(v);
       break;
     }
     case OIT_WEIGHTED: {
@@ -1036,52 +1084,15 @@ int oit_resolve_debug(oit_ctx* c, float* out_rgba, uint32_t* fk_key, uint32_t* f
   hipStream_t s = static_cast<hipStream_t>(stream);
   const uint32_t alg = c->cfg.algorithm;
   const bool link_tails = !c->resolved;
-  if (link_tails && alg == OIT_LOOP64 && c->cfg.tail_blend && !c->segments.empty()) {
-    int rc = ensure_tail_capacity(c, c->frame_frags, s);
-    if (rc) return rc;
-    c->tl_clean = false;  // the classification pushes tail fragments
-  }
   const oit::Common k = common_of(c);
   const oit::TailBuf tb = tail_of(c);
   oit::ResolveOut o{reinterpret_cast<float4*>(out_rgba), fk_key, fk_val, counts};
   hipError_t e = hipSuccess;
-  if (link_tails && alg == OIT_LOOP64 && !c->segments.empty()) {  // the stores of every segment (counted at append)
-    const int chunks = (c->cfg.variant & OIT_VARIANT_STORE_CHUNKS_1) ? 1
-                       : (c->cfg.variant & OIT_VARIANT_STORE_CHUNKS_4) ? 4 : 2;
-    uint64_t masks = 0;  // one per 64-fragment chunk of each segment
-    for (const auto& v : c->segments) masks += (v.count + 63u) / 64u;
-    int rc = reserve(c, &c->l64_big, &c->cap_l64_big, masks ? masks : 1);
-    if (rc) return rc;
-    uint64_t m0 = 0;
-    for (const auto& v : c->segments) {
-      uint64_t* big = c->l64_big + m0;
-      e = staged(c, kStStore, s, [&] { return oit::launch_loop64_store(k, v, c->l64, c->l64_cnt, big, chunks, s); });
-      if (e != hipSuccess) return status_of(e);
-      m0 += (v.count + 63u) / 64u;
-    }
-    if (c->cfg.tail_blend && tb.head) {
-      m0 = 0;
-      for (const auto& v : c->segments) {
-        const uint64_t* big = c->l64_big + m0;
-        e = staged(c, kStClassify, s, [&] { return oit::launch_loop64_classify(k, v, c->l64, big, tb, s); });
-        if (e != hipSuccess) return status_of(e);
-        m0 += (v.count + 63u) / 64u;
-      }
-    }
-  }
-  if (link_tails && alg == OIT_LOOP) {  // the second geometry pass (oitLoop.frag.glsl:105-180)
-    for (const auto& v : c->segments) {
-      e = staged(c, kStClassify, s, [&] { return oit::launch_loop32_color(k, v, c->l32_z, c->l32_c, tb, s); });
-      if (e != hipSuccess) return status_of(e);
-    }
-  }
   // Linked List: only fragments whose node would be at or past the pool's
   // end (id >= cap - 1) can be tails
   const uint64_t first_tail = alg == OIT_LINKEDLIST ? (c->ll_cap ? c->ll_cap - 1 : 0) : 0;
   const bool no_tails = !tb.next || first_tail >= c->frame_frags;
-  // Loop64's classification, which runs after every store, links its tail
-  // fragments itself; the other algorithms queue them for this pass
-  if (link_tails && tb.head && !no_tails && alg != OIT_LOOP64) {
+  if (link_tails && tb.head && !no_tails) {
     e = staged(c, kStTailLink, s, [&] {
       return oit::launch_tail_link(tb, (uint32_t)first_tail, (uint32_t)c->frame_frags, s);
     });
@@ -1126,14 +1137,38 @@ int oit_resolve_debug(oit_ctx* c, float* out_rgba, uint32_t* fk_key, uint32_t* f
       c->kb_clean = e == hipSuccess;  // the composite set every word it read back to its clear value
       break;
     }
-    case OIT_LOOP64:
-      e = staged(c, kStResolve, s, [&] { return oit::launch_loop64_resolve(k, c->l64, c->l64_cnt, tbr, o, s); });
-      c->l64_clean = e == hipSuccess;  // the composite emptied every slot it read
-      break;
     case OIT_LOOP:
-      e = staged(c, kStResolve, s, [&] { return oit::launch_loop32_resolve(k, c->l32_z, c->l32_c, tbr, o, s); });
-      c->l32_clean = e == hipSuccess;  // the composite emptied every slot it read
+    case OIT_LOOP64: {
+      oit::TileSrc src;
+      src.T = c->T;
+      src.spp = k.spp;
+      src.frags = c->frame_frags;
+      std::vector<oit::TileSeg> segs;
+      for (const auto& v : c->segments) segs.push_back({v.target, v.depth, v.rgba, v.id_base, 0u});
+      if (!segs.empty()) src.one = segs[0];
+      if (segs.size() > 1) {
+        src.nseg = (uint32_t)segs.size();
+        src.segs = c->tile_segs;
+        e = oit::launch_set_segs(segs.data(), src.nseg, c->tile_segs, s);
+        if (e != hipSuccess) return status_of(e);
+      }
+      oit::TileDst dst;
+      dst.out = o.out;
+      dst.fk_key = o.fk_key;
+      dst.fk_val = o.fk_val;
+      dst.counts = o.counts;
+      dst.T = c->T;
+      dst.spp = k.spp;
+      dst.background = k.background;
+      dst.rgba = k.opq_rgba;
+      dst.tab = k.tab;
+      const int mode = alg == OIT_LOOP ? oit::kTileLoop32 : oit::kTileLoop64;
+      e = staged(c, kStResolve, s, [&] {
+        return oit::launch_tile_resolve(tiles_of(c), src, dst, k.K, mode, c->cfg.tail_blend != 0, s);
+      });
+      c->tile_clean = e == hipSuccess;  // the composite took every run it listed
       break;
+    }
     case OIT_INTERLOCK: {
       oit::LLBuf ll{c->ll_head, c->ll_cd, c->ll_next, c->ll_cap, c->d_counters + 1, c->d_counters};
       ll.err = dev_err(c);
@@ -1195,6 +1230,13 @@ int oit_get_stats(oit_ctx* c, oit_stats* out, void* stream) {
       return OIT_ERR_DEVICE;
     for (uint32_t v : rg) tails += v;
   }
+  if (tiled(c->cfg.algorithm) && c->tile_ctl && c->appends > 0 && c->resolved) {  // counted by the composite
+    uint32_t tw[oit::kTileTailWords];
+    if (hipMemcpyAsync(tw, c->tile_ctl + oit::kTileTails, sizeof tw, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+      return OIT_ERR_DEVICE;
+    for (uint32_t v : tw) tails += v;
+  }
   std::memset(out, 0, sizeof *out);
   out->fragments = c->frame_frags;
   out->ll_overflow = h[1];
@@ -1209,8 +1251,7 @@ int oit_get_stats(oit_ctx* c, oit_stats* out, void* stream) {
     c->ll_clean = false;
     c->ll_dirty_upto = c->ll_alloc;
     c->counters_clean = false;
-    c->l64_clean = false;
-    c->l32_clean = false;
+    c->tile_clean = false;
     c->wb_clean = false;
     c->kb_clean = false;
     c->tl_clean = false;

@@ -5,631 +5,11 @@
 //
 // Built with: hipcc --offload-arch=gfx950 -O3 -ffp-contract=off
 //             -Xclang -target-feature -Xclang -packed-fp32-ops
-#include "oit_kernels.hpp"
+#include "oit_frame.hpp"
 
 namespace oit {
 
 namespace {
-
-constexpr uint32_t kBlock = 256;
-
-inline uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
-
-// A run of consecutive lanes that carry the same target. Fragment ids grow
-// with the lane, so a run is a block of consecutive ids of one target, and
-// no fragment outside the wave can have an id inside it.
-struct Run {
-  uint32_t lane;
-  uint32_t start_lane;
-  uint32_t end_lane;
-  bool start;
-  bool end;
-};
-
-// Must be reached by all 64 lanes (callers keep every lane alive and give
-// lanes without a fragment a target of kEmpty).
-__device__ __forceinline__ Run same_target_run(uint32_t t) {
-  Run r;
-  r.lane = lane_id();
-  const uint32_t tp = __shfl_up(t, 1u);
-  const uint32_t tn = __shfl_down(t, 1u);
-  r.start = (r.lane == 0) || (tp != t);
-  r.end = (r.lane == 63) || (tn != t);
-  const uint64_t starts = __ballot(r.start);
-  const uint64_t ends = __ballot(r.end);
-  const uint64_t le = (2ull << r.lane) - 1ull;  // lanes <= this lane
-  r.start_lane = 63u - (uint32_t)__builtin_clzll(starts & le);
-  r.end_lane = r.lane + (uint32_t)__builtin_ctzll(ends >> r.lane);
-  return r;
-}
-
-// Colour-pass tail list value of frame-local fragment lid: ((lid + 1) << 1)
-// | boundary flag, so that 0 can terminate the lists; its link word is
-// next[lid]. Values order as ids do.
-__device__ __forceinline__ uint32_t tail_value(uint32_t lid, uint32_t flag) { return ((lid + 1u) << 1) | flag; }
-__device__ __forceinline__ uint32_t tail_index(uint32_t v) { return (v >> 1) - 1u; }
-// values below this have link words in arrays of `cap` fragments
-__device__ __forceinline__ uint32_t tail_value_cap(uint32_t cap) { return (cap + 1u) << 1; }
-
-// Colour-pass tail lists, phase 1: a tail fragment `lid` stores its
-// premultiplied colour at index lid, and its record (target << 32) | tail
-// value goes to the frame's tail queue. The queue is cut into regions of
-// 1024 fragment ids, each with its own counter, and a record goes to the
-// region of its fragment's id: a fragment enters the tail once, so region
-// r's entries fit in rec[r * 1024 ..]. The lanes of one region share one
-// returning atomic, so a wave waits for one round trip however many tail
-// fragments it finds. The queue holds only tail fragments, so the link pass
-// reads nothing of the others. Called by every active lane of the wave that
-// may hold a tail fragment.
-__device__ __forceinline__ void tail_queue_push(bool tail, uint32_t t, uint32_t lid, uint32_t flag, float4 payload,
-                                                const TailBuf& tb, uint32_t mask) {
-  tail = tail && lid < tb.cap && tb.qn != nullptr;
-  if (tail) {
-    tb.rgba[lid] = payload;
-    if (tb.mask) tb.mask[lid] = mask;
-  }
-  const uint32_t r = lid >> kTailRegionShift;
-  const uint32_t lane = lane_id();
-  // group the lanes by region (cross-lane work only), then one atomic per
-  // group, all of them in flight together
-  uint64_t rem = __ballot(tail);
-  uint32_t my_leader = 0;
-  uint64_t my_group = 0;
-  while (rem) {
-    const uint32_t leader = (uint32_t)__builtin_ctzll(rem);
-    const uint32_t rl = __builtin_amdgcn_readlane(r, leader);
-    const uint64_t m = __ballot(tail && r == rl);
-    if ((m >> lane) & 1ull) {
-      my_leader = leader;
-      my_group = m;
-    }
-    rem &= ~m;
-  }
-  uint32_t q = 0;
-  if (tail && lane == my_leader) q = atomicAdd(&tb.qn[r], (uint32_t)__builtin_popcountll(my_group));
-  q = __shfl(q, (int)my_leader);
-  if (tail)
-    tb.rec[((uint64_t)r << kTailRegionShift) + q + lanes_below(my_group)] = ((uint64_t)t << 32) | tail_value(lid, flag);
-}
-
-// tail_queue_push over kU chunks of a wave (chunk u: tail[u], t[u], lid[u],
-// payload[u]; no boundary flag, full coverage), with every chunk's region
-// counter atomics in flight together: the wave waits one round trip for all
-// of them. Must be reached by all 64 lanes.
-template <int kU>
-__device__ __forceinline__ void tail_queue_push_n(const bool (&tail_in)[kU], const uint32_t (&t)[kU],
-                                                  const uint32_t (&lid)[kU], const float4 (&payload)[kU],
-                                                  const TailBuf& tb) {
-  const uint32_t lane = lane_id();
-  bool tail[kU];
-  uint32_t r[kU], leader[kU], q[kU];
-  uint64_t group[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    tail[u] = tail_in[u] && lid[u] < tb.cap && tb.qn != nullptr;
-    if (tail[u]) {
-      tb.rgba[lid[u]] = payload[u];
-      if (tb.mask) tb.mask[lid[u]] = 0xFFFFFFFFu;
-    }
-    r[u] = lid[u] >> kTailRegionShift;
-    // group the lanes by region (cross-lane work only)
-    uint64_t rem = __ballot(tail[u]);
-    leader[u] = 0;
-    group[u] = 0;
-    while (rem) {
-      const uint32_t l = (uint32_t)__builtin_ctzll(rem);
-      const uint32_t rl = __builtin_amdgcn_readlane(r[u], l);
-      const uint64_t m = __ballot(tail[u] && r[u] == rl);
-      if ((m >> lane) & 1ull) {
-        leader[u] = l;
-        group[u] = m;
-      }
-      rem &= ~m;
-    }
-    q[u] = 0u;
-    asm volatile("" : "+v"(q[u]));  // the zeros are written before any atomic goes out
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u)
-    if (tail[u] && lane == leader[u]) q[u] = atomicAdd(&tb.qn[r[u]], (uint32_t)__builtin_popcountll(group[u]));
-  returns_done();
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const uint32_t base = __shfl(q[u], (int)leader[u]);
-    if (tail[u])
-      tb.rec[((uint64_t)r[u] << kTailRegionShift) + base + lanes_below(group[u])] =
-          ((uint64_t)t[u] << 32) | tail_value(lid[u], 0u);
-  }
-}
-
-// A converged wave's tail fragments straight onto their targets' lists,
-// for a pass that runs after every fragment of the frame is stored (no link
-// pass follows), over kU chunks of the wave (chunk u: tail[u], t[u], lid[u],
-// ...): neighbouring lanes of one target are chained in the wave and
-// published with one exchange on the list head (k_tail_link does the same
-// for queued records), every chunk's exchanges in flight together; each
-// chunk's count goes to its region's counter, which the queue would
-// otherwise have filled. Must be reached by all 64 lanes (lanes without a
-// tail fragment pass tail = false).
-template <int kU>
-__device__ __forceinline__ void tail_list_push_n(const bool (&tail)[kU], const uint32_t (&t)[kU],
-                                                 const uint32_t (&lid)[kU], const uint32_t (&flag)[kU],
-                                                 const float4 (&payload)[kU], const TailBuf& tb) {
-  const uint32_t lane = lane_id();
-  bool ex[kU];
-  uint32_t lo[kU], old[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const bool tl = tail[u] && lid[u] < tb.cap;
-    if (tl) {
-      tb.rgba[lid[u]] = payload[u];
-      if (tb.mask) tb.mask[lid[u]] = 0xFFFFFFFFu;
-    }
-    const uint32_t v = tail_value(lid[u], flag[u]);
-    const Run r = same_target_run(tl ? t[u] : kEmpty);
-    const uint32_t v_prev = __shfl_up(v, 1u);
-    lo[u] = __shfl(v, (int)r.start_lane);
-    if (tl && !r.start) st_relaxed(&tb.next[lid[u]], v_prev);
-    ex[u] = tl && r.end;
-    const uint64_t m = __ballot(tl);
-    if (m != 0ull && lane == (uint32_t)__builtin_ctzll(m))
-      atomicAdd(&tb.qn[lid[u] >> kTailRegionShift], (uint32_t)__builtin_popcountll(m));
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    old[u] = 0u;
-    asm volatile("" : "+v"(old[u]));  // the zeros are written before any exchange goes out
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u)
-    if (ex[u]) old[u] = __hip_atomic_exchange(&tb.head[t[u]], tail_value(lid[u], flag[u]), __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-  returns_done();
-#pragma unroll
-  for (int u = 0; u < kU; ++u)
-    if (ex[u]) st_relaxed(&tb.next[tail_index(lo[u])], old[u]);
-}
-
-// Sorted register array of K (sort key, colour) pairs, ascending; inserting x
-// returns the element pushed out of the back (x itself if it does not fit):
-// insertionSortTail, oitCompositeDefines.glsl:116-139, unrolled into selects.
-template <int K>
-struct FrontK {
-  uint64_t sk[K];
-  uint32_t col[K];
-  __device__ __forceinline__ void init() {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      sk[k] = kEmpty64;
-      col[k] = 0u;
-    }
-  }
-  __device__ __forceinline__ void insert(uint64_t x, uint32_t xc, uint64_t& ev, uint32_t& evc) {
-    const bool fits = x < sk[K - 1];
-    ev = fits ? sk[K - 1] : x;
-    evc = fits ? col[K - 1] : xc;
-#pragma unroll
-    for (int j = K - 1; j > 0; --j) {
-      const bool before = x < sk[j - 1];
-      const bool here = x < sk[j];
-      sk[j] = before ? sk[j - 1] : (here ? x : sk[j]);
-      col[j] = before ? col[j - 1] : (here ? xc : col[j]);
-    }
-    const bool first = x < sk[0];
-    sk[0] = first ? x : sk[0];
-    col[0] = first ? xc : col[0];
-  }
-  // The same insert when at most w - 1 slots can be occupied (w is wave
-  // uniform): slots at and beyond w hold the +inf sentinel before and after
-  // the insert, so whole blocks of four slots at or beyond w are skipped
-  // with one scalar branch each (executing more slots is also exact).
-  __device__ __forceinline__ void insert_bounded(uint64_t x, uint32_t xc, uint64_t& ev, uint32_t& evc, int w) {
-    const bool fits = x < sk[K - 1];
-    ev = fits ? sk[K - 1] : x;
-    evc = fits ? col[K - 1] : xc;
-#pragma unroll
-    for (int b = ((K - 1) / 4) * 4; b >= 0; b -= 4) {
-      if (b < w) {
-#pragma unroll
-        for (int j = (b + 3 < K - 1 ? b + 3 : K - 1); j >= b && j > 0; --j) {
-          const bool before = x < sk[j - 1];
-          const bool here = x < sk[j];
-          sk[j] = before ? sk[j - 1] : (here ? x : sk[j]);
-          col[j] = before ? col[j - 1] : (here ? xc : col[j]);
-        }
-      }
-    }
-    const bool first = x < sk[0];
-    sk[0] = first ? x : sk[0];
-    col[0] = first ? xc : col[0];
-  }
-};
-
-// FrontK with a third payload moved alongside (the ordered interlock's sample
-// masks under coverage shading); the same bounded insert.
-template <int K>
-struct FrontKM {
-  uint64_t sk[K];
-  uint32_t col[K];
-  uint32_t msk[K];
-  __device__ __forceinline__ void init() {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      sk[k] = kEmpty64;
-      col[k] = 0u;
-      msk[k] = 0u;
-    }
-  }
-  __device__ __forceinline__ void insert_bounded(uint64_t x, uint32_t xc, uint32_t xm, uint64_t& ev, uint32_t& evc,
-                                                 int w) {
-    const bool fits = x < sk[K - 1];
-    ev = fits ? sk[K - 1] : x;
-    evc = fits ? col[K - 1] : xc;
-#pragma unroll
-    for (int b = ((K - 1) / 4) * 4; b >= 0; b -= 4) {
-      if (b < w) {
-#pragma unroll
-        for (int j = (b + 3 < K - 1 ? b + 3 : K - 1); j >= b && j > 0; --j) {
-          const bool before = x < sk[j - 1];
-          const bool here = x < sk[j];
-          sk[j] = before ? sk[j - 1] : (here ? x : sk[j]);
-          col[j] = before ? col[j - 1] : (here ? xc : col[j]);
-          msk[j] = before ? msk[j - 1] : (here ? xm : msk[j]);
-        }
-      }
-    }
-    const bool first = x < sk[0];
-    sk[0] = first ? x : sk[0];
-    col[0] = first ? xc : col[0];
-    msk[0] = first ? xm : msk[0];
-  }
-};
-
-// Sorted register array of K sort keys only (depth key << 32 | node index),
-// ascending: the colours are reloaded by node index after the walk, which
-// keeps one third fewer registers live during the latency-bound walk.
-template <int K>
-struct FrontKeys {
-  uint64_t sk[K];
-  __device__ __forceinline__ void init() {
-#pragma unroll
-    for (int k = 0; k < K; ++k) sk[k] = kEmpty64;
-  }
-  // insertionSortTail with a wave-uniform bound w on the occupied slots + 1
-  __device__ __forceinline__ uint64_t insert_bounded(uint64_t x, int w) {
-    const uint64_t ev = x < sk[K - 1] ? sk[K - 1] : x;
-#pragma unroll
-    for (int b = ((K - 1) / 4) * 4; b >= 0; b -= 4) {
-      if (b < w) {
-#pragma unroll
-        for (int j = (b + 3 < K - 1 ? b + 3 : K - 1); j >= b && j > 0; --j) {
-          const bool before = x < sk[j - 1];
-          const bool here = x < sk[j];
-          sk[j] = before ? sk[j - 1] : (here ? x : sk[j]);
-        }
-      }
-    }
-    sk[0] = x < sk[0] ? x : sk[0];
-    return ev;
-  }
-};
-
-// Largest value of v over the active lanes, as a wave-uniform (scalar) value.
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint32_t w = __shfl_xor(v, o);
-    v = w > v ? w : v;
-  }
-  return __builtin_amdgcn_readfirstlane(v);
-}
-
-// Front-to-back blend of the first n sorted packed colours
-// (oitLinkedList.frag.glsl:162-166, oitSimple.frag.glsl:161-165).
-template <int K>
-__device__ __forceinline__ float4 blend_front(const FrontK<K>& a, uint32_t n, const CodecTables* tab) {
-  float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-    if ((uint32_t)k < n) c = over(c, decode_premult(a.col[k], tab));
-  return c;
-}
-
-// Tail values held in registers per walk of an unordered tail list, and
-// the walks a fold takes before it sorts a longer list instead. At 1080p
-// with K = 8 the longest tail is 14 (1 % of the tails need a second walk);
-// a window of 16 cost the K = 8 composites two to three waves per SIMD.
-constexpr int kTailWindow = 8;
-constexpr uint32_t kTailWalks = 4;
-
-// One walk of an unordered tail list: the kTailWindow largest values below
-// `bound`, in descending order (0 = none), by an insertion network in
-// registers; returns how many values of the list lie below `bound`, and in
-// `flagged` the number of boundary-flagged values of the whole list. A walk
-// longer than the arrays hold (a cycle) reports kErrWalk and sets `bad`.
-__device__ __forceinline__ uint32_t tail_window(const TailBuf& tb, uint32_t head, uint32_t vcap, uint32_t bound,
-                                                uint32_t (&w)[kTailWindow], uint32_t& flagged, bool& bad) {
-#pragma unroll
-  for (int k = 0; k < kTailWindow; ++k) w[k] = 0u;
-  uint32_t n = 0, fl = 0, hops = 0;
-  uint32_t v = head;
-  while (v != 0u && v < vcap) {  // a link outside the arrays ends the walk
-    if (++hops > tb.cap) {
-      report_error(tb.err, kErrWalk);
-      bad = true;
-      break;
-    }
-    const uint32_t nx = tb.next[tail_index(v)];
-    fl += v & 1u;
-    if (v < bound) {
-      ++n;
-      uint32_t x = v;
-#pragma unroll
-      for (int k = 0; k < kTailWindow; ++k) {
-        const uint32_t hi = w[k] > x ? w[k] : x;
-        x = w[k] > x ? x : w[k];
-        w[k] = hi;
-      }
-    }
-    v = nx;
-  }
-  flagged = fl;
-  return n;
-}
-
-// A tail list longer than kTailWindow * kTailWalks, sorted into descending
-// order in place: a bottom-up merge sort of the singly linked list (runs of
-// 1, 2, 4, ... merged pass by pass, each pass relinking every node once),
-// O(n log n) link reads instead of one walk per window. The list is the
-// composite lane's own and acyclic (tail_window walked it to its end first);
-// a link at or above vcap ends it. Returns the new head.
-__device__ __forceinline__ uint32_t tail_sort_desc(const TailBuf& tb, uint32_t head, uint32_t vcap) {
-  auto nxt = [&](uint32_t v) -> uint32_t {
-    const uint32_t x = tb.next[tail_index(v)];
-    return x < vcap ? x : 0u;
-  };
-  for (uint32_t run = 1;; run <<= 1) {
-    uint32_t p = head, out = 0u, last = 0u, merges = 0u;
-    while (p != 0u) {
-      ++merges;
-      uint32_t q = p, np = 0u;
-      while (np < run && q != 0u) {
-        ++np;
-        q = nxt(q);
-      }
-      uint32_t nq = run;
-      while (np > 0u || (nq > 0u && q != 0u)) {
-        uint32_t e;
-        if (np == 0u || (nq > 0u && q != 0u && q > p)) {  // descending: the larger value first
-          e = q;
-          q = nxt(q);
-          --nq;
-        } else {
-          e = p;
-          p = nxt(p);
-          --np;
-        }
-        if (last == 0u) out = e;
-        else tb.next[tail_index(last)] = e;
-        last = e;
-      }
-      p = q;
-    }
-    if (last != 0u) tb.next[tail_index(last)] = 0u;
-    head = out;
-    if (merges <= 1u) return head;
-  }
-}
-
-// Colour buffer after the colour pass: the tail fragments of target t over
-// the background in id order (the ROP's primitive order, main.cpp:548-558),
-// folded newest first: acc = t_n over ... over t_1, then acc over the
-// background. The list is unordered, so each walk takes the next
-// kTailWindow values in descending order (one walk for most targets, up to
-// kTailWalks) and loads their colours four at a time; a longer tail is
-// sorted in place and folded in one walk. `skip` boundary-flagged entries are in the A-buffer and not blended
-// (Loop64 identical keys, see k_loop64_classify): the flagged ones with the
-// lowest ids.
-// tail_fold with the list's head value already loaded (a composite issues
-// that load with its own first loads instead of after them).
-__device__ __forceinline__ float4 tail_fold_from(const TailBuf& tb, uint32_t head, float4 bg, uint32_t skip) {
-  const uint32_t vcap = tail_value_cap(tb.cap);
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (head == 0u || head >= vcap) return over(acc, bg);
-  uint32_t keep = 0xFFFFFFFFu;  // flagged entries to blend
-  uint32_t bound = 0xFFFFFFFFu;
-  bool bad = false;
-  for (bool first = true;; first = false) {
-    uint32_t w[kTailWindow];
-    uint32_t flagged;
-    const uint32_t n = tail_window(tb, head, vcap, bound, w, flagged, bad);
-    if (first && skip > 0u) keep = flagged > skip ? flagged - skip : 0u;
-    if (first && !bad && n > (uint32_t)kTailWindow * kTailWalks) {  // a long tail: sorted, then one walk
-      for (uint32_t v = tail_sort_desc(tb, head, vcap); v != 0u && v < vcap;) {
-        const uint32_t id = tail_index(v);
-        const uint32_t nx = tb.next[id];
-        if (!(v & 1u) || keep > 0u) {
-          acc = over(acc, tb.rgba[id]);
-          if (v & 1u) --keep;
-        }
-        v = nx;
-      }
-      break;
-    }
-#pragma unroll
-    for (int g = 0; g < kTailWindow; g += 4) {
-      if (w[g] == 0u) break;
-      float4 c[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) c[j] = w[g + j] ? tb.rgba[tail_index(w[g + j])] : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t v = w[g + j];
-        if (v != 0u && (!(v & 1u) || keep > 0u)) {
-          acc = over(acc, c[j]);
-          if (v & 1u) --keep;
-        }
-      }
-    }
-    if (bad || n <= (uint32_t)kTailWindow) break;
-    bound = w[kTailWindow - 1];
-  }
-  return over(acc, bg);
-}
-
-__device__ __forceinline__ float4 tail_fold(const TailBuf& tb, uint32_t t, float4 bg, uint32_t skip) {
-  return tail_fold_from(tb, tb.head[t], bg, skip);
-}
-
-// Sample shading with spp samples per pixel lays targets out sample-major
-// (sample * pixels + pixel). pm_index(t) is target t's place in pixel-major
-// order (pixel * spp + sample) and pm_target(a) its inverse. The stream gives
-// a fragment's covered samples consecutive ids, so structures indexed
-// pixel-major (the WBOIT accumulators) take one wave's atomics on one run of
-// entries, and composites that walk targets in pixel-major order give a
-// pixel's samples neighbouring lanes, whose list nodes share cache lines.
-// spp is 1, 2, 4 or 8: shifts and compares, no divisions.
-__device__ __forceinline__ uint32_t pm_index(uint32_t t, uint32_t T, uint32_t spp) {
-  if (spp <= 1u) return t;
-  const uint32_t sh = (uint32_t)__builtin_ctz(spp);
-  const uint32_t px = T >> sh;
-  uint32_t smp = 0;
-  for (uint32_t k = 1; k < spp; ++k) smp += t >= k * px ? 1u : 0u;
-  return ((t - smp * px) << sh) | smp;
-}
-__device__ __forceinline__ uint32_t pm_target(uint32_t a, uint32_t T, uint32_t spp) {
-  if (spp <= 1u) return a;
-  const uint32_t sh = (uint32_t)__builtin_ctz(spp);
-  return (a & (spp - 1u)) * (T >> sh) + (a >> sh);
-}
-
-// Colour buffer of target t before the colour-pass tail: the colour of the
-// frame's opaque pass, else the clear colour.
-__device__ __forceinline__ float4 dest_of(const Common& c, uint32_t t) {
-  return c.opq_rgba ? c.opq_rgba[t] : c.background;
-}
-
-// Early depth test of a transparent fragment against the frame's opaque pass
-// (early_fragment_tests with post_depth_coverage, oitColorDepthDefines.glsl:
-// 24-37; VK_COMPARE_OP_LESS without depth write, main.cpp:526-528,541-543):
-// the samples of mask m whose opaque depth key is larger than key (one test
-// at target t unless coverage shading). Zero: the fragment does not exist.
-__device__ __forceinline__ uint32_t opaque_visible(const uint64_t* z, uint32_t T, uint32_t cov, uint32_t t,
-                                                   uint32_t key, uint32_t m) {
-  if (!z) return m;
-  if (cov > 1u) {
-    uint32_t r = 0u;
-    for (uint32_t s = 0; s < cov; ++s)
-      if (((m >> s) & 1u) && key < (uint32_t)(z[(uint64_t)s * T + t] >> 32)) r |= 1u << s;
-    return r;
-  }
-  return key < (uint32_t)(z[t] >> 32) ? m : 0u;
-}
-
-// Coverage shading: the ROP blends each tail fragment into the samples of
-// its mask; per sample the newest-first fold over the sample's colour (the
-// opaque pass's, else the clear colour), then the sum over samples in order
-// divided by their count (the MSAA resolve). Without an opaque pass a target
-// without tail fragments keeps the clear colour.
-__device__ __forceinline__ float4 tail_fold_cov(const TailBuf& tb, uint32_t t, const Common& c) {
-  const uint32_t S = c.cov;
-  const uint32_t vcap = tail_value_cap(tb.cap);
-  const uint32_t head = tb.head ? tb.head[t] : 0u;
-  const bool empty = head == 0u || head >= vcap;
-  if (empty && !c.opq_rgba) return c.background;
-  float4 acc[8];
-#pragma unroll
-  for (int s = 0; s < 8; ++s) acc[s] = make_float4(0.f, 0.f, 0.f, 0.f);
-  uint32_t bound = 0xFFFFFFFFu;
-  bool bad = false;
-  while (!empty) {  // windows of the unordered list, newest first (tail_fold_from)
-    uint32_t w[kTailWindow];
-    uint32_t flagged;
-    const uint32_t n = tail_window(tb, head, vcap, bound, w, flagged, bad);
-    if (bound == 0xFFFFFFFFu && !bad && n > (uint32_t)kTailWindow * kTailWalks) {  // a long tail: sorted, one walk
-      for (uint32_t v = tail_sort_desc(tb, head, vcap); v != 0u && v < vcap;) {
-        const uint32_t id = tail_index(v);
-        const uint32_t nx = tb.next[id];
-        const uint32_t m = tb.mask[id];
-        const float4 col = tb.rgba[id];
-#pragma unroll
-        for (int s = 0; s < 8; ++s)
-          if ((uint32_t)s < S && ((m >> s) & 1u)) acc[s] = over(acc[s], col);
-        v = nx;
-      }
-      break;
-    }
-#pragma unroll
-    for (int g = 0; g < kTailWindow; g += 4) {
-      if (w[g] == 0u) break;
-      float4 col[4];
-      uint32_t msk[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const bool h = w[g + j] != 0u;
-        col[j] = h ? tb.rgba[tail_index(w[g + j])] : make_float4(0.f, 0.f, 0.f, 0.f);
-        msk[j] = h ? tb.mask[tail_index(w[g + j])] : 0u;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int s = 0; s < 8; ++s)
-          if ((uint32_t)s < S && ((msk[j] >> s) & 1u)) acc[s] = over(acc[s], col[j]);
-    }
-    if (bad || n <= (uint32_t)kTailWindow) break;
-    bound = w[kTailWindow - 1];
-  }
-  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    if ((uint32_t)s < S) {
-      const float4 cb = over(acc[s], c.opq_rgba ? c.opq_rgba[(uint64_t)s * c.T + t] : c.background);
-      sum = make_float4(sum.x + cb.x, sum.y + cb.y, sum.z + cb.z, sum.w + cb.w);
-    }
-  }
-  const float fs = (float)S;
-  return make_float4(sum.x / fs, sum.y / fs, sum.z / fs, sum.w / fs);
-}
-
-// Coverage-shaded front blend (oitLinkedList.frag.glsl:147-160,
-// oitSimple.frag.glsl:142-159): per sample, front to back over the sorted
-// layers whose mask holds it; the sample colours summed in order and divided
-// by the sample count.
-template <int K>
-__device__ __forceinline__ float4 blend_front_cov(const uint32_t* cols, const uint32_t* masks, uint32_t n, uint32_t S,
-                                                  const float* s_dec, const float* s_alpha) {
-  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (uint32_t s = 0; s < S; ++s) {
-    float4 sc = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-      if ((uint32_t)k < n && ((masks[k] >> s) & 1u)) sc = over(sc, decode_premult_lds(cols[k], s_dec, s_alpha));
-    sum = make_float4(sum.x + sc.x, sum.y + sc.y, sum.z + sc.z, sum.w + sc.w);
-  }
-  const float fs = (float)S;
-  return make_float4(sum.x / fs, sum.y / fs, sum.z / fs, sum.w / fs);
-}
-
-template <int K>
-__device__ __forceinline__ void write_debug(const ResolveOut& o, uint32_t t, const FrontK<K>& a, uint32_t n,
-                                            uint32_t count, bool ids_from_nodes, bool vals_are_colors) {
-  if (o.fk_key) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) o.fk_key[(uint64_t)t * K + k] = (uint32_t)k < n ? (uint32_t)(a.sk[k] >> 32) : kEmpty;
-  }
-  if (o.fk_val) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      uint32_t v = kEmpty;
-      if ((uint32_t)k < n) {
-        v = vals_are_colors ? a.col[k] : (uint32_t)a.sk[k];
-        if (ids_from_nodes) v -= 1u;  // node n holds fragment id n - 1
-      }
-      o.fk_val[(uint64_t)t * K + k] = v;
-    }
-  }
-  if (o.counts) o.counts[t] = count;
-}
 
 // ---------------------------------------------------------------------------
 // Fill
@@ -681,12 +61,6 @@ __global__ __launch_bounds__(kBlock) void k_fill_ranges(FillArgs a) {
 // fragment in draw order; here the allocation is the fragment's own index, so
 // no global counter is contended), overflow -> tail (:59-68), node payload
 // (:75-82). The link word is set to kUnset for the link kernel.
-// Codec thresholds staged in LDS for the block.
-__device__ __forceinline__ void stage_thresholds(float* s_thr, const CodecTables* tab) {
-  for (uint32_t k = threadIdx.x; k < 257u; k += kBlock) s_thr[k] = tab->thr[k];
-  __syncthreads();
-}
-
 template <bool kTail>
 __global__ __launch_bounds__(kBlock) void k_ll_store(Common c, FragView f, LLBuf ll, TailBuf tb) {
   __shared__ float s_thr[257];
@@ -996,13 +370,6 @@ __device__ __forceinline__ float4 ll_walk_reset_keys(uint32_t t, const LLBuf& ll
   return over(col, tailc);
 }
 
-__device__ __forceinline__ void stage_decode(float* s_dec, float* s_alpha, const CodecTables* tab) {
-  for (uint32_t k = threadIdx.x; k < 256u; k += kBlock) {
-    s_dec[k] = tab->dec[k];
-    s_alpha[k] = tab->alpha[k];
-  }
-}
-
 // Composite of the Linked List (oitLinkedList.frag.glsl:106-172) that leaves
 // the structure clean for the next frame: head[t] = 0 (the clear of
 // oitRender.cpp:206-212 done by the reader) and next[p] = kUnset for every
@@ -1110,19 +477,6 @@ __global__ __launch_bounds__(kBlock) void k_ll_resolve_cov(Common c, LLBuf ll, T
 // unit (64 * kU fragments) and no resolve tile (kBlock targets) spans two
 // frames. Each frame gets exactly the single-frame result.
 // ---------------------------------------------------------------------------
-
-// Last frame in [lo, hi) whose base is <= key (bases ascend); key is wave
-// uniform, so the probes are scalar loads.
-template <bool kTargets>
-__device__ __forceinline__ uint32_t find_frame(const BatchFrameDev* fr, uint32_t lo, uint32_t hi, uint64_t key) {
-  while (hi - lo > 1u) {
-    const uint32_t mid = (lo + hi) >> 1;
-    const uint64_t base = kTargets ? (uint64_t)fr[mid].target_base : (uint64_t)fr[mid].frag_base;
-    if (base <= key) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
 
 // ---------------------------------------------------------------------------
 // Binned batch frames (BatchFrameDev::mode == kModeBin): the fragments of
@@ -1306,13 +660,6 @@ __global__ __launch_bounds__(kBlock) void k_bin_scatter(BatchArgs b, LLBuf ll) {
       ll.next[s] = (uint32_t)i + 1u;
     }
   }
-}
-
-// Orders LDS ops of one wave: every lane's earlier LDS access has completed
-// and none is moved across (the wave's lanes exchange data through LDS).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
 }
 
 // Every global load the lane issued has returned, and no memory access is
@@ -2028,283 +1375,6 @@ __global__ __launch_bounds__(kBlock) void k_kbuf_resolve_cov(Common c, KBuf kb, 
 }
 
 // ---------------------------------------------------------------------------
-// Loop32: oitLoop.frag.glsl (the geometry is drawn twice)
-// ---------------------------------------------------------------------------
-
-// Depth pass (:57-100): the K nearest distinct depth keys per target, sorted,
-// by a u32 atomicMin chain that stops at an empty slot or its own key; the two
-// pretests use plain loads (slots only decrease within the pass). Two
-// consecutive lanes of one target (a sphere's front and back) run one chain
-// carrying both keys, as in k_loop64_store, with the set rule: a carried key
-// that meets its equal in a slot, or equals the other carried key, is done.
-// Each wave takes kU chunks of 64 consecutive fragments: the chunks' loads,
-// pretests (with four probe slots) and atomic chains are in flight together,
-// one dependent round trip per chain step of all of them.
-template <int K, int kU>
-__global__ __launch_bounds__(kBlock) void k_loop32_depth_m(Common c, FragView f, uint32_t* __restrict__ zs) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t first = ((uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * (64u * kU);
-  uint32_t t[kU];
-  float dv[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {  // every chunk's target and depth in one round trip
-    const uint64_t i = first + (uint64_t)u * 64u + lane;
-    const bool in = i < f.count;
-    t[u] = in ? ld_stream(&f.target[i]) : kEmpty;
-    dv[u] = in ? ld_stream(&f.depth[i]) : 0.f;
-  }
-  uint32_t a[kU], b[kU];
-  bool hasb[kU], act[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    uint32_t tt = t[u] < c.T ? t[u] : kEmpty;
-    uint32_t z = 0u;
-    if (tt != kEmpty) {
-      z = depth_key(dv[u]);
-      if (!opaque_visible(c.opq_z, c.T, 1u, tt, z, 1u)) tt = kEmpty;
-    }
-    const Run r = same_target_run(tt);
-    const uint32_t zn = __shfl_down(z, 1u);
-    const bool lead = tt != kEmpty && ((r.lane - r.start_lane) & 1u) == 0u;
-    hasb[u] = lead && r.lane < r.end_lane && zn != z;
-    a[u] = z;
-    b[u] = 0u;
-    if (hasb[u]) {
-      a[u] = z < zn ? z : zn;
-      b[u] = z < zn ? zn : z;
-    }
-    act[u] = lead;
-    t[u] = tt;
-  }
-  // the pretests and the first slots of every chunk in one round trip
-  constexpr int kProbe = K / 2 < 4 ? K / 2 : 4;
-  int j[kU];
-  {
-    uint32_t probe[kU][kProbe > 0 ? kProbe : 1], z_last[kU], z_mid[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (act[u]) {
-#pragma unroll
-        for (int k = 0; k < kProbe; ++k) probe[u][k] = zs[(uint64_t)k * c.T + t[u]];
-        z_last[u] = zs[(uint64_t)(K - 1) * c.T + t[u]];
-        z_mid[u] = zs[(uint64_t)(K / 2) * c.T + t[u]];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      j[u] = 0;
-      if (act[u]) {
-        if (a[u] > z_last[u]) {
-          act[u] = false;
-        } else if (a[u] > z_mid[u]) {
-          j[u] = K / 2;
-        } else {
-#pragma unroll
-          for (int k = 0; k < kProbe; ++k) j[u] += probe[u][k] < a[u] ? 1 : 0;
-        }
-      }
-    }
-  }
-  // the chains, one step of every live chain per round trip
-  for (;;) {
-    uint32_t old[kU];
-    bool any = false;
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (act[u]) {
-        old[u] = __hip_atomic_fetch_min(&zs[(uint64_t)j[u] * c.T + t[u]], a[u], __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-        any = true;
-      }
-    }
-    returns_done();
-    if (!any) break;
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (!act[u]) continue;
-      if (old[u] == kEmpty || old[u] == a[u]) {  // a is in slot j now (or was already): b goes on
-        if (hasb[u]) {
-          a[u] = b[u];
-          hasb[u] = false;
-        } else {
-          act[u] = false;
-        }
-      } else if (old[u] > a[u]) {  // a took slot j and old comes out
-        if (!hasb[u]) {
-          a[u] = old[u];
-        } else if (old[u] == b[u]) {  // the two carried keys are equal: one of them is done
-          a[u] = b[u];
-          hasb[u] = false;
-        } else if (old[u] < b[u]) {
-          a[u] = old[u];
-        } else {
-          a[u] = b[u];
-          b[u] = old[u];
-        }
-      }  // else a smaller key holds slot j: a goes on unchanged
-      if (++j[u] >= K) act[u] = false;
-    }
-  }
-}
-
-// Colour pass (:105-180): behind the K-th depth -> tail-blend the shaded
-// colour; else the slot of its depth by binary search, where the colour of the
-// latest fragment in primitive order is kept ((id + 1) << 32 | colour,
-// atomicMax), the result of the reference's plain store in draw order.
-// Each wave takes kU chunks of 64 consecutive fragments: every chunk's
-// fields, then every chunk's lower-half depth slots, in one round trip each;
-// the upper half only where a pixel holds more than K/2 depths below the
-// fragment's.
-template <int K, bool kTail, int kU>
-__global__ __launch_bounds__(kBlock) void k_loop32_color_m(Common c, FragView f, const uint32_t* __restrict__ zs,
-                                                           uint64_t* __restrict__ cs, TailBuf tb) {
-  __shared__ float s_thr[257];
-  stage_thresholds(s_thr, c.tab);
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t first = ((uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * (64u * kU);
-  uint32_t t[kU], z[kU];
-  float dv[kU];
-  float4 cv[kU];
-  bool valid[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const uint64_t i = first + (uint64_t)u * 64u + lane;
-    valid[u] = i < f.count;
-    t[u] = valid[u] ? ld_stream(&f.target[i]) : kEmpty;
-    dv[u] = valid[u] ? ld_stream(&f.depth[i]) : 0.f;
-    cv[u] = valid[u] ? ld_stream(&f.rgba[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    if (t[u] >= c.T) valid[u] = false;
-    z[u] = valid[u] ? depth_key(dv[u]) : 0u;
-    if (valid[u] && !opaque_visible(c.opq_z, c.T, 1u, t[u], z[u], 1u)) valid[u] = false;
-    if (!valid[u]) t[u] = kEmpty;
-  }
-  // the first half of every chunk's depth slots in one round trip, loaded by
-  // every lane (one without a fragment reads target 0's), so no load waits
-  // behind another; the second half only where the first is all nearer
-  constexpr int kHalf = K / 2 > 0 ? K / 2 : K;
-  uint32_t below[kU], ts[kU];
-  {
-    uint32_t zk[kU][kHalf];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      ts[u] = valid[u] ? t[u] : 0u;
-#pragma unroll
-      for (int k = 0; k < kHalf; ++k) zk[u][k] = zs[(uint64_t)k * c.T + ts[u]];
-    }
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      below[u] = 0;
-#pragma unroll
-      for (int k = 0; k < kHalf; ++k) below[u] += valid[u] && zk[u][k] < z[u] ? 1u : 0u;
-    }
-  }
-  if constexpr (kHalf < K) {
-    bool more[kU], any = false;
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      more[u] = valid[u] && below[u] == (uint32_t)kHalf;
-      any = any || more[u];
-    }
-    if (__ballot(any)) {  // wave-uniform: then every lane loads, as above
-      uint32_t zk[kU][K - kHalf];
-#pragma unroll
-      for (int u = 0; u < kU; ++u)
-#pragma unroll
-        for (int k = kHalf; k < K; ++k) zk[u][k - kHalf] = zs[(uint64_t)k * c.T + ts[u]];
-#pragma unroll
-      for (int u = 0; u < kU; ++u)
-#pragma unroll
-        for (int k = kHalf; k < K; ++k) below[u] += more[u] && zk[u][k - kHalf] < z[u] ? 1u : 0u;
-    }
-  }
-  bool tail[kU];
-  uint32_t lid[kU];
-  float4 payload[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    lid[u] = f.id_base + (uint32_t)(first + (uint64_t)u * 64u + lane);
-    tail[u] = false;
-    payload[u] = valid[u] ? cv[u] : make_float4(0.f, 0.f, 0.f, 0.f);
-    if (valid[u]) {
-      if (below[u] == (uint32_t)K) {
-        tail[u] = true;
-      } else {
-        const uint64_t v = ((uint64_t)(lid[u] + 1u) << 32) | encode_color_lds(cv[u], s_thr);
-        (void)__hip_atomic_fetch_max(&cs[(uint64_t)below[u] * c.T + t[u]], v, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-  }
-  if constexpr (kTail) tail_queue_push_n<kU>(tail, t, lid, payload, tb);
-}
-
-// Composite (:186-222): the layers up to the first empty depth, front to back,
-// over the colour buffer. The slots it read are set back to empty (depth
-// kEmpty, colour 0) for the next frame: the stored depths are a prefix, and
-// the colour pass writes only the slot of a stored depth.
-template <int K, bool kColorTail, bool kDebug>
-__global__ __launch_bounds__(kBlock) void k_loop32_resolve(Common c, uint32_t* __restrict__ zs,
-                                                           uint64_t* __restrict__ cs, TailBuf tb, ResolveOut o) {
-  __shared__ float s_dec[256];
-  __shared__ float s_alpha[256];
-  stage_decode(s_dec, s_alpha, c.tab);
-  __syncthreads();
-  const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= c.T) return;
-  uint32_t z[K], col[K];
-  uint32_t n = 0;
-  bool alive = true;
-  // depths are sorted with the empty slots last: the upper half is loaded
-  // only where the lower half is full
-  constexpr int kHalf = K / 2 > 0 ? K / 2 : K;
-  const uint32_t th = kColorTail ? tb.head[t] : 0u;  // tail list head, with the depths
-#pragma unroll
-  for (int k = 0; k < kHalf; ++k) z[k] = zs[(uint64_t)k * c.T + t];
-#pragma unroll
-  for (int k = kHalf; k < K; ++k) z[k] = kEmpty;
-  if (z[kHalf - 1] != kEmpty) {
-#pragma unroll
-    for (int k = kHalf; k < K; ++k) z[k] = zs[(uint64_t)k * c.T + t];
-  }
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    alive = alive && z[k] != kEmpty;
-    n += alive ? 1u : 0u;
-  }
-  // the stored layers' colours, loaded together once n is known
-#pragma unroll
-  for (int k = 0; k < K; ++k) col[k] = (uint32_t)k < n ? (uint32_t)cs[(uint64_t)k * c.T + t] : 0u;
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    if ((uint32_t)k < n) {
-      zs[(uint64_t)k * c.T + t] = kEmpty;
-      cs[(uint64_t)k * c.T + t] = 0ull;
-    }
-  }
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-    if ((uint32_t)k < n) acc = over(acc, decode_premult_lds(col[k], s_dec, s_alpha));
-  float4 d = dest_of(c, t);
-  if (kColorTail) d = tail_fold_from(tb, th, d, 0u);
-  o.out[t] = over(acc, d);
-  if (kDebug) {
-    if (o.fk_key) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) o.fk_key[(uint64_t)t * K + k] = (uint32_t)k < n ? z[k] : kEmpty;
-    }
-    if (o.fk_val) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) o.fk_val[(uint64_t)t * K + k] = (uint32_t)k < n ? col[k] : kEmpty;
-    }
-    if (o.counts) o.counts[t] = n;
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Ordered interlock: oitInterlock.frag.glsl:52-148 with pixel_interlock_ordered
 // ---------------------------------------------------------------------------
 
@@ -2509,387 +1579,6 @@ __global__ __launch_bounds__(kBlock, (K == 16 && !kCov) ? 6 : 1) void k_interloc
       for (int k = 0; k < K; ++k) o.fk_val[(uint64_t)t * K + k] = (uint32_t)k < n ? (uint32_t)a.sk[k] : kEmpty;
     }
     if (o.counts) o.counts[t] = count;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Loop64: oitLoop64.frag.glsl
-// ---------------------------------------------------------------------------
-
-// Ascending sort of N (a power of two) values held in registers: a bitonic
-// network with compile-time indices (no spills, no dynamic indexing).
-template <int N>
-__device__ __forceinline__ void sort_u64(uint64_t* v) {
-#pragma unroll
-  for (int size = 2; size <= N; size <<= 1) {
-#pragma unroll
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        const int j = i ^ stride;
-        if (j > i) {
-          const bool up = (i & size) == 0;
-          const uint64_t x = v[i], y = v[j];
-          const bool swap = up ? (x > y) : (x < y);
-          v[i] = swap ? y : x;
-          v[j] = swap ? x : y;
-        }
-      }
-    }
-  }
-}
-
-// A chunk's mask, read as one wave-uniform (scalar) value.
-__device__ __forceinline__ uint64_t big_mask_load(const uint64_t* p) {
-  const uint64_t m = *p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)m);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(m >> 32));
-  return ((uint64_t)hi << 32) | lo;
-}
-
-// Per-target count of the frame's fragments that pass the opaque depth
-// test: one returnless atomic per run of one target in a wave. Runs at
-// append, so that the stores, at resolve, know every pixel's final count.
-// kU chunks of 64 fragments per wave, their loads in one round trip; the
-// depths are read only when an opaque pass can cull.
-template <int kU>
-__global__ __launch_bounds__(kBlock) void k_loop64_count(Common c, FragView f, uint32_t* __restrict__ cnt) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t first = ((uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * (64u * kU);
-  const bool culls = c.opq_z != nullptr;
-  uint32_t t[kU];
-  float dv[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const uint64_t i = first + (uint64_t)u * 64u + lane;
-    const bool in = i < f.count;
-    t[u] = in ? ld_stream(&f.target[i]) : kEmpty;
-    dv[u] = (in && culls) ? ld_stream(&f.depth[i]) : 0.f;
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    uint32_t tt = t[u] < c.T ? t[u] : kEmpty;
-    if (culls && tt != kEmpty && !opaque_visible(c.opq_z, c.T, 1u, tt, depth_key(dv[u]), 1u)) tt = kEmpty;
-    const Run r = same_target_run(tt);
-    if (tt != kEmpty && r.start) atomicAdd(&cnt[tt], r.end_lane - r.lane + 1u);
-  }
-}
-
-// Colour pass (oitLoop64.frag.glsl:65-141): key = depth << 32 | colour (:79).
-// The slots end as the K smallest keys of each pixel for any arrival order;
-// this pass gets there by one of two routes per pixel, chosen by the
-// pixel's count of the frame's fragments:
-// - at most K fragments: every one of them is kept, so each takes a slot
-//   index from its count (one returning atomic per run of one target,
-//   counting down to 0) and stores its key unsorted; the composite sorts
-//   the slots. No fragment of such a pixel is in the tail.
-// - more than K: the two pretests of USE_EARLYDEPTH (:82-101, plain loads:
-//   slots only decrease within a frame, so a stale value only lets more
-//   fragments try), then the atomicMin chain (:109-121), which keeps the
-//   slots sorted. Two consecutive lanes of one target (a sphere's front and
-//   back fragment) run one chain that carries both keys: at each slot the
-//   smaller carried key goes in, the key that comes out joins the larger
-//   one, and the chain ends when both are placed or pushed past slot K-1.
-//   The multiset of slots and carried keys is the same as after the two
-//   single chains, so the result is identical; the pair costs one chain
-//   instead of two and its lanes do not contend for the same slots.
-// Each wave takes kU chunks of 64 consecutive fragments: the chunks' loads,
-// counts, pretests and chain steps are in flight together.
-template <int K, int kU>
-__global__ __launch_bounds__(kBlock) void k_loop64_store_m(Common c, FragView f, uint64_t* __restrict__ slots,
-                                                           uint32_t* __restrict__ cnt, uint64_t* __restrict__ big) {
-  __shared__ float s_thr[257];
-  stage_thresholds(s_thr, c.tab);
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t first = ((uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * (64u * kU);
-  uint32_t t[kU];
-  float dv[kU];
-  float4 cv[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {  // every chunk's fields in one round trip
-    const uint64_t i = first + (uint64_t)u * 64u + lane;
-    const bool in = i < f.count;
-    t[u] = in ? ld_stream(&f.target[i]) : kEmpty;
-    dv[u] = in ? ld_stream(&f.depth[i]) : 0.f;
-    cv[u] = in ? ld_stream(&f.rgba[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  uint64_t z[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    uint32_t tt = t[u] < c.T ? t[u] : kEmpty;
-    z[u] = kEmpty64;
-    if (tt != kEmpty) {
-      const uint32_t key = depth_key(dv[u]);
-      if (opaque_visible(c.opq_z, c.T, 1u, tt, key, 1u)) z[u] = ((uint64_t)key << 32) | encode_color_lds(cv[u], s_thr);
-      else tt = kEmpty;
-    }
-    t[u] = tt;
-  }
-  // every chunk's pixel counts in one round trip, loaded by every lane (one
-  // without a fragment reads target 0's), so no load waits behind another
-  uint32_t n[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) n[u] = cnt[t[u] != kEmpty ? t[u] : 0u];
-  // pixels of at most K fragments: a slot index per fragment from the count,
-  // every chunk's atomics in flight together
-  uint32_t base[kU], start_lane[kU], rank[kU];
-  bool small[kU], sub[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    small[u] = t[u] != kEmpty && n[u] <= (uint32_t)K;
-    const Run r = same_target_run(small[u] ? t[u] : kEmpty);
-    sub[u] = small[u] && r.start;
-    rank[u] = r.end_lane - r.lane + 1u;  // the run's length, at its first lane
-    start_lane[u] = r.start_lane;
-    base[u] = 0u;
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u)
-    if (sub[u]) base[u] = atomicSub(&cnt[t[u]], rank[u]);
-  returns_done();
-#pragma unroll
-  for (int u = 0; u < kU; ++u)  // this lane's index + 1
-    base[u] = __shfl(base[u], (int)start_lane[u]) - (lane_id() - start_lane[u]);
-  // pixels of more than K: their fragments' lanes, per 64-fragment chunk,
-  // for the classification (which skips the rest); pairs and chains
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const uint64_t m = __ballot(t[u] != kEmpty && !small[u]);
-    if (lane == 0u && first + (uint64_t)u * 64u < f.count) big[first / 64u + u] = m;
-  }
-  uint64_t a[kU], b[kU];
-  bool hasb[kU], act[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const uint32_t tb = small[u] ? kEmpty : t[u];
-    const Run r = same_target_run(tb);
-    const uint32_t zn_lo = __shfl_down((uint32_t)z[u], 1u);
-    const uint32_t zn_hi = __shfl_down((uint32_t)(z[u] >> 32), 1u);
-    const uint64_t zn = ((uint64_t)zn_hi << 32) | zn_lo;
-    const bool lead = tb != kEmpty && ((r.lane - r.start_lane) & 1u) == 0u;
-    hasb[u] = lead && r.lane < r.end_lane;
-    a[u] = z[u];
-    b[u] = 0;
-    if (hasb[u]) {
-      a[u] = z[u] < zn ? z[u] : zn;
-      b[u] = z[u] < zn ? zn : z[u];
-    }
-    act[u] = lead;
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u)  // the stores of the kept fragments (index base - 1 < K)
-    if (small[u] && base[u] - 1u < (uint32_t)K) slots[(uint64_t)(base[u] - 1u) * c.T + t[u]] = z[u];
-  // the pretests and the first slots of every chunk in one round trip
-  constexpr int kProbe = K / 2 < 4 ? K / 2 : 4;
-  int j[kU];
-  {
-    uint64_t probe[kU][kProbe > 0 ? kProbe : 1], s_last[kU], s_mid[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (act[u]) {
-#pragma unroll
-        for (int k = 0; k < kProbe; ++k) probe[u][k] = slots[(uint64_t)k * c.T + t[u]];
-        s_last[u] = slots[(uint64_t)(K - 1) * c.T + t[u]];
-        s_mid[u] = slots[(uint64_t)(K / 2) * c.T + t[u]];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      j[u] = 0;
-      if (act[u]) {
-        if (a[u] > s_last[u]) {
-          act[u] = false;
-        } else if (a[u] > s_mid[u]) {
-          j[u] = K / 2;
-        } else {
-#pragma unroll
-          for (int k = 0; k < kProbe; ++k) j[u] += probe[u][k] < a[u] ? 1 : 0;
-        }
-      }
-    }
-  }
-  // the chains, one step of every live chain per round trip
-  for (;;) {
-    uint64_t old[kU];
-    bool any = false;
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (act[u]) {
-        old[u] = __hip_atomic_fetch_min(&slots[(uint64_t)j[u] * c.T + t[u]], a[u], __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-        any = true;
-      }
-    }
-    returns_done();
-    if (!any) break;
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (!act[u]) continue;
-      if (old[u] == kEmpty64) {  // placed in an empty slot: b (if any) goes to the next one
-        if (hasb[u]) {
-          a[u] = b[u];
-          hasb[u] = false;
-        } else {
-          act[u] = false;
-        }
-      } else {
-        const uint64_t up = old[u] > a[u] ? old[u] : a[u];  // the key that leaves slot j
-        if (hasb[u] && b[u] < up) {
-          a[u] = b[u];
-          b[u] = up;
-        } else {
-          a[u] = up;
-        }
-      }
-      if (++j[u] >= K) act[u] = false;
-    }
-  }
-}
-
-// Tail classification: a fragment whose key is above the final K-th key was
-// evicted or rejected (the colours oitLoop64.frag.glsl:131-136 tail-blends);
-// one equal to it is "boundary": identical (depth, colour) keys are the same
-// bits in the A-buffer, and the resolve keeps the lowest ids of them in front.
-// Only pixels of more than K fragments can have tails (the others keep every
-// fragment): the store left, per 64-fragment chunk, the mask of the lanes
-// whose fragment belongs to such a pixel, and a chunk with an empty mask is
-// skipped. Each wave takes kU chunks and loads, one round trip each: the
-// masked lanes' targets and depths, then every lane's K-th slot, then the
-// colours of the lanes at or past the K-th depth; the tail fragments go
-// onto their lists with every chunk's exchanges in flight together.
-template <int K, int kU>
-__global__ __launch_bounds__(kBlock) void k_loop64_classify(Common c, FragView f, const uint64_t* __restrict__ slots,
-                                                            const uint64_t* __restrict__ bigm, TailBuf tb) {
-  __shared__ float s_thr[257];
-  __shared__ float s_dec[256];
-  __shared__ float s_alpha[256];
-  stage_decode(s_dec, s_alpha, c.tab);
-  stage_thresholds(s_thr, c.tab);  // its barrier also publishes the decode tables
-  const uint32_t lane = lane_id();
-  const uint64_t first = ((uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * (64u * kU);
-  bool big[kU];
-  uint64_t any = 0;
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const uint64_t m = first + (uint64_t)u * 64u < f.count ? big_mask_load(&bigm[first / 64u + u]) : 0ull;
-    big[u] = (m >> lane) & 1ull;
-    any |= m;
-  }
-  if (any == 0ull) return;  // wave-uniform: no fragment of this wave can be in the tail
-  uint32_t t[kU];
-  float dv[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const uint64_t i = first + (uint64_t)u * 64u + lane;
-    t[u] = big[u] ? ld_stream(&f.target[i]) : 0u;
-    dv[u] = big[u] ? ld_stream(&f.depth[i]) : 0.f;
-  }
-  // every chunk's K-th slots in one round trip, loaded by every lane (a lane
-  // outside such a pixel reads target 0's: one line for all of them), so no
-  // load waits behind another
-  uint64_t sk[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) sk[u] = slots[(uint64_t)(K - 1) * c.T + t[u]];
-  uint32_t key[kU];
-  bool cand[kU];
-  float4 cv[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    key[u] = depth_key(dv[u]);
-    // the key's high half is the depth: a nearer fragment stays in the slots
-    cand[u] = big[u] && key[u] >= (uint32_t)(sk[u] >> 32);
-    cv[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u)  // the candidates' colours, one round trip
-    if (cand[u]) cv[u] = ld_stream(&f.rgba[first + (uint64_t)u * 64u + lane]);
-  returns_done();
-  bool tail[kU];
-  uint32_t flag[kU], lid[kU];
-  float4 payload[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    tail[u] = false;
-    flag[u] = 0u;
-    payload[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (cand[u]) {
-      const uint32_t col = encode_color_lds(cv[u], s_thr);
-      const uint64_t z = ((uint64_t)key[u] << 32) | col;
-      if (z >= sk[u]) {
-        tail[u] = true;
-        flag[u] = z == sk[u] ? 1u : 0u;
-        payload[u] = decode_premult_lds(col, s_dec, s_alpha);
-      }
-    }
-    lid[u] = f.id_base + (uint32_t)(first + (uint64_t)u * 64u + lane);
-  }
-  tail_list_push_n<kU>(tail, t, lid, flag, payload, tb);
-}
-
-// Composite (oitLoop64.frag.glsl:162-183): blend slots front to back until
-// the first empty one. The slots it read are set back to empty for the next
-// frame (the occupied ones are a prefix: slots stay sorted, and no key is
-// the empty key), so the next clear need not write the whole A-buffer.
-template <int K, bool kColorTail, bool kDebug>
-__global__ __launch_bounds__(kBlock) void k_loop64_resolve(Common c, uint64_t* __restrict__ slots,
-                                                           uint32_t* __restrict__ cnt, TailBuf tb, ResolveOut o) {
-  __shared__ float s_dec[256];
-  __shared__ float s_alpha[256];
-  stage_decode(s_dec, s_alpha, c.tab);
-  __syncthreads();
-  const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= c.T) return;
-  // slots are sorted with the empty ones last: the upper half is loaded only
-  // where the lower half is full
-  constexpr int kHalf = K / 2 > 0 ? K / 2 : K;
-  const uint32_t th = kColorTail ? tb.head[t] : 0u;  // tail list head, with the slots
-  const uint32_t n_frame = cnt[t];  // more than K: chained, sorted; else 0 and the slots unsorted
-  uint64_t s[K];
-#pragma unroll
-  for (int k = 0; k < kHalf; ++k) s[k] = slots[(uint64_t)k * c.T + t];
-  const bool upper = (uint32_t)(s[kHalf - 1] >> 32) != kEmpty;
-#pragma unroll
-  for (int k = kHalf; k < K; ++k) s[k] = upper ? slots[(uint64_t)k * c.T + t] : kEmpty64;
-  // a pixel of at most K fragments stored them unsorted (empty slots last,
-  // the empty key being the largest): sort; sorted slots stay as they are.
-  // The network's size is wave-uniform: half of K where no lane holds more.
-  if (__ballot(upper)) sort_u64<K>(s);
-  else sort_u64<kHalf>(s);
-  if (n_frame) cnt[t] = 0u;
-  float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
-  uint32_t n = 0;
-  bool alive = true;
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    alive = alive && (uint32_t)(s[k] >> 32) != kEmpty;
-    if (alive) {
-      col = over(col, decode_premult_lds((uint32_t)s[k], s_dec, s_alpha));
-      ++n;
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-    if ((uint32_t)k < n) slots[(uint64_t)k * c.T + t] = kEmpty64;
-  float4 d = dest_of(c, t);
-  if (kColorTail) {
-    uint32_t skip = 0;
-    if (n == (uint32_t)K) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) skip += s[k] == s[K - 1] ? 1u : 0u;
-    }
-    d = tail_fold_from(tb, th, d, skip);
-  }
-  o.out[t] = over(col, d);
-  if (kDebug) {
-    if (o.fk_key) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) o.fk_key[(uint64_t)t * K + k] = (uint32_t)k < n ? (uint32_t)(s[k] >> 32) : kEmpty;
-    }
-    if (o.fk_val) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) o.fk_val[(uint64_t)t * K + k] = (uint32_t)k < n ? (uint32_t)s[k] : kEmpty;
-    }
-    if (o.counts) o.counts[t] = n;
   }
 }
 
@@ -3141,7 +1830,11 @@ __global__ __launch_bounds__(kBlock) void k_codec_selftest(const CodecTables* ta
   uint32_t first = 0xFFFFFFFFu;
   for (uint64_t b = (uint64_t)lo + (uint64_t)blockIdx.x * kBlock + threadIdx.x; b < hi; b += stride) {
     const float c = __uint_as_float((uint32_t)b);
-    if (code_rgb_fast(c, s_thr) != code_rgb(c, tab->thr)) {
+    // the quick encode of a colour whose channels divide to about c, over
+    // alphas from 1/64 to 1 that vary with the pattern
+    const float al = (float)(1u + (((uint32_t)b * 2654435761u) >> 26)) * (1.0f / 64.0f);
+    const float4 pc = make_float4(c * al, c * (al * 0.999f), c * (al * 0.5f), al);
+    if (code_rgb_fast(c, s_thr) != code_rgb(c, tab->thr) || encode_color_quick(pc, tab) != encode_color(pc, tab)) {
       ++bad;
       if ((uint32_t)b < first) first = (uint32_t)b;
     }
@@ -3149,19 +1842,6 @@ __global__ __launch_bounds__(kBlock) void k_codec_selftest(const CodecTables* ta
   if (bad) {
     atomicAdd(mismatches, bad);
     atomicMin(first_bad, first);
-  }
-}
-
-template <template <int> class F, typename... A>
-hipError_t dispatch_k(uint32_t K, A&&... args) {
-  switch (K) {
-    case 1: return F<1>::run(args...);
-    case 2: return F<2>::run(args...);
-    case 4: return F<4>::run(args...);
-    case 8: return F<8>::run(args...);
-    case 16: return F<16>::run(args...);
-    case 32: return F<32>::run(args...);
-    default: return hipErrorInvalidValue;
   }
 }
 
@@ -3185,48 +1865,6 @@ struct SpinStore {
     const dim3 g(blocks_for(f.count)), b(kBlock);
     if (c.tail && tb.head) hipLaunchKernelGGL((k_spin_store<K, true>), g, b, 0, s, c, f, kb, tb);
     else hipLaunchKernelGGL((k_spin_store<K, false>), g, b, 0, s, c, f, kb, tb);
-    return hipGetLastError();
-  }
-};
-
-template <int K>
-struct Loop64Store {
-  static hipError_t run(const Common& c, const FragView& f, uint64_t* slots, uint32_t* cnt, uint64_t* big,
-                        int chunks, hipStream_t s) {
-    if (f.count == 0) return hipSuccess;
-    const int u = chunks >= 4 ? 4 : (chunks >= 2 ? 2 : 1);
-    const uint64_t per_block = (uint64_t)kBlock * u;
-    const dim3 g((uint32_t)((f.count + per_block - 1) / per_block)), b(kBlock);
-    if (u == 4) hipLaunchKernelGGL((k_loop64_store_m<K, 4>), g, b, 0, s, c, f, slots, cnt, big);
-    else if (u == 2) hipLaunchKernelGGL((k_loop64_store_m<K, 2>), g, b, 0, s, c, f, slots, cnt, big);
-    else hipLaunchKernelGGL((k_loop64_store_m<K, 1>), g, b, 0, s, c, f, slots, cnt, big);
-    return hipGetLastError();
-  }
-};
-
-template <int K>
-struct Loop64Classify {
-  static hipError_t run(const Common& c, const FragView& f, const uint64_t* slots, const uint64_t* big,
-                        const TailBuf& tb, hipStream_t s) {
-    if (f.count == 0) return hipSuccess;
-    constexpr int kU = 4;  // 64-fragment chunks per wave
-    const uint32_t blocks = (uint32_t)((f.count + kBlock * kU - 1) / (kBlock * kU));
-    hipLaunchKernelGGL((k_loop64_classify<K, kU>), dim3(blocks), dim3(kBlock), 0, s, c, f, slots, big, tb);
-    return hipGetLastError();
-  }
-};
-
-template <int K>
-struct Loop64Resolve {
-  static hipError_t run(const Common& c, uint64_t* slots, uint32_t* cnt, const TailBuf& tb, const ResolveOut& o,
-                        hipStream_t s) {
-    const bool dbg = o.fk_key || o.fk_val || o.counts;
-    const bool ctail = c.tail && tb.head != nullptr;
-    const dim3 g(blocks_for(c.T)), b(kBlock);
-#define OIT_L64(CT, DBG) hipLaunchKernelGGL((k_loop64_resolve<K, CT, DBG>), g, b, 0, s, c, slots, cnt, tb, o)
-    if (ctail) { if (dbg) OIT_L64(true, true); else OIT_L64(true, false); }
-    else { if (dbg) OIT_L64(false, true); else OIT_L64(false, false); }
-#undef OIT_L64
     return hipGetLastError();
   }
 };
@@ -3370,30 +2008,6 @@ hipError_t launch_kbuf_resolve(const Common& c, const KBuf& kb, const TailBuf& t
   return dispatch_k<KBufResolve>(c.K, c, kb, tb, o, s);
 }
 
-hipError_t launch_loop64_count(const Common& c, const FragView& f, uint32_t* cnt, hipStream_t s) {
-  if (f.count == 0) return hipSuccess;
-  constexpr int kU = 4;
-  const uint32_t blocks = (uint32_t)((f.count + kBlock * kU - 1) / (kBlock * kU));
-  hipLaunchKernelGGL((k_loop64_count<kU>), dim3(blocks), dim3(kBlock), 0, s, c, f, cnt);
-  return hipGetLastError();
-}
-
-hipError_t launch_loop64_store(const Common& c, const FragView& f, uint64_t* slots, uint32_t* cnt, uint64_t* big,
-                               int chunks, hipStream_t s) {
-  return dispatch_k<Loop64Store>(c.K, c, f, slots, cnt, big, chunks, s);
-}
-
-hipError_t launch_loop64_classify(const Common& c, const FragView& f, const uint64_t* slots, const uint64_t* big,
-                                  const TailBuf& tb, hipStream_t s) {
-  if (f.count == 0) return hipSuccess;
-  return dispatch_k<Loop64Classify>(c.K, c, f, slots, big, tb, s);
-}
-
-hipError_t launch_loop64_resolve(const Common& c, uint64_t* slots, uint32_t* cnt, const TailBuf& tb,
-                                 const ResolveOut& o, hipStream_t s) {
-  return dispatch_k<Loop64Resolve>(c.K, c, slots, cnt, tb, o, s);
-}
-
 hipError_t launch_wboit_store(const Common& c, const FragView& f, const WBBuf& wb, float view_near, float view_span,
                               hipStream_t s) {
   if (f.count == 0) return hipSuccess;
@@ -3532,45 +2146,6 @@ hipError_t launch_kbuf_resolve_cov(const Common& c, const KBuf& kb, const TailBu
 namespace {
 
 template <int K>
-struct Loop32Depth {
-  static hipError_t run(const Common& c, const FragView& f, uint32_t* zs, hipStream_t s) {
-    if (f.count == 0) return hipSuccess;
-    constexpr int kU = 2;  // 64-fragment chunks per wave
-    const uint32_t blocks = (uint32_t)((f.count + kBlock * kU - 1) / (kBlock * kU));
-    hipLaunchKernelGGL((k_loop32_depth_m<K, kU>), dim3(blocks), dim3(kBlock), 0, s, c, f, zs);
-    return hipGetLastError();
-  }
-};
-
-template <int K>
-struct Loop32Color {
-  static hipError_t run(const Common& c, const FragView& f, const uint32_t* zs, uint64_t* cs, const TailBuf& tb,
-                        hipStream_t s) {
-    if (f.count == 0) return hipSuccess;
-    constexpr int kU = 2;  // 64-fragment chunks per wave
-    const dim3 g((uint32_t)((f.count + kBlock * kU - 1) / (kBlock * kU))), b(kBlock);
-    if (c.tail && tb.head) hipLaunchKernelGGL((k_loop32_color_m<K, true, kU>), g, b, 0, s, c, f, zs, cs, tb);
-    else hipLaunchKernelGGL((k_loop32_color_m<K, false, kU>), g, b, 0, s, c, f, zs, cs, tb);
-    return hipGetLastError();
-  }
-};
-
-template <int K>
-struct Loop32Resolve {
-  static hipError_t run(const Common& c, uint32_t* zs, uint64_t* cs, const TailBuf& tb, const ResolveOut& o,
-                        hipStream_t s) {
-    const bool dbg = o.fk_key || o.fk_val || o.counts;
-    const bool ctail = c.tail && tb.head != nullptr;
-    const dim3 g(blocks_for(c.T)), b(kBlock);
-#define OIT_L32(CT, DBG) hipLaunchKernelGGL((k_loop32_resolve<K, CT, DBG>), g, b, 0, s, c, zs, cs, tb, o)
-    if (ctail) { if (dbg) OIT_L32(true, true); else OIT_L32(true, false); }
-    else { if (dbg) OIT_L32(false, true); else OIT_L32(false, false); }
-#undef OIT_L32
-    return hipGetLastError();
-  }
-};
-
-template <int K>
 struct InterlockResolve {
   static hipError_t run(const Common& c, const LLBuf& ll, const ResolveOut& o, hipStream_t s) {
     uint32_t blocks = blocks_for(c.T);
@@ -3585,22 +2160,6 @@ struct InterlockResolve {
 };
 
 }  // namespace
-
-hipError_t launch_loop32_depth(const Common& c, const FragView& f, uint32_t* zs, hipStream_t s) {
-  if (f.count == 0) return hipSuccess;
-  return dispatch_k<Loop32Depth>(c.K, c, f, zs, s);
-}
-
-hipError_t launch_loop32_color(const Common& c, const FragView& f, const uint32_t* zs, uint64_t* cs,
-                               const TailBuf& tb, hipStream_t s) {
-  if (f.count == 0) return hipSuccess;
-  return dispatch_k<Loop32Color>(c.K, c, f, zs, cs, tb, s);
-}
-
-hipError_t launch_loop32_resolve(const Common& c, uint32_t* zs, uint64_t* cs, const TailBuf& tb, const ResolveOut& o,
-                                 hipStream_t s) {
-  return dispatch_k<Loop32Resolve>(c.K, c, zs, cs, tb, o, s);
-}
 
 hipError_t launch_interlock_resolve(const Common& c, const LLBuf& ll, const ResolveOut& o, hipStream_t s) {
   if (!ll.full || (c.cov > 1u && !ll.mask)) return hipErrorInvalidValue;

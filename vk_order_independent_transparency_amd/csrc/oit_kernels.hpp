@@ -153,6 +153,79 @@ hipError_t launch_bin_prepare(const BatchArgs& a, const LLBuf& ll, uint32_t tile
 hipError_t launch_bin_resolve(const BatchArgs& a, const LLBuf& ll, uint32_t K, bool tail, uint32_t grid_cap,
                               hipStream_t s);
 
+// ---- Tile path (oit_tiles.hip) --------------------------------------------
+// Tiles of 64 consecutive targets (in list order: pixel-major under sample
+// shading); a frame's fragments as runs per tile.
+constexpr uint32_t kTileRuns = 64;        // runs in a tile's own slots, and its lists for later ones
+constexpr uint32_t kTileTails = 64;       // ctl: first tail counter
+constexpr uint32_t kTileTailWords = 64;   // tail fragments, counted by tile number mod 64
+constexpr uint32_t kTileCtlWords = kTileTails + kTileTailWords;
+constexpr uint32_t kTileShares = kTileCtlWords;  // ctl: shares of a tile that have ended (frames of few tiles); 0 between frames
+constexpr uint32_t kSharedTiles = 4096;
+constexpr uint32_t kTileCtlAll = kTileShares + kSharedTiles;
+constexpr uint32_t kDeepBlocks = 1024;    // waves of the deep composite (tickets hand out its tiles)
+inline uint64_t tile_count(uint64_t targets) { return (targets + 63u) / 64u; }
+
+struct TileBuf {
+  uint32_t* cnt = nullptr;   // [tiles] runs of the frame; 0 between frames
+  uint64_t* run = nullptr;   // [tiles][kTileRuns] first id << 32 | length
+  uint32_t* more = nullptr;  // [tiles][kTileRuns] later runs: first id + 1 of each list's last one, 0 = empty
+  uint64_t* link = nullptr;  // [fragments] of a later run, at its first id: length << 32 | the list's next value
+  uint32_t* deep = nullptr;  // [tiles] queue of the tiles left to the deep composite
+  uint32_t* ctl = nullptr;   // [kTileCtlAll] queue length and ticket per group, tail counters (zeroed by the appends), shares
+  uint32_t deep_base = 0;    // the group's part of the queue
+  uint32_t ctl_index = 0;    // the group's queue length in ctl (its ticket follows)
+};
+// Part of a frame's fragments in the caller's arrays.
+struct TileSeg {
+  const uint32_t* target;
+  const float* depth;
+  const float4* rgba;
+  uint32_t id_base;
+  uint32_t pad;
+};
+constexpr uint32_t kSegArgs = 64;
+struct SegArgs {
+  TileSeg s[kSegArgs];
+  uint32_t n;
+};
+struct TileSrc {
+  TileSeg one{};                  // the only segment
+  const TileSeg* segs = nullptr;  // nseg > 1: the segments, ascending first ids
+  uint32_t nseg = 1;
+  uint32_t T = 0, spp = 1;        // targets and samples per pixel of the frame
+  uint64_t frags = 0;             // fragments of the frame
+  const uint64_t* cd = nullptr;   // stored payloads (depth key << 32 | packed colour) by id, and list index mod 64
+  const uint8_t* loc = nullptr;
+};
+struct TileDst {
+  float4* out = nullptr;          // [T]
+  uint32_t* fk_key = nullptr;     // as ResolveOut
+  uint32_t* fk_val = nullptr;
+  uint32_t* counts = nullptr;
+  uint32_t T = 0, spp = 1;
+  uint32_t tile0 = 0;             // the frame's first tile
+  float4 background{};
+  const float4* rgba = nullptr;   // the opaque pass's colours, or null
+  const CodecTables* tab = nullptr;
+};
+// Order and tail of a composite: the Linked List (by depth, then id; evicted
+// colours blended in walk order), Loop64 (by depth, then packed colour; the
+// rest blended in id order with packed colours), Loop32 (one layer per
+// depth, the newest fragment's; the rest with full colours), the Spinlock
+// (by depth, then id; the rest in id order with packed colours).
+enum TileMode { kTileList = 0, kTileLoop64, kTileLoop32, kTileKBuf };
+// Pass 1 of one append.
+hipError_t launch_tile_link(const Common& c, const FragView& f, const TileBuf& tb, hipStream_t s);
+// Writes a segment table to the device (kernel arguments, no copy).
+hipError_t launch_set_segs(const TileSeg* segs, uint32_t n, TileSeg* dst, hipStream_t s);
+// Composite; returns the run structures to their clear values.
+hipError_t launch_tile_resolve(const TileBuf& tb, const TileSrc& src, const TileDst& dst, uint32_t K, int mode,
+                               bool tail, hipStream_t s);
+template <int K>  // its case of one layer count
+hipError_t tile_resolve_k(const TileBuf& tb, const TileSrc& src, const TileDst& dst, int mode, bool tail,
+                          hipStream_t s);
+
 hipError_t launch_ll_store(const Common& c, const FragView& f, const LLBuf& ll, const TailBuf& tb, hipStream_t s);
 hipError_t launch_ll_link(const Common& c, const FragView& f, const LLBuf& ll, hipStream_t s);
 // Fused colour pass: store + ordered link in one kernel. Requires next[] of
@@ -170,21 +243,6 @@ hipError_t launch_simple_store(const Common& c, const FragView& f, const KBuf& k
 hipError_t launch_spin_store(const Common& c, const FragView& f, const KBuf& kb, const TailBuf& tb, hipStream_t s);
 hipError_t launch_kbuf_resolve(const Common& c, const KBuf& kb, const TailBuf& tb, const ResolveOut& o, hipStream_t s);
 
-// chunks: 64-fragment chunks per wave (1: one fragment per lane; 2 or 4:
-// every chunk's loads and chain steps in flight together)
-// Per-target counts of a segment's fragments (at append).
-hipError_t launch_loop64_count(const Common& c, const FragView& f, uint32_t* cnt, hipStream_t s);
-// The stores of a segment, once every segment of the frame is counted;
-// `big` gets one mask per 64-fragment chunk of the segment (lanes whose
-// pixel holds more than K fragments).
-hipError_t launch_loop64_store(const Common& c, const FragView& f, uint64_t* slots, uint32_t* cnt, uint64_t* big,
-                               int chunks, hipStream_t s);
-hipError_t launch_loop64_classify(const Common& c, const FragView& f, const uint64_t* slots, const uint64_t* big,
-                                  const TailBuf& tb, hipStream_t s);
-// Also sets the slots it reads back to empty.
-hipError_t launch_loop64_resolve(const Common& c, uint64_t* slots, uint32_t* cnt, const TailBuf& tb,
-                                 const ResolveOut& o, hipStream_t s);
-
 hipError_t launch_wboit_store(const Common& c, const FragView& f, const WBBuf& wb, float view_near, float view_span,
                               hipStream_t s);
 hipError_t launch_wboit_resolve(const Common& c, const WBBuf& wb, const ResolveOut& o, hipStream_t s);
@@ -197,14 +255,6 @@ hipError_t launch_ll_resolve_cov(const Common& c, const LLBuf& ll, const TailBuf
                                  hipStream_t s);
 hipError_t launch_kbuf_resolve_cov(const Common& c, const KBuf& kb, const TailBuf& tb, const ResolveOut& o,
                                    hipStream_t s);
-// Loop32 (oitLoop.frag.glsl): depth pass per append, colour pass per append
-// at resolve time, composite
-hipError_t launch_loop32_depth(const Common& c, const FragView& f, uint32_t* zs, hipStream_t s);
-hipError_t launch_loop32_color(const Common& c, const FragView& f, const uint32_t* zs, uint64_t* cs,
-                               const TailBuf& tb, hipStream_t s);
-// Also sets the slots it reads back to empty.
-hipError_t launch_loop32_resolve(const Common& c, uint32_t* zs, uint64_t* cs, const TailBuf& tb, const ResolveOut& o,
-                                 hipStream_t s);
 // ordered interlock: Linked List append with shaded colours, then per-pixel
 // critical sections replayed in primitive order
 hipError_t launch_interlock_resolve(const Common& c, const LLBuf& ll, const ResolveOut& o, hipStream_t s);

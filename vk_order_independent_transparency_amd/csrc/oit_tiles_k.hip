@@ -1,0 +1,13 @@
+// oit_tiles_k.hip - the tile path's composites for one layer count
+// (OIT_TILE_K, one object per value: they compile side by side).
+#include "oit_tiles.hpp"
+
+namespace oit {
+
+template <>
+hipError_t tile_resolve_k<OIT_TILE_K>(const TileBuf& tb, const TileSrc& src, const TileDst& dst, int mode, bool tail,
+                                      hipStream_t s) {
+  return TileResolve<OIT_TILE_K>::run(tb, src, dst, mode, tail, s);
+}
+
+}  // namespace oit
