@@ -13,6 +13,14 @@
 // The per-frame semantics are those of the single-frame Linked List
 // (oitLinkedList.frag.glsl:51-85 append, :106-172 composite); a pool sized
 // from the exact fragment counts never overflows, so no colour-pass tail.
+//
+// By default nothing is linked per target: the frames go through the tile
+// path (oit_tiles.hpp), whose composite reads the callers' fragments itself,
+// since they stay valid until the run has ended. The 24-frame mix (205 M
+// fragments, 155 to 2810 spheres a frame, a fifth clustered) takes 2.9 ms so
+// and 6.9 ms with lists, whose ordered inserts walk past each other on the
+// clustered pixels. A tuning that asks for anything but the defaults gets the
+// list or bucket kernels it names.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -96,7 +104,8 @@ bool same_table(const std::vector<BatchFrameDev>& a, const std::vector<BatchFram
 
 // Frames with at least `bin_density` fragments per target are binned
 // (bucket per target) instead of linked (list per target).
-int make_plan(const oit_batch_frame* fr, uint32_t n, Plan& p, float bin_density) {
+// `schedule`: with the interleaved append schedule of the lists.
+int make_plan(const oit_batch_frame* fr, uint32_t n, Plan& p, float bin_density, bool schedule = true) {
   if (n > 0 && !fr) return OIT_ERR_INVALID_ARG;
   std::vector<uint32_t> order(n);
   for (uint32_t i = 0; i < n; ++i) {
@@ -164,6 +173,9 @@ int make_plan(const oit_batch_frame* fr, uint32_t n, Plan& p, float bin_density)
   }
   p.pool_slots = frag;
   p.heads = tgt;
+  p.rounds = 0;
+  p.sched.clear();
+  if (!schedule) return OIT_OK;
   // interleaved append: up to kRounds rounds; round q takes slices
   // floor(q S / R) .. floor((q + 1) S / R) - 1 of every frame
   uint64_t max_slices = 0;
@@ -230,7 +242,12 @@ struct oit_batch {
   uint32_t* deep_q = nullptr;
   uint32_t* tile_sum = nullptr;
   uint32_t* deep_n = nullptr;
-  bool dirty = false;            // a run did not complete: re-initialise before the next
+  // tile path: run structures per tile of 64 heads, links per fragment
+  oit::TileBuf tile;
+  uint64_t cap_tile_heads = 0, cap_tile_frags = 0;
+  bool prefer_lists = false;     // the tuner found the lists faster on its frames
+  bool dirty = false;            // a run did not complete: re-initialise before the next (lists)
+  bool tile_dirty = false;       // likewise (tile path)
   // frame table
   BatchFrameDev* d_table = nullptr;
   BatchFrameDev* h_table = nullptr;  // pinned staging
@@ -242,6 +259,7 @@ struct oit_batch {
   bool table_ev_pending = false;
   std::vector<BatchFrameDev> uploaded;
   bool uploaded_valid = false;
+  bool uploaded_sched = false;
   // concurrency and graphs
   hipStream_t side[kSide] = {};
   hipEvent_t fork_ev = nullptr;
@@ -257,6 +275,14 @@ struct oit_batch {
 
 namespace {
 
+void drop_tiles(oit_batch* b) {
+  for (void* q : {(void*)b->tile.cnt, (void*)b->tile.run, (void*)b->tile.more, (void*)b->tile.deep,
+                  (void*)b->tile.link, (void*)b->tile.bucket, (void*)b->tile.ctl})
+    (void)hipFree(q);
+  b->tile = oit::TileBuf{};
+  b->cap_tile_heads = b->cap_tile_frags = 0;
+}
+
 void release(oit_batch* b) {
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
   (void)hipFree(b->d_tab);
@@ -268,6 +294,7 @@ void release(oit_batch* b) {
   (void)hipFree(b->deep_q);
   (void)hipFree(b->tile_sum);
   (void)hipFree(b->deep_n);
+  drop_tiles(b);
   (void)hipFree(b->d_table);
   if (b->h_table) (void)hipHostFree(b->h_table);
   (void)hipFree(b->d_sched);
@@ -339,6 +366,68 @@ int ensure_pool(oit_batch* b, uint64_t nodes, uint64_t heads, hipStream_t s) {
   return OIT_OK;
 }
 
+bool same_tuning(const oit_batch_tuning& a, const oit_batch_tuning& t) { return std::memcmp(&a, &t, sizeof a) == 0; }
+
+bool tile_path(const oit_batch* b) { return !b->prefer_lists && same_tuning(b->tuning, default_tuning()); }
+
+// Bytes of the tile path's structures.
+uint64_t tile_bytes(uint64_t frags, uint64_t heads) {
+  return frags * 20u + oit::tile_count(heads) * (8u + oit::kTileRuns * 12u);
+}
+
+// Grows the tile path's structures (never shrinks) and clears new ones.
+int ensure_tiles(oit_batch* b, uint64_t frags, uint64_t heads, hipStream_t s) {
+  int rc;
+  if (frags > b->cap_tile_frags || heads > b->cap_tile_heads) {
+    if ((rc = st(hipDeviceSynchronize()))) return rc;
+    if (b->gexec) {  // captured launches hold the old pointers
+      (void)hipGraphExecDestroy(b->gexec);
+      b->gexec = nullptr;
+    }
+  }
+  if (frags > b->cap_tile_frags) {
+    (void)hipFree(b->tile.link);
+    (void)hipFree(b->tile.bucket);
+    b->tile.link = b->tile.bucket = nullptr;
+    b->cap_tile_frags = 0;
+    const uint64_t want = round_up(frags, 1ull << 20);
+    const uint64_t cap = want < kMaxPoolSlots ? want : frags;
+    if ((rc = st(hipMalloc((void**)&b->tile.link, cap * sizeof(uint64_t))))) return rc;
+    if ((rc = st(hipMalloc((void**)&b->tile.bucket, (cap + cap / 2u) * sizeof(uint64_t))))) return rc;
+    b->cap_tile_frags = cap;
+  }
+  bool fill = b->tile_dirty;
+  if (heads > b->cap_tile_heads) {
+    (void)hipFree(b->tile.cnt);
+    (void)hipFree(b->tile.run);
+    (void)hipFree(b->tile.more);
+    (void)hipFree(b->tile.deep);
+    b->tile.cnt = b->tile.more = b->tile.deep = nullptr;
+    b->tile.run = nullptr;
+    b->cap_tile_heads = 0;
+    const uint64_t cap = round_up(heads, 1ull << 16), tiles = oit::tile_count(cap);
+    if ((rc = st(hipMalloc((void**)&b->tile.cnt, tiles * sizeof(uint32_t))))) return rc;
+    if ((rc = st(hipMalloc((void**)&b->tile.run, tiles * oit::kTileRuns * sizeof(uint64_t))))) return rc;
+    if ((rc = st(hipMalloc((void**)&b->tile.more, tiles * oit::kTileRuns * sizeof(uint32_t))))) return rc;
+    if ((rc = st(hipMalloc((void**)&b->tile.deep, tiles * sizeof(uint32_t))))) return rc;
+    b->cap_tile_heads = cap;
+    fill = true;
+  }
+  if (!b->tile.ctl) {
+    if ((rc = st(hipMalloc((void**)&b->tile.ctl, oit::kTileCtlBatch * sizeof(uint32_t))))) return rc;
+    fill = true;
+  }
+  if (fill && b->cap_tile_heads) {
+    const uint64_t tiles = oit::tile_count(b->cap_tile_heads);
+    const oit::FillRange r[3] = {{b->tile.cnt, tiles, 0u},
+                                 {b->tile.more, tiles * oit::kTileRuns, 0u},
+                                 {b->tile.ctl, oit::kTileCtlBatch, 0u}};
+    if ((rc = st(oit::launch_fill_ranges(r, 3, s)))) return rc;
+  }
+  b->tile_dirty = false;
+  return OIT_OK;
+}
+
 int ensure_table(oit_batch* b, uint32_t n) {
   if (n <= b->table_cap) return OIT_OK;
   int rc;
@@ -366,7 +455,8 @@ int ensure_table(oit_batch* b, uint32_t n) {
 int upload_table(oit_batch* b, const Plan& p, hipStream_t s) {
   int rc;
   if ((rc = ensure_table(b, (uint32_t)p.table.size()))) return rc;
-  if (b->uploaded_valid && same_table(b->uploaded, p.table)) return OIT_OK;
+  // (a table uploaded without a schedule is uploaded again for the lists)
+  if (b->uploaded_valid && (p.sched.empty() || b->uploaded_sched) && same_table(b->uploaded, p.table)) return OIT_OK;
   if (p.table.empty()) return OIT_OK;
   if (b->table_ev_pending) {  // the previous copy has read the staging buffer
     if ((rc = st(hipEventSynchronize(b->table_ev)))) return rc;
@@ -389,17 +479,18 @@ int upload_table(oit_batch* b, const Plan& p, hipStream_t s) {
     b->sched_cap = cap;
   }
   std::memcpy(b->h_table, p.table.data(), p.table.size() * sizeof(BatchFrameDev));
-  std::memcpy(b->h_sched, p.sched.data(), p.sched.size() * sizeof(uint32_t));
+  if (!p.sched.empty()) std::memcpy(b->h_sched, p.sched.data(), p.sched.size() * sizeof(uint32_t));
   if ((rc = st(hipMemcpyAsync(b->d_table, b->h_table, p.table.size() * sizeof(BatchFrameDev),
                               hipMemcpyHostToDevice, s))))
     return rc;
-  if ((rc = st(hipMemcpyAsync(b->d_sched, b->h_sched, p.sched.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
-                              s))))
+  if (!p.sched.empty() && (rc = st(hipMemcpyAsync(b->d_sched, b->h_sched, p.sched.size() * sizeof(uint32_t),
+                                                  hipMemcpyHostToDevice, s))))
     return rc;
   if ((rc = st(hipEventRecord(b->table_ev, s)))) return rc;
   b->table_ev_pending = true;
   b->uploaded = p.table;
   b->uploaded_valid = true;
+  b->uploaded_sched = !p.sched.empty();
   return OIT_OK;
 }
 
@@ -418,6 +509,33 @@ BatchArgs args_for(const oit_batch* b, const Plan& p) {
   a.deep_n = b->deep_n;
   a.cursor_cap = (uint32_t)b->cap_heads;
   return a;
+}
+
+// A group's run structures: its part of the deep queue, its counters, its
+// shares.
+oit::TileBuf group_tiles(const oit_batch* b, const Group& g, uint32_t gi) {
+  oit::TileBuf t = b->tile;
+  t.tile_first = g.tile0 * (kTile / 64u);
+  t.deep_base = t.tile_first;
+  t.ctl_index = 2u * gi;
+  t.share0 = oit::kTileShares + gi * oit::kSharedTiles;
+  t.ticket0 = oit::kTileTickets + gi * oit::kTicketWords;
+  return t;
+}
+
+int launch_tile_link(const oit_batch* b, const Plan& p, hipStream_t s) {
+  BatchArgs a = args_for(b, p);
+  a.units = (uint32_t)(p.pool_slots / 512u);
+  return st(oit::launch_tile_link_batch(a, b->tile, s));
+}
+
+int launch_tile_group(const oit_batch* b, const Plan& p, const Group& g, uint32_t gi, hipStream_t s) {
+  BatchArgs a = args_for(b, p);
+  a.f0 = g.f0;
+  a.f1 = g.f1;
+  a.tile0 = g.tile0;
+  a.tiles = g.tiles;
+  return st(oit::launch_tile_batch(a, group_tiles(b, g, gi), g.K, g.tail != 0, s));
 }
 
 int launch_append(const oit_batch* b, const Plan& p, uint32_t chunks, hipStream_t s) {
@@ -455,8 +573,13 @@ int launch_group(const oit_batch* b, const Plan& p, const Group& g, uint32_t gi,
 // Append + every group's resolve on s (resolve groups forked when asked).
 int enqueue(oit_batch* b, const Plan& p, hipStream_t s) {
   int rc;
-  if ((rc = launch_append(b, p, b->tuning.append_chunks, s))) return rc;
-  if ((rc = launch_bin(b, p, b->tuning.append_chunks, s))) return rc;
+  const bool tiles = tile_path(b);
+  if (tiles) {
+    if ((rc = launch_tile_link(b, p, s))) return rc;
+  } else {
+    if ((rc = launch_append(b, p, b->tuning.append_chunks, s))) return rc;
+    if ((rc = launch_bin(b, p, b->tuning.append_chunks, s))) return rc;
+  }
   const bool fork = (b->flags & OIT_BATCH_CONCURRENT) && p.groups.size() > 1;
   if (fork && (rc = st(hipEventRecord(b->fork_ev, s)))) return rc;
   bool used[kSide] = {};
@@ -472,9 +595,10 @@ int enqueue(oit_batch* b, const Plan& p, hipStream_t s) {
         used[j] = true;
       }
     }
-    if ((rc = launch_group(b, p, gr, (uint32_t)g, b->tuning.resolve_variant[ki][gr.tail],
-                           b->tuning.resolve_blocks[ki][gr.tail], gs)))
-      return rc;
+    if (tiles) rc = launch_tile_group(b, p, gr, (uint32_t)g, gs);
+    else rc = launch_group(b, p, gr, (uint32_t)g, b->tuning.resolve_variant[ki][gr.tail],
+                           b->tuning.resolve_blocks[ki][gr.tail], gs);
+    if (rc) return rc;
   }
   for (int j = 0; j < kSide; ++j) {
     if (!used[j]) continue;
@@ -516,10 +640,26 @@ int run_graph(oit_batch* b, const Plan& p, hipStream_t s) {
   return st(hipGraphLaunch(b->gexec, s));
 }
 
+// Grows what the path in use needs for these pool nodes and heads. The tile
+// path takes 20 bytes a fragment, the lists 12: without memory for the one,
+// the batch goes over to the other.
+int ensure_path(oit_batch* b, uint64_t nodes, uint64_t heads, hipStream_t s) {
+  if (tile_path(b)) {
+    const int rc = ensure_tiles(b, nodes ? nodes - 1u : 0u, heads, s);
+    if (rc != OIT_ERR_OOM) return rc;
+    drop_tiles(b);
+    b->prefer_lists = true;
+    ++b->tuning_version;
+  }
+  return ensure_pool(b, nodes, heads, s);
+}
+
 int prepare(oit_batch* b, const oit_batch_frame* frames, uint32_t n, Plan& p, hipStream_t s) {
   int rc;
-  if ((rc = make_plan(frames, n, p, b->tuning.bin_density))) return rc;
-  return ensure_pool(b, p.pool_slots + 1, p.heads, s);
+  const bool tiles = tile_path(b);
+  if ((rc = make_plan(frames, n, p, b->tuning.bin_density, !tiles))) return rc;
+  if ((rc = ensure_path(b, p.pool_slots + 1, p.heads, s))) return rc;
+  return tiles && !tile_path(b) ? make_plan(frames, n, p, b->tuning.bin_density) : OIT_OK;
 }
 
 }  // namespace
@@ -578,8 +718,9 @@ int oit_batch_query(const oit_batch* b, const oit_batch_frame* frames, uint32_t 
   if (rc) return rc;
   out->pool_nodes = p.pool_slots + 1;
   out->head_entries = p.heads;
-  // nodes 12 B; per head: the head, a bucket cursor and a deep-queue entry; a scan base per tile
-  out->bytes = out->pool_nodes * 12u + out->head_entries * 12u + out->head_entries / kTile * 4u;
+  // lists: nodes 12 B; per head: the head, a bucket cursor and a deep-queue entry; a scan base per tile
+  out->bytes = tile_path(b) ? tile_bytes(p.pool_slots, p.heads)
+                            : out->pool_nodes * 12u + out->head_entries * 12u + out->head_entries / kTile * 4u;
   out->groups = (uint32_t)p.groups.size();
   out->frames = n;
   return OIT_OK;
@@ -589,7 +730,7 @@ int oit_batch_reserve(oit_batch* b, uint64_t pool_nodes, uint64_t head_entries) 
   if (!b) return OIT_ERR_INVALID_ARG;
   if (pool_nodes > kMaxPoolSlots + 1 || head_entries > kMaxHeads) return OIT_ERR_CAPACITY;
   DeviceGuard g(b->device);
-  const int rc = ensure_pool(b, pool_nodes, head_entries, nullptr);
+  const int rc = ensure_path(b, pool_nodes, head_entries, nullptr);
   if (rc) return rc;
   return st(hipStreamSynchronize(nullptr));
 }
@@ -608,7 +749,7 @@ int oit_batch_run(oit_batch* b, const oit_batch_frame* frames, uint32_t n, void*
     rc = upload_table(b, p, s);
     if (!rc) rc = enqueue(b, p, s);
   }
-  if (rc) b->dirty = true;
+  if (rc) b->dirty = b->tile_dirty = true;
   return rc;
 }
 
@@ -617,8 +758,13 @@ int oit_batch_tune(oit_batch* b, const oit_batch_frame* frames, uint32_t n, void
   DeviceGuard g(b->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
   Plan p;
-  int rc = prepare(b, frames, n, p, s);
+  int rc = make_plan(frames, n, p, b->tuning.bin_density);
   if (rc) return rc;
+  rc = ensure_tiles(b, p.pool_slots, p.heads, s);
+  const bool no_tiles = rc == OIT_ERR_OOM;
+  if (no_tiles) drop_tiles(b);
+  else if (rc) return rc;
+  if ((rc = ensure_pool(b, p.pool_slots + 1, p.heads, s))) return rc;
   if (p.table.empty()) return OIT_OK;
   if ((rc = upload_table(b, p, s))) return rc;
   const size_t G = p.groups.size();
@@ -728,13 +874,39 @@ int oit_batch_tune(oit_batch* b, const oit_batch_frame* frames, uint32_t n, void
       }
     }
   }
+  // the whole run: the best of the lists' choices against the tile path
+  float lists_ms = 0.f, tiles_ms = 0.f;
+  for (int rep = 0; rep < 6 && !rc && !no_tiles; ++rep) {
+    const bool tiles = (rep & 1) != 0;
+    if ((rc = st(hipEventRecord(ev[0], s)))) break;
+    if (tiles) {
+      rc = launch_tile_link(b, p, s);
+    } else {
+      rc = launch_append(b, p, best.append_chunks, s);
+      if (!rc) rc = launch_bin(b, p, best.append_chunks, s);
+    }
+    for (size_t gi = 0; gi < G && !rc; ++gi) {
+      const Group& g = p.groups[gi];
+      const int ki = k_index(g.K);
+      rc = tiles ? launch_tile_group(b, p, g, (uint32_t)gi, s)
+                 : launch_group(b, p, g, (uint32_t)gi, best.resolve_variant[ki][g.tail], best.resolve_blocks[ki][g.tail], s);
+    }
+    if (rc) break;
+    if ((rc = st(hipEventRecord(ev[1], s)))) break;
+    if ((rc = st(hipEventSynchronize(ev[1])))) break;
+    float ms = 0.f;
+    if ((rc = st(hipEventElapsedTime(&ms, ev[0], ev[1])))) break;
+    float& m = tiles ? tiles_ms : lists_ms;
+    if (rep < 2 || ms < m) m = ms;
+  }
   for (auto& e : ev)
     if (e) (void)hipEventDestroy(e);
   if (rc) {
-    b->dirty = true;
+    b->dirty = b->tile_dirty = true;
     return rc;
   }
-  b->tuning = best;
+  b->prefer_lists = no_tiles || lists_ms < tiles_ms;
+  b->tuning = b->prefer_lists ? best : default_tuning();
   ++b->tuning_version;
   return OIT_OK;
 }
@@ -748,6 +920,7 @@ int oit_batch_get_tuning(const oit_batch* b, oit_batch_tuning* out) {
 int oit_batch_set_tuning(oit_batch* b, const oit_batch_tuning* t) {
   if (!b || !t || !tuning_valid(*t)) return OIT_ERR_INVALID_ARG;
   b->tuning = *t;
+  b->prefer_lists = false;
   ++b->tuning_version;
   return OIT_OK;
 }

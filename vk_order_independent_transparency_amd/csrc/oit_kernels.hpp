@@ -159,10 +159,18 @@ hipError_t launch_bin_resolve(const BatchArgs& a, const LLBuf& ll, uint32_t K, b
 constexpr uint32_t kTileRuns = 64;        // runs in a tile's own slots, and its lists for later ones
 constexpr uint32_t kTileTails = 64;       // ctl: first tail counter
 constexpr uint32_t kTileTailWords = 64;   // tail fragments, counted by tile number mod 64
+constexpr uint32_t kTileBucket = kTileTails - 2u;  // ctl: entries of the bucket array given out (two words; batches)
 constexpr uint32_t kTileCtlWords = kTileTails + kTileTailWords;
 constexpr uint32_t kTileShares = kTileCtlWords;  // ctl: shares of a tile that have ended (frames of few tiles); 0 between frames
 constexpr uint32_t kSharedTiles = 4096;
 constexpr uint32_t kTileCtlAll = kTileShares + kSharedTiles;
+constexpr uint32_t kTileTickets = kTileShares + kBatchMaxGroups * kSharedTiles;  // a batch's groups run side by side
+// ctl, batches: the next queue entries of a group's binning and of its binned
+// composite: eight counters each, 64 bytes apart, counter c handing out the
+// entries c, c + 8, ... to the blocks c, c + 8, ... (one chiplet's)
+constexpr uint32_t kTicketLanes = 8;
+constexpr uint32_t kTicketWords = 2u * kTicketLanes * 16u;
+constexpr uint32_t kTileCtlBatch = kTileTickets + kBatchMaxGroups * kTicketWords;
 constexpr uint32_t kDeepBlocks = 1024;    // waves of the deep composite (tickets hand out its tiles)
 inline uint64_t tile_count(uint64_t targets) { return (targets + 63u) / 64u; }
 
@@ -175,6 +183,10 @@ struct TileBuf {
   uint32_t* ctl = nullptr;   // [kTileCtlAll] queue length and ticket per group, tail counters (zeroed by the appends), shares
   uint32_t deep_base = 0;    // the group's part of the queue
   uint32_t ctl_index = 0;    // the group's queue length in ctl (its ticket follows)
+  uint32_t share0 = kTileShares;  // the group's shares in ctl, from tile `tile_first` on
+  uint32_t tile_first = 0;
+  uint32_t ticket0 = 0;      // the group's tickets in ctl
+  uint64_t* bucket = nullptr;     // [fragments * 3 / 2] a batch's binned tiles: depth key << 32 | packed colour per target, oldest first
 };
 // Part of a frame's fragments in the caller's arrays.
 struct TileSeg {
@@ -225,6 +237,16 @@ hipError_t launch_tile_resolve(const TileBuf& tb, const TileSrc& src, const Tile
 template <int K>  // its case of one layer count
 hipError_t tile_resolve_k(const TileBuf& tb, const TileSrc& src, const TileDst& dst, int mode, bool tail,
                           hipStream_t s);
+
+// A batch's frames: pass 1 over every frame (a.units units of 512 fragments),
+// and the composite of a (K, tail) group's tiles (a.tile0, a.tiles in units
+// of 256 targets).
+hipError_t launch_tile_link_batch(const BatchArgs& a, const TileBuf& tb, hipStream_t s);
+// Puts the fragments of a group's queued tiles in order per target (tb.bucket).
+hipError_t launch_tile_bin(const BatchArgs& a, const TileBuf& tb, uint32_t tiles, uint32_t split, hipStream_t s);
+hipError_t launch_tile_batch(const BatchArgs& a, const TileBuf& tb, uint32_t K, bool tail, hipStream_t s);
+template <int K>
+hipError_t tile_batch_k(const BatchArgs& a, const TileBuf& tb, bool tail, hipStream_t s);
 
 hipError_t launch_ll_store(const Common& c, const FragView& f, const LLBuf& ll, const TailBuf& tb, hipStream_t s);
 hipError_t launch_ll_link(const Common& c, const FragView& f, const LLBuf& ll, hipStream_t s);

@@ -412,23 +412,44 @@ __device__ __forceinline__ uint32_t key_depth(double k) { return (hi32(k) << 2) 
 // (`deferred`), queues the tile for the deep composite, which writes all of
 // it, counts the tails of those shares and then clears. Queue entry: the
 // tile; with shares (at most kSharedTiles tiles) the deferred ones << 16 too.
+// `queue` (a batch, where many tiles are queued) collects a wave's entries:
+// one atomic on the queue's length for 64 of them. (An atomic each, on one
+// address, took as long as the composite.)
+struct TileQueue {
+  uint32_t n = 0, entry = 0;
+  __device__ __forceinline__ void flush(const TileBuf& tb) {
+    if (n == 0u) return;
+    uint32_t at = 0;
+    if (lane_id() == 0u) at = atomicAdd(&tb.ctl[tb.ctl_index], n);
+    at = rfl(at);
+    if (lane_id() < n) tb.deep[tb.deep_base + at + lane_id()] = entry;
+    n = 0u;
+  }
+  __device__ __forceinline__ void push(const TileBuf& tb, uint32_t e) {
+    if (lane_id() == n) entry = e;
+    if (++n == 64u) flush(tb);
+  }
+};
+
 __device__ __forceinline__ void end_share(const TileBuf& tb, uint32_t tile, uint32_t m, uint32_t first, uint32_t split,
-                                          bool deferred) {
+                                          bool deferred, TileQueue* queue) {
   uint32_t entry = tile;
   if (split > 0u) {
+    entry -= tb.tile_first;
     uint32_t sum = 0;
     if (lane_id() == 0u) {
       const uint32_t mine = 1u + (deferred ? 256u << (first >> (6u - split)) : 0u);
-      sum = mine + atomicAdd(&tb.ctl[kTileShares + tile], mine);
+      sum = mine + atomicAdd(&tb.ctl[tb.share0 + entry], mine);
     }
     sum = rfl(sum);
     if ((sum & 255u) != (1u << split)) return;
-    if (lane_id() == 0u) tb.ctl[kTileShares + tile] = 0u;
+    if (lane_id() == 0u) tb.ctl[tb.share0 + entry] = 0u;
     deferred = sum > 255u;
     entry |= (sum >> 8) << 16;
   }
   if (deferred) {
-    if (lane_id() == 0u) tb.deep[tb.deep_base + atomicAdd(&tb.ctl[tb.ctl_index], 1u)] = entry;
+    if (queue) queue->push(tb, entry);
+    else if (lane_id() == 0u) tb.deep[tb.deep_base + atomicAdd(&tb.ctl[tb.ctl_index], 1u)] = entry;
   } else {
     if (lane_id() == 0u) tb.cnt[tile] = 0u;
     if (m > kTileRuns) tb.more[(uint64_t)tile * kTileRuns + lane_id()] = 0u;
@@ -810,7 +831,8 @@ __device__ __forceinline__ TileAhead load_ahead(const TileBuf& tb, uint32_t tile
 // targets from `first` on: see the head of the file.
 template <int K, int kMode, bool kTail, bool kStored, bool kGeneral, typename Lds>
 __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_t split, const TileAhead& ahead, const TileBuf& tb, const TileSrc& src,
-                                          const TileDst& dst, Lds& w, const float* s_dec, const float* s_alpha) {
+                                          const TileDst& dst, Lds& w, const float* s_dec, const float* s_alpha,
+                                          TileQueue* queue) {
   const uint32_t lane = lane_id();
   const uint32_t a = (tile - dst.tile0) * kTileTargets + lane;  // list index in the frame
   const bool in = a < dst.T;
@@ -845,6 +867,12 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
       start = (uint32_t)(rec >> 32);
       len = (uint32_t)rec;
     }
+    if constexpr (kMode == kTileList) {
+      if ((__builtin_amdgcn_readlane(wave_scan_u32(len), 63) >> split) > cap) {  // binned instead
+        end_share(tb, tile, m, first, split, true, queue);
+        return;
+      }
+    }
     // the runs in ascending order of their first ids
     uint32_t rank = 0;
     for (uint32_t j = 0; j < m; ++j) rank += __builtin_amdgcn_readlane(start, j) < start ? 1u : 0u;
@@ -857,11 +885,14 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
     clear_marks(w);
     if (size <= kMaxPositions) mark_run(w, lane < m, incl - len);  // 64 runs of at most 64: always
     w.delta[lane] = start - (incl - len);
+  } else if constexpr (kMode == kTileList) {
+    end_share(tb, tile, m, first, split, true, queue);
+    return;
   } else {
     // short runs: gathered and sorted in the entries' space, of which their
     // deltas then take the end
     if (m > kManyRuns) {
-      end_share(tb, tile, m, first, split, true);
+      end_share(tb, tile, m, first, split, true, queue);
       return;
     }
     uint64_t* const run = reinterpret_cast<uint64_t*>(&w.e[0]);
@@ -883,7 +914,7 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
       if (c + lane < got) delta[c + lane] = (uint32_t)(rec >> 32) - off;
     }
     if (size > kMaxPositions) {
-      end_share(tb, tile, m, first, split, true);
+      end_share(tb, tile, m, first, split, true, queue);
       return;
     }
   }
@@ -892,13 +923,15 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
   // time, each part reading all of the runs and keeping its own fragments; a
   // part that is still too large is halved
   uint32_t shift = 6u - split;
-  while (shift > 0u && (size >> (6u - shift)) > cap) --shift;
+  if constexpr (kMode != kTileList) {
+    while (shift > 0u && (size >> (6u - shift)) > cap) --shift;
+  }
   for (uint32_t t0 = first; t0 < last;) {
     const uint32_t part = t0 >> shift;
     if (!build_lists<kStored, kGeneral>(w, src, dst.tab, deltas, id0, size, shift, part, cap)) {
       wave_lds_sync();
-      if (shift == 0u) {  // one target's fragments
-        end_share(tb, tile, m, first, split, true);
+      if (shift == 0u || kMode == kTileList) {  // one target's fragments
+        end_share(tb, tile, m, first, split, true, queue);
         return;
       }
       --shift;
@@ -930,7 +963,7 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
   if constexpr (kTail && kMode != kTileList) {
     if (__ballot(L.tails != 0u) != 0ull) count_tails(tb, tile, L.tails);
   }
-  end_share(tb, tile, m, first, split, false);
+  end_share(tb, tile, m, first, split, false, queue);
 }
 
 // ---------------------------------------------------------------------------
@@ -1307,7 +1340,7 @@ __global__ __launch_bounds__(kBlock, tile_waves<K>()) void k_tile_resolve(TileAr
     const TileAhead next = load_ahead(g.tb, (item + stride) >> split, tiles);
     const uint32_t first = (item & ((1u << split) - 1u)) << (6u - split);
     tile_wave<K, kMode, kTail, kStored, kGeneral>(item >> split, first, split, now, g.tb, g.src, g.dst, s_w[wave],
-                                                  s_dec, s_alpha);
+                                                  s_dec, s_alpha, nullptr);
     now = next;
   }
 }
@@ -1331,11 +1364,277 @@ __global__ __launch_bounds__(64) void k_tile_deep(TileArgs args) {
     q = rfl(q);
     if (q >= n) break;
     const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
-    const uint32_t tile = g.split ? entry & 0xFFFFu : entry, shares = g.split ? entry >> 16 : 1u;
+    const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
+    const uint32_t shares = g.split ? entry >> 16 : 1u;
     deep_wave<K, kMode, kTail, kStored>(tile, shares, g.split, g.tb, g.src, g.dst, w, s_dec, s_alpha);
     wave_lds_sync();
   }
 }
+
+constexpr uint32_t kTileDeepFlag = 1u << 31;  // queue entry of a batch: left to the deep composite
+
+// A batch group's frames: the same composite, each tile with its frame's
+// arrays and size.
+struct TileBatchArgs {
+  TileBuf tb;
+  const BatchFrameDev* frames;
+  uint32_t f0, f1;
+  uint32_t tile0, tiles, split;
+  const CodecTables* tab;
+};
+using BatchArgsPtr = const __attribute__((address_space(4))) TileBatchArgs*;
+__device__ __forceinline__ const TileBatchArgs& fresh_batch_args() {
+  auto p = (BatchArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const TileBatchArgs*)p;
+}
+using FramePtr = const __attribute__((address_space(4))) BatchFrameDev*;
+// The frame of a tile, from the frame of an earlier one on.
+__device__ __forceinline__ uint32_t next_frame(FramePtr fr, uint32_t f, uint32_t f1, uint32_t tile) {
+  while (f + 1u < f1 && fr[f + 1u].target_base <= (uint64_t)tile * kTileTargets) ++f;
+  return f;
+}
+__device__ __forceinline__ void frame_views(FramePtr fr, uint32_t f, const CodecTables* tab, TileSrc& src,
+                                            TileDst& dst) {
+  src.one.target = fr[f].target;
+  src.one.depth = fr[f].depth;
+  src.one.rgba = fr[f].rgba;
+  src.one.id_base = fr[f].frag_base;
+  src.T = dst.T = fr[f].T;
+  dst.tile0 = fr[f].target_base / kTileTargets;
+  dst.out = fr[f].out;
+  dst.background = make_float4(fr[f].background.x, fr[f].background.y, fr[f].background.z, fr[f].background.w);
+  dst.tab = tab;
+}
+
+template <int K, bool kTail>
+__global__ __launch_bounds__(kBlock, tile_waves<K>()) void k_tile_batch(TileBatchArgs args) {
+  __shared__ float s_dec[256];
+  __shared__ float s_alpha[256];
+  __shared__ TileLds<tile_entries(false), false> s_w[kBlock / 64];
+  stage_decode(s_dec, s_alpha, args.tab);
+  __syncthreads();
+  const uint32_t wave = rfl(threadIdx.x >> 6);
+  const uint32_t stride = gridDim.x * (kBlock / 64);
+  const uint32_t end = args.tile0 + args.tiles, split = args.split;
+  uint32_t item = (args.tile0 << split) + blockIdx.x * (kBlock / 64) + wave;
+  const uint32_t items = end << split;
+  if (item >= items) return;
+  TileAhead now = load_ahead(args.tb, item >> split, end);
+  uint32_t f = args.f0;
+  TileQueue queue;
+  for (; item < items; item += stride) {
+    const TileBatchArgs& g = fresh_batch_args();
+    const TileAhead next = load_ahead(g.tb, (item + stride) >> split, end);
+    const auto fr = (FramePtr)g.frames;
+    f = rfl(next_frame(fr, f, g.f1, item >> split));
+    TileSrc src;
+    TileDst dst;
+    frame_views(fr, f, g.tab, src, dst);
+    const uint32_t first = (item & ((1u << split) - 1u)) << (6u - split);
+    tile_wave<K, kTileList, kTail, false, false>(item >> split, first, split, now, g.tb, src, dst, s_w[wave], s_dec,
+                                                 s_alpha, &queue);
+    now = next;
+  }
+  queue.flush(args.tb);
+}
+
+// Sorted register array of K packed keys for a list walk (newest element
+// first), with the colours in an LDS column per lane: key = (depth key << 30)
+// | order << 6 | slot, where order falls with every element walked, so that
+// equal depths put the smaller id first, and slot is the element's place in
+// the lane's column of K + 1. An insert writes its colour to the free slot
+// and bubbles the key in; the slot of the key pushed out is the next free
+// one.
+template <int K>
+struct FrontS {
+  double v[K];
+  uint32_t free;  // the lane's free slot
+  uint32_t* col;  // the lane's column, slots kBlock words apart
+  __device__ __forceinline__ void init(uint32_t* column) {
+    uint32_t high = 0x3FFFFFFFu, low = 0xFFFFFFC0u;
+    asm volatile("" : "+v"(high), "+v"(low));  // or the sentinels are kept in registers across the tiles
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = pack2(high, low + (uint32_t)(k + 1));
+    free = 0u;
+    col = column;
+  }
+  // `step` is the element's place in the walk (below 2^24).
+  static __device__ __forceinline__ double key_of(uint64_t cd, uint32_t step, uint32_t slot) {
+    const uint32_t key = (uint32_t)(cd >> 32);
+    return pack2(key >> 2, (key << 30) | ((0xFFFFFFu - step) << 6) | slot);
+  }
+  // Returns the colour pushed out; a lane that is not `on` puts in a sentinel.
+  // The first step + 1 places can be occupied; those behind hold sentinels,
+  // one of which is pushed out (step is wave-uniform).
+  __device__ __forceinline__ uint32_t insert(uint64_t cd, uint32_t step, bool on) {
+    const double key = key_of(cd, step, free);
+    double x = pack2(on ? hi32(key) : 0x3FFFFFFFu, on ? lo32(key) : 0xFFFFFFC0u | free);
+    col[free * kBlock] = (uint32_t)cd;
+#pragma unroll
+    for (int b = 0; b < K; b += 4) {
+      if ((uint32_t)b <= step) {
+#pragma unroll
+        for (int j = b; j < b + 4 && j < K; ++j) {
+          double up;
+          asm("v_max_f64 %1, %0, %2\n\tv_min_f64 %0, %0, %2" : "+v"(v[j]), "=&v"(up) : "v"(x));
+          x = up;
+        }
+      }
+    }
+    free = lo32(x) & 63u;
+    return col[free * kBlock];
+  }
+  __device__ __forceinline__ uint32_t colour(int k) const { return col[(lo32(v[k]) & 63u) * kBlock]; }
+};
+
+// A binned target: its first place behind the tile's base and, in the high
+// bit, whether its entries lie 16 apart (a row of 16 targets) or follow each
+// other.
+constexpr uint32_t kBinRow = 1u << 31;
+__device__ __forceinline__ uint32_t bin_step(uint32_t at) { return at & kBinRow ? 16u : 1u; }
+__device__ __forceinline__ uint32_t bin_at(uint32_t at) { return at & ~kBinRow; }
+
+// The binned tiles' composite (k_tile_bin has put their fragments in order):
+// a wave per tile, a lane per target, each its bucket from the newest on.
+template <int K, bool kTail>
+__global__ __launch_bounds__(kBlock, K <= 8 ? 8 : (K <= 16 ? 6 : 4)) void k_tile_binned(TileBatchArgs args) {
+  const uint32_t n_tiles = rfl(ld_relaxed(&args.tb.ctl[args.tb.ctl_index]));
+  if (blockIdx.x / kTicketLanes * (kBlock / 64) * kTicketLanes >= n_tiles) return;
+  __shared__ float s_dec[256];
+  __shared__ float s_alpha[256];
+  __shared__ uint32_t s_col[(K + 1) * kBlock];
+  stage_decode(s_dec, s_alpha, args.tab);
+  __syncthreads();
+  const uint32_t lane = lane_id();
+  const uint32_t turn = blockIdx.x % kTicketLanes;
+  constexpr uint32_t kWaves = kBlock / 64;
+  uint32_t next = 0;
+  for (uint32_t q = (blockIdx.x / kTicketLanes * kWaves + rfl(threadIdx.x >> 6)) * kTicketLanes + turn; q < n_tiles;
+       q = rfl(next)) {
+    const TileBatchArgs& g = fresh_batch_args();
+    if (lane == 0u)
+      next = turn + gridDim.x * kWaves +
+             kTicketLanes * atomicAdd(&g.tb.ctl[g.tb.ticket0 + (kTicketLanes + turn) * 16u], 1u);
+    const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
+    if (entry & kTileDeepFlag) continue;  // the deep composite's
+    const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
+    const auto fr = (FramePtr)g.frames;
+    TileSrc src;
+    TileDst dst;
+    frame_views(fr, rfl(find_frame<true>(g.frames, g.f0, g.f1, (uint64_t)tile * kTileTargets)), g.tab, src, dst);
+    const auto* const bucket = (const __attribute__((address_space(1))) uint64_t*)g.tb.bucket;
+    const uint64_t rec = g.tb.run[(uint64_t)tile * kTileRuns + lane];
+    const uint32_t* const more = &g.tb.more[(uint64_t)tile * kTileRuns];
+    const uint64_t base = ((uint64_t)more[1] << 32) | more[0];
+    const uint32_t n = (uint32_t)(rec >> 32), most = wave_top_u32(n);
+    const uint32_t step = bin_step((uint32_t)rec), newest = bin_at((uint32_t)rec) + (n - 1u) * step;
+    const auto* const entry_of = bucket + base;
+    FrontS<K> a;
+    a.init(s_col + threadIdx.x);
+    float4 tailc = make_float4(0.f, 0.f, 0.f, 0.f);
+    constexpr uint32_t kU = 4;  // entries of a trip; the next trip's are on their way
+    uint64_t ahead[kU];
+#pragma unroll
+    for (uint32_t u = 0; u < kU; ++u) ahead[u] = entry_of[u < n ? newest - u * step : 0u];
+#pragma nounroll
+    for (uint32_t s = 0; s < most; s += kU) {
+      uint64_t cd[kU];
+#pragma unroll
+      for (uint32_t u = 0; u < kU; ++u) cd[u] = ahead[u];
+#pragma unroll
+      for (uint32_t u = 0; u < kU; ++u) ahead[u] = entry_of[s + kU + u < n ? newest - (s + kU + u) * step : 0u];
+      // most trips of a long list are behind the K in every lane
+      uint64_t front = s < (uint32_t)K ? 1ull : 0ull;
+#pragma unroll
+      for (uint32_t u = 0; u < kU; ++u)
+        front |= __ballot(s + u < n) & __ballot(a.key_of(cd[u], s + u, 0u) < a.v[K - 1]);
+      uint32_t behind[kU];  // what falls behind; 0 leaves the tail as it is
+#pragma unroll
+      for (uint32_t u = 0; u < kU; ++u) behind[u] = (uint32_t)cd[u];
+      if (front != 0ull) {
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) behind[u] = a.insert(cd[u], s + u, s + u < n);
+      }
+      if (kTail) {
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) {
+          const bool tail = s + u >= (uint32_t)K && s + u < n;
+          tailc = over(tailc, decode_premult_lds(tail ? behind[u] : 0u, s_dec, s_alpha));
+        }
+      }
+    }
+    float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+    {
+      if ((k & 3) == 0) asm volatile("" ::: "memory");  // colours in fours: fewer registers
+      if ((uint32_t)k < most && (uint32_t)k < n) col = over(col, decode_premult_lds(a.colour(k), s_dec, s_alpha));
+    }
+    const uint32_t t = (tile - dst.tile0) * kTileTargets + lane;
+    if (t < dst.T) dst.out[t] = over(over(col, tailc), dst.background);
+    if (lane == 0u) g.tb.cnt[tile] = 0u;
+    g.tb.more[(uint64_t)tile * kTileRuns + lane] = 0u;
+  }
+}
+
+template <int K, bool kTail>
+__global__ __launch_bounds__(64) void k_tile_batch_deep(TileBatchArgs args) {
+  if (rfl(ld_relaxed(&args.tb.ctl[args.tb.ctl_index + 1u])) == 0u) return;  // none flagged
+  const uint32_t n = rfl(ld_relaxed(&args.tb.ctl[args.tb.ctl_index]));
+  __shared__ float s_dec[256];
+  __shared__ float s_alpha[256];
+  __shared__ DeepLds<K> w;
+  for (uint32_t k = threadIdx.x; k < 256u; k += 64u) {
+    s_dec[k] = args.tab->dec[k];
+    s_alpha[k] = args.tab->alpha[k];
+  }
+  __syncthreads();
+  for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
+    const TileBatchArgs& g = fresh_batch_args();
+    const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
+    if (!(entry & kTileDeepFlag)) continue;
+    const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry & ~kTileDeepFlag;
+    const auto fr = (FramePtr)g.frames;
+    TileSrc src;
+    TileDst dst;
+    frame_views(fr, rfl(find_frame<true>(g.frames, g.f0, g.f1, (uint64_t)tile * kTileTargets)), g.tab, src, dst);
+    deep_wave<K, kTileList, kTail, false>(tile, 1u, 0u, g.tb, src, dst, w, s_dec, s_alpha);
+    wave_lds_sync();
+  }
+}
+
+// Waves that share a tile, 1 << split: few tiles get 2, 4 or 8 each, as long
+// as all are resident (a 145x103 frame of 130 thousand fragments, 234 tiles:
+// 80 us with a wave each, one tile after another's latency, 22 with eight).
+inline uint32_t tile_split(uint32_t tiles) {
+  uint32_t split = 0;
+  while (split < 3u && ((uint64_t)tiles << (split + 1u)) <= kSharedTiles) ++split;
+  return split;
+}
+
+template <int K>
+struct TileBatch {
+  template <bool kTail>
+  static hipError_t go(const BatchArgs& a, const TileBuf& tb, hipStream_t s) {
+    const uint32_t tiles = a.tiles * (kBlock / kTileTargets), split = tile_split(tiles);
+    const TileBatchArgs args{tb, a.frames, a.f0, a.f1, a.tile0 * (kBlock / kTileTargets), tiles, split, a.tab};
+    const uint32_t want = ((tiles << split) + kBlock / 64 - 1u) / (kBlock / 64);
+    const uint32_t fit = kComputeUnits * (uint32_t)tile_waves<K>();
+    hipLaunchKernelGGL((k_tile_batch<K, kTail>), dim3(want < fit ? want : fit), dim3(kBlock), 0, s, args);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = launch_tile_bin(a, tb, tiles, split, s);
+    if (e != hipSuccess) return e;
+    const uint32_t need = (tiles + kBlock / 64 - 1u) / (kBlock / 64);
+    const uint32_t most = kComputeUnits * (K >= 32 ? 4u : 8u);
+    const uint32_t blocks = need < most ? (need + kTicketLanes - 1u) / kTicketLanes * kTicketLanes : most;
+    hipLaunchKernelGGL((k_tile_binned<K, kTail>), dim3(blocks), dim3(kBlock), 0, s, args);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL((k_tile_batch_deep<K, kTail>), dim3(tiles < kComputeUnits ? tiles : kComputeUnits), dim3(64), 0, s,
+                       args);
+    return hipGetLastError();
+  }
+};
 
 template <int K>
 struct TileResolve {
@@ -1343,11 +1642,7 @@ struct TileResolve {
   static hipError_t go(const TileBuf& tb, const TileSrc& src, const TileDst& dst, hipStream_t s) {
     const uint32_t tiles = (dst.T + kTileTargets - 1u) / kTileTargets;
     const uint32_t fit = kComputeUnits * (uint32_t)tile_waves<K>();  // blocks resident at once
-    // few tiles: 2, 4 or 8 waves take a share each, as long as all are
-    // resident (a 145x103 frame of 130 thousand fragments, 234 tiles: 80 us
-    // with a wave each, one tile after another's latency)
-    uint32_t split = 0;
-    while (split < 3u && ((uint64_t)tiles << (split + 1u)) <= kSharedTiles) ++split;
+    const uint32_t split = tile_split(tiles);
     const uint32_t want = ((tiles << split) + kBlock / 64 - 1u) / (kBlock / 64);
     const dim3 g(want < fit ? want : fit), b(kBlock);
     // kGeneral: several segments, or the debug outputs

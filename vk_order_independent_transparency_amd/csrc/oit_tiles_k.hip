@@ -10,4 +10,9 @@ hipError_t tile_resolve_k<OIT_TILE_K>(const TileBuf& tb, const TileSrc& src, con
   return TileResolve<OIT_TILE_K>::run(tb, src, dst, mode, tail, s);
 }
 
+template <>
+hipError_t tile_batch_k<OIT_TILE_K>(const BatchArgs& a, const TileBuf& tb, bool tail, hipStream_t s) {
+  return tail ? TileBatch<OIT_TILE_K>::go<true>(a, tb, s) : TileBatch<OIT_TILE_K>::go<false>(a, tb, s);
+}
+
 }  // namespace oit
