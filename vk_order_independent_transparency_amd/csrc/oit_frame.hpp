@@ -409,6 +409,8 @@ __device__ __forceinline__ float4 dest_of(const Common& c, uint32_t t) {
   return c.opq_rgba ? c.opq_rgba[t] : c.background;
 }
 
+constexpr uint32_t kMaxCoverage = 8;  // samples of a coverage mask
+
 // Early depth test of a transparent fragment against the frame's opaque pass
 // (early_fragment_tests with post_depth_coverage, oitColorDepthDefines.glsl:
 // 24-37; VK_COMPARE_OP_LESS without depth write, main.cpp:526-528,541-543):
@@ -418,12 +420,30 @@ __device__ __forceinline__ uint32_t opaque_visible(const uint64_t* z, uint32_t T
                                                    uint32_t key, uint32_t m) {
   if (!z) return m;
   if (cov > 1u) {
+    // every plane's key in one round trip, whether the sample is covered or not
+    const uint32_t* const keys = reinterpret_cast<const uint32_t*>(z) + 1;
+    uint32_t k[kMaxCoverage];
+#pragma unroll
+    for (uint32_t s = 0; s < kMaxCoverage; ++s) k[s] = s < cov ? keys[2u * ((uint64_t)s * T + t)] : 0u;
     uint32_t r = 0u;
-    for (uint32_t s = 0; s < cov; ++s)
-      if (((m >> s) & 1u) && key < (uint32_t)(z[(uint64_t)s * T + t] >> 32)) r |= 1u << s;
-    return r;
+#pragma unroll
+    for (uint32_t s = 0; s < kMaxCoverage; ++s) r |= key < k[s] ? 1u << s : 0u;
+    return r & m;
   }
   return key < (uint32_t)(z[t] >> 32) ? m : 0u;
+}
+
+// The opaque depth key of each of a lane's kU targets (kEmpty without a target
+// or an opaque pass), loaded together: tested one after the other, each test
+// would wait for its own load.
+template <int kU>
+__device__ __forceinline__ void opaque_keys(const uint64_t* z, const uint32_t (&t)[kU], uint32_t (&k)[kU]) {
+#pragma unroll
+  for (int u = 0; u < kU; ++u) k[u] = kEmpty;
+  if (!z) return;
+#pragma unroll
+  for (int u = 0; u < kU; ++u)
+    if (t[u] != kEmpty) k[u] = reinterpret_cast<const uint32_t*>(z)[2u * (uint64_t)t[u] + 1u];
 }
 
 // Coverage shading: the ROP blends each tail fragment into the samples of

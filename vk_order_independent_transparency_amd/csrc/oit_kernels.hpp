@@ -162,7 +162,7 @@ constexpr uint32_t kTileTailWords = 64;   // tail fragments, counted by tile num
 constexpr uint32_t kTileBucket = kTileTails - 2u;  // ctl: entries of the bucket array given out (two words; batches)
 constexpr uint32_t kTileCtlWords = kTileTails + kTileTailWords;
 constexpr uint32_t kTileShares = kTileCtlWords;  // ctl: shares of a tile that have ended (frames of few tiles); 0 between frames
-constexpr uint32_t kSharedTiles = 4096;
+constexpr uint32_t kSharedTiles = 8192;
 constexpr uint32_t kTileCtlAll = kTileShares + kSharedTiles;
 constexpr uint32_t kTileTickets = kTileShares + kBatchMaxGroups * kSharedTiles;  // a batch's groups run side by side
 // ctl, batches: the next queue entries of a group's binning and of its binned

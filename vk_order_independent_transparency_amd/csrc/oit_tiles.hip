@@ -22,11 +22,14 @@ __device__ __forceinline__ void link_wave(const FragView& f, uint32_t T, uint32_
     dv[u] = (opq && in) ? ld_stream(&f.depth[i]) : 0.f;
   }
   bool lead[kU];
-  uint32_t len[kU], pos[kU];
+  uint32_t len[kU], pos[kU], behind[kU];
+#pragma unroll
+  for (int u = 0; u < kU; ++u)
+    if (t[u] >= T) t[u] = kEmpty;
+  opaque_keys<kU>(opq, t, behind);
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
-    if (t[u] >= T) t[u] = kEmpty;
-    if (opq && t[u] != kEmpty && !opaque_visible(opq, T, 1u, t[u], depth_key(dv[u]), 1u)) t[u] = kEmpty;
+    if (opq && depth_key(dv[u]) >= behind[u]) t[u] = kEmpty;
     const uint32_t tile = t[u] == kEmpty ? kEmpty : tile0 + (pm_index(t[u], T, spp) >> 6);
     const uint32_t before = __shfl_up(tile, 1u);
     const bool start = lane == 0u || before != tile;
@@ -159,8 +162,8 @@ __global__ __launch_bounds__(kBinThreads, 8) void k_tile_bin(BinArgs g) {
   BinWave& w = s_w[wave];
   const uint32_t turn = blockIdx.x % kTicketLanes;
   for (uint32_t q = blockIdx.x; q < n_tiles;) {
-    if (threadIdx.x == 0)
-      s_next = gridDim.x + turn + kTicketLanes * atomicAdd(&g.tb.ctl[g.tb.ticket0 + turn * 16u], 1u);
+    uint32_t ticket = 0;
+    if (threadIdx.x == 0) ticket = draw_ticket(g.tb, g.tb.ticket0 + turn * 16u);
     const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
     const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
     const uint32_t m = rfl(g.tb.cnt[tile]);
@@ -169,6 +172,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void k_tile_bin(BinArgs g) {
         g.tb.deep[g.tb.deep_base + q] = entry | kTileDeepFlag;
         atomicAdd(&g.tb.ctl[g.tb.ctl_index + 1u], 1u);
       }
+      if (threadIdx.x == 0) s_next = gridDim.x + turn + kTicketLanes * ticket;
       __syncthreads();
       q = rfl(s_next);
       __syncthreads();
@@ -190,6 +194,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void k_tile_bin(BinArgs g) {
       });
     }
     w.at[lane] = 0u;
+    if (threadIdx.x == 0) s_next = gridDim.x + turn + kTicketLanes * ticket;
     __syncthreads();
     if (m <= kBinThreads) {
       const uint64_t mine = threadIdx.x < m ? s_run[threadIdx.x] : 0ull;

@@ -286,11 +286,14 @@ __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const Co
   const uint32_t n_starts = (uint32_t)__builtin_popcount(lo_bits) + (uint32_t)__builtin_popcount(hi_bits);
   const uint32_t below = wave_scan_u32(n_starts) - n_starts;
   uint32_t used = 0;  // entries so far
-  for (uint32_t b = 0; b < nb; b += kU) {
-    uint32_t id[kU], loc[kU], key[kU], col[kU];
-    bool act[kU];
-    float4 cv[kU];
-    float dv[kU];
+  // the fields of kU batches; the next kU are loaded while these are listed
+  struct Fields {
+    uint32_t id, loc, key, col;
+    float4 cv;
+    float dv;
+    bool act;
+  };
+  auto load = [&](uint32_t b, Fields (&f)[kU]) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const uint32_t bb = b + (uint32_t)u;
@@ -299,27 +302,49 @@ __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const Co
           __builtin_amdgcn_readlane(hi_bits, bb & 63u),
           __builtin_amdgcn_mbcnt_lo(__builtin_amdgcn_readlane(lo_bits, bb & 63u),
                                     __builtin_amdgcn_readlane(below, bb & 63u)));
-      act[u] = pos < size;
+      f[u].act = pos < size;
       // lanes past the last fragment read the first one's fields: every lane
       // loads, so no load waits behind a branch
-      const uint32_t at = *(const LdsWord*)(deltas + 4u * k) + pos;
-      id[u] = act[u] ? at : id0;
+      const uint32_t at = *(const LdsWord*)(deltas + 4u * (f[u].act ? k : 0u)) + pos;
+      f[u].id = f[u].act ? at : id0;
     }
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       if constexpr (kStored) {
-        const uint64_t cd = ld_global_stream(&src.cd[id[u]]);
-        key[u] = (uint32_t)(cd >> 32);
-        col[u] = (uint32_t)cd;
-        loc[u] = ld_global_stream(&src.loc[id[u]]);
+        const uint64_t cd = ld_global_stream(&src.cd[f[u].id]);
+        f[u].key = (uint32_t)(cd >> 32);
+        f[u].col = (uint32_t)cd;
+        f[u].loc = ld_global_stream(&src.loc[f[u].id]);
       } else {
-        const TileSeg s = seg_of<kMany>(src, id[u]);
-        const uint32_t i = id[u] - s.id_base;
-        loc[u] = ld_global_stream(&s.target[i]);
-        dv[u] = ld_global_stream(&s.depth[i]);
-        cv[u] = ld_global_stream(&s.rgba[i]);
+        const TileSeg s = seg_of<kMany>(src, f[u].id);
+        const uint32_t i = f[u].id - s.id_base;
+        f[u].loc = ld_global_stream(&s.target[i]);
+        f[u].dv = ld_global_stream(&s.depth[i]);
+        f[u].cv = ld_global_stream(&s.rgba[i]);
       }
     }
+  };
+  Fields ahead[kU];
+  load(0u, ahead);
+  for (uint32_t b = 0; b < nb; b += kU) {
+    uint32_t id[kU], loc[kU], key[kU], col[kU];
+    bool act[kU];
+    float4 cv[kU];
+    float dv[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      id[u] = ahead[u].id;
+      loc[u] = ahead[u].loc;
+      act[u] = ahead[u].act;
+      if constexpr (kStored) {
+        key[u] = ahead[u].key;
+        col[u] = ahead[u].col;
+      } else {
+        dv[u] = ahead[u].dv;
+        cv[u] = ahead[u].cv;
+      }
+    }
+    if (b + kU < nb) load(b + kU, ahead);
     // onto the targets' lists, batch after batch
     uint32_t v[kU], old[kU];
 #pragma unroll
@@ -549,7 +574,19 @@ __device__ __forceinline__ bool tile_composite(TileLane& L, const TileSrc& src, 
     deferred = deferred || (tie && L.cnt > (uint32_t)(kMode == kTileLoop32 ? K : N));
     if (__ballot(deferred) != 0ull) return false;
     if constexpr (kMode == kTileLoop64 && N > 1) {
-      if (__ballot(tie) != 0ull) order_ties<N>(end, v);
+      if (__ballot(tie) != 0ull) {
+        // fragments of one colour too (the two sides of a sphere where they
+        // meet) stay in id order: nothing to do
+        bool mixed = false;
+        uint32_t before = entry_at(key_value<kMode>(v[0])).col;
+#pragma unroll
+        for (int k = 1; k < N; ++k) {
+          const uint32_t c = entry_at(key_value<kMode>(v[k])).col;
+          mixed = mixed || (key_depth(v[k]) == key_depth(v[k - 1]) && c != before && key_depth(v[k]) != kEmpty);
+          before = c;
+        }
+        if (__ballot(mixed) != 0ull) order_ties<N>(end, v);
+      }
     }
   }
   float4 col = zero;
@@ -604,14 +641,21 @@ __device__ __forceinline__ bool tile_composite(TileLane& L, const TileSrc& src, 
       } else if constexpr (kLast) {
         const bool deep = L.cnt > (uint32_t)K;
         const double kth = v[K - 1];
-        bool split = false;
+        const uint32_t kth_value = key_value<kMode>(kth), kth_col = entry_at(kth_value).col;
+        uint32_t equal = 0;  // Loop64: fragments of the K-th's depth
         uint32_t q = deep ? L.head : end;
         while (__ballot(q != end) != 0ull) {
           if (q != end) {
             const uint32_t key = entry_at(q).key;
-            const bool tail = kMode == kTileLoop32 ? key > key_depth(kth) : sort_key<kMode>(key, q) > kth;
+            bool tail = key > key_depth(kth);
+            if constexpr (kMode == kTileLoop64) {
+              if (key == key_depth(kth)) {
+                const uint32_t c = entry_at(q).col;
+                tail = c > kth_col || (c == kth_col && q > kth_value);
+                ++equal;
+              }
+            }
             if (tail) {
-              if constexpr (kMode == kTileLoop64) split = split || key == key_depth(kth);
               if constexpr (kMode == kTileLoop32) acc = over(acc, full_colour<kGeneral>(src, entry_id(q)));
               else acc = over(acc, decode_premult_lds(entry_at(q).col, s_dec, s_alpha));
               ++behind;
@@ -619,9 +663,12 @@ __device__ __forceinline__ bool tile_composite(TileLane& L, const TileSrc& src, 
             q = entry_at(q).next;
           }
         }
-        // Loop64: the order of the ties decides which of them are behind
+        // Loop64: where that depth goes on behind the N, its colours decide
         if constexpr (kMode == kTileLoop64) {
-          if (__ballot(split) != 0ull) return false;
+          uint32_t kept = 0;
+#pragma unroll
+          for (int k = 0; k < K; ++k) kept += key_depth(v[k]) == key_depth(kth) ? 1u : 0u;
+          if (__ballot(deep && key_depth(v[N - 1]) == key_depth(kth) && equal > kept) != 0ull) return false;
         }
       }
       d = over(acc, d);
@@ -1301,6 +1348,14 @@ constexpr int tile_entries(bool id) { return id ? 520 : 696; }
 template <int K>
 constexpr int tile_waves() { return K >= 32 ? 3 : 4; }
 
+// Draws a ticket (one lane). The address is hidden: for a wave-uniform one the
+// compiler combines the wave's lanes and waits for the result at once.
+__device__ __forceinline__ uint32_t draw_ticket(const TileBuf& tb, uint32_t counter) {
+  uint32_t at = counter;
+  asm volatile("" : "+v"(at));
+  return atomicAdd(&tb.ctl[at], 1u);
+}
+
 // The composites' arguments. They are read from the kernel arguments where
 // they are used: `fresh_args` hides the address from the compiler once per
 // tile, or it would keep all of them (some 90 scalar registers) in registers
@@ -1509,15 +1564,15 @@ __global__ __launch_bounds__(kBlock, K <= 8 ? 8 : (K <= 16 ? 6 : 4)) void k_tile
   const uint32_t lane = lane_id();
   const uint32_t turn = blockIdx.x % kTicketLanes;
   constexpr uint32_t kWaves = kBlock / 64;
-  uint32_t next = 0;
-  for (uint32_t q = (blockIdx.x / kTicketLanes * kWaves + rfl(threadIdx.x >> 6)) * kTicketLanes + turn; q < n_tiles;
-       q = rfl(next)) {
+  for (uint32_t q = (blockIdx.x / kTicketLanes * kWaves + rfl(threadIdx.x >> 6)) * kTicketLanes + turn; q < n_tiles;) {
     const TileBatchArgs& g = fresh_batch_args();
-    if (lane == 0u)
-      next = turn + gridDim.x * kWaves +
-             kTicketLanes * atomicAdd(&g.tb.ctl[g.tb.ticket0 + (kTicketLanes + turn) * 16u], 1u);
+    uint32_t ticket = 0;
+    if (lane == 0u) ticket = draw_ticket(g.tb, g.tb.ticket0 + (kTicketLanes + turn) * 16u);
     const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
-    if (entry & kTileDeepFlag) continue;  // the deep composite's
+    if (entry & kTileDeepFlag) {  // the deep composite's
+      q = turn + gridDim.x * kWaves + kTicketLanes * rfl(ticket);
+      continue;
+    }
     const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
     const auto fr = (FramePtr)g.frames;
     TileSrc src;
@@ -1575,6 +1630,7 @@ __global__ __launch_bounds__(kBlock, K <= 8 ? 8 : (K <= 16 ? 6 : 4)) void k_tile
     if (t < dst.T) dst.out[t] = over(over(col, tailc), dst.background);
     if (lane == 0u) g.tb.cnt[tile] = 0u;
     g.tb.more[(uint64_t)tile * kTileRuns + lane] = 0u;
+    q = turn + gridDim.x * kWaves + kTicketLanes * rfl(ticket);
   }
 }
 
@@ -1604,20 +1660,40 @@ __global__ __launch_bounds__(64) void k_tile_batch_deep(TileBatchArgs args) {
   }
 }
 
-// Waves that share a tile, 1 << split: few tiles get 2, 4 or 8 each, as long
-// as all are resident (a 145x103 frame of 130 thousand fragments, 234 tiles:
-// 80 us with a wave each, one tile after another's latency, 22 with eight).
-inline uint32_t tile_split(uint32_t tiles) {
-  uint32_t split = 0;
-  while (split < 3u && ((uint64_t)tiles << (split + 1u)) <= kSharedTiles) ++split;
-  return split;
+// Waves that share a tile, 1 << split, of `slots` resident waves: the least of
+// rounds x cost, where a wave pays for the fragments it reads (all of the
+// tile's, once for every part that fits its LDS, and about 200 fragments'
+// time besides) and for those it lists and sorts (its share). Few tiles get
+// up to eight waves each (a 145x103 frame of 130 thousand fragments, 234
+// tiles: 80 us with a wave each, one tile after another's latency, 22 with
+// eight); and so do tiles a little more numerous than the waves, or larger
+// than one part (808x402, 3.5 M fragments, 5076 tiles: 136 us with a wave
+// each, in two rounds of two parts, 73 with two).
+inline uint32_t tile_split(uint32_t tiles, uint32_t slots, uint64_t frags, uint32_t cap) {
+  if (tiles > kSharedTiles || tiles > 2u * slots) return 0;
+  const uint64_t n = tiles ? frags / tiles : 0u;
+  uint32_t best = 0;
+  uint64_t least = ~0ull;
+  for (uint32_t split = 0; split <= 3u; ++split) {
+    const uint64_t rounds = (((uint64_t)tiles << split) + slots - 1u) / slots;
+    const uint64_t parts = ((n + n / 4u) >> split) / cap + 1u;  // a quarter more: tiles differ
+    const uint64_t cost = rounds * (parts * (n + 200u) + (n >> split));
+    if (cost < least) {
+      least = cost;
+      best = split;
+    }
+  }
+  return best;
 }
+constexpr uint32_t kListedFragments = 300;  // a tile of a batch group, whose fragments are not counted apart
 
 template <int K>
 struct TileBatch {
   template <bool kTail>
   static hipError_t go(const BatchArgs& a, const TileBuf& tb, hipStream_t s) {
-    const uint32_t tiles = a.tiles * (kBlock / kTileTargets), split = tile_split(tiles);
+    const uint32_t tiles = a.tiles * (kBlock / kTileTargets);
+    const uint32_t split = tile_split(tiles, kComputeUnits * (uint32_t)tile_waves<K>() * (kBlock / 64),
+                                      (uint64_t)tiles * kListedFragments, tile_entries(false));
     const TileBatchArgs args{tb, a.frames, a.f0, a.f1, a.tile0 * (kBlock / kTileTargets), tiles, split, a.tab};
     const uint32_t want = ((tiles << split) + kBlock / 64 - 1u) / (kBlock / 64);
     const uint32_t fit = kComputeUnits * (uint32_t)tile_waves<K>();
@@ -1642,9 +1718,13 @@ struct TileResolve {
   static hipError_t go(const TileBuf& tb, const TileSrc& src, const TileDst& dst, hipStream_t s) {
     const uint32_t tiles = (dst.T + kTileTargets - 1u) / kTileTargets;
     const uint32_t fit = kComputeUnits * (uint32_t)tile_waves<K>();  // blocks resident at once
-    const uint32_t split = tile_split(tiles);
+    const uint32_t split = tile_split(tiles, fit * (kBlock / 64), src.frags, tile_entries(kMode == kTileLoop32));
     const uint32_t want = ((tiles << split) + kBlock / 64 - 1u) / (kBlock / 64);
-    const dim3 g(want < fit ? want : fit), b(kBlock);
+    // three rounds of resident blocks: tiles differ in depth, and the blocks
+    // of the later rounds go where the earlier ones have ended (1600x900 Loop32
+    // K = 16: 247 us with one round, 204 with three; 1920x1080 Loop64: 155, 159)
+    const uint32_t most = 3u * fit;
+    const dim3 g(want < most ? want : most), b(kBlock);
     // kGeneral: several segments, or the debug outputs
     const bool dbg = dst.fk_key || dst.fk_val || dst.counts || (!kStored && src.nseg > 1u);
     const TileArgs args{tb, src, dst, tiles, split};
