@@ -1143,6 +1143,7 @@ int oit_resolve_debug(oit_ctx* c, float* out_rgba, uint32_t* fk_key, uint32_t* f
       src.T = c->T;
       src.spp = k.spp;
       src.frags = c->frame_frags;
+      src.opq = k.opq_z;
       std::vector<oit::TileSeg> segs;
       for (const auto& v : c->segments) segs.push_back({v.target, v.depth, v.rgba, v.id_base, 0u});
       if (!segs.empty()) src.one = segs[0];

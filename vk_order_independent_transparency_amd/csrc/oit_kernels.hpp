@@ -207,6 +207,7 @@ struct TileSrc {
   uint32_t nseg = 1;
   uint32_t T = 0, spp = 1;        // targets and samples per pixel of the frame
   uint64_t frags = 0;             // fragments of the frame
+  const uint64_t* opq = nullptr;  // opaque depth planes, or null
   const uint64_t* cd = nullptr;   // stored payloads (depth key << 32 | packed colour) by id, and list index mod 64
   const uint8_t* loc = nullptr;
 };

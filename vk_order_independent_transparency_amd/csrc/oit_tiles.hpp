@@ -268,11 +268,16 @@ __device__ __forceinline__ void mark_run(Lds& w, bool on, uint32_t off) {
 // Returns false (wave-uniform) where the fragments are more than `cap`.
 template <bool kStored, bool kMany, typename Lds>
 __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const CodecTables* tab, uint32_t deltas,
-                                            uint32_t id0, uint32_t size, uint32_t shift, uint32_t part, uint32_t cap) {
+                                            uint32_t id0, uint32_t size, uint32_t shift, uint32_t part, uint32_t cap,
+                                            uint32_t target, bool in) {
   constexpr int kU = 3;  // 64-fragment batches in flight together
   const uint32_t lane = lane_id();
   const uint32_t nb = (size + 63u) >> 6;
   const uint32_t end = lds_address(&w.e[0]);
+  // the lane's target's opaque depth: fragments behind it are not listed
+  const bool opaque = src.opq != nullptr;
+  uint32_t front = kEmpty;
+  if (opaque && in) front = *((const __attribute__((address_space(1))) uint32_t*)src.opq + 2u * (uint64_t)target + 1u);
   w.head[lane] = end;
   w.count[lane] = 0u;
   if (lane == 0u) {
@@ -361,6 +366,10 @@ __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const Co
         col[u] = encode_color_quick(cv[u], tab);
       }
       act[u] = act[u] && (loc[u] >> shift) == part;
+      if (opaque) {
+        const uint32_t z = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(loc[u] << 2), (int)front);
+        act[u] = act[u] && key[u] < z;
+      }
       const uint64_t on = __ballot(act[u]);
       v[u] = end + (used + lanes_below(on) + 1u) * Lds::kSize;
       used += (uint32_t)__builtin_popcountll(on);
@@ -975,7 +984,7 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
   }
   for (uint32_t t0 = first; t0 < last;) {
     const uint32_t part = t0 >> shift;
-    if (!build_lists<kStored, kGeneral>(w, src, dst.tab, deltas, id0, size, shift, part, cap)) {
+    if (!build_lists<kStored, kGeneral>(w, src, dst.tab, deltas, id0, size, shift, part, cap, L.t, in)) {
       wave_lds_sync();
       if (shift == 0u || kMode == kTileList) {  // one target's fragments
         end_share(tb, tile, m, first, split, true, queue);
@@ -1033,6 +1042,9 @@ struct DeepLds {
 template <bool kStored, typename Lds, typename F>
 __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const TileSrc& src, const TileDst& dst,
                                                uint32_t tile, uint32_t m, bool keep, F&& body) {
+  const uint32_t list_index = (tile - dst.tile0) * kTileTargets + lane_id();
+  const bool in = list_index < dst.T;
+  const uint32_t t = in ? pm_target(list_index, dst.T, dst.spp) : 0u;
   const uint32_t lane = lane_id();
   if (keep) {
     body(true);
@@ -1089,7 +1101,7 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
       mark_run(w.g, lane < r, incl - len);
       w.g.delta[lane] = start - (incl - len);
       wave_lds_sync();
-      (void)build_lists<kStored, true>(w.g, src, dst.tab, lds_address(w.g.delta), rfl(start), N, 6u, 0u, kDeepEntries);
+      (void)build_lists<kStored, true>(w.g, src, dst.tab, lds_address(w.g.delta), rfl(start), N, 6u, 0u, kDeepEntries, t, in);
       body(first == 0u && lo == 0u);
       ++groups;
       wave_lds_sync();
