@@ -1008,6 +1008,7 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
     else if (L.most <= 8u || R <= 8) done = OIT_TILE_SIZE(8);
     else if (L.most <= 12u || R <= 12) done = OIT_TILE_SIZE(12);
     else if (L.most <= 16u || R <= 16) done = OIT_TILE_SIZE(16);
+    else if (kMode == kTileLoop64 && R > 20 && L.most <= 20u) done = OIT_TILE_SIZE(20);  // (24 spill)
     else if (L.most <= 24u || R <= 24) done = OIT_TILE_SIZE(24);
     else done = OIT_TILE_SIZE(32);
 #undef OIT_TILE_SIZE
