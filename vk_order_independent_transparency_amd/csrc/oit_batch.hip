@@ -17,10 +17,11 @@
 // By default nothing is linked per target: the frames go through the tile
 // path (oit_tiles.hpp), whose composite reads the callers' fragments itself,
 // since they stay valid until the run has ended. The 24-frame mix (205 M
-// fragments, 155 to 2810 spheres a frame, a fifth clustered) takes 2.9 ms so
-// and 6.9 ms with lists, whose ordered inserts walk past each other on the
+// fragments, 155 to 2810 spheres a frame, a fifth clustered) takes 3.6 ms so
+// and 6.6 ms with lists, whose ordered inserts walk past each other on the
 // clustered pixels. A tuning that asks for anything but the defaults gets the
-// list or bucket kernels it names.
+// list or bucket kernels it names; so does a batch without memory for the
+// tiles (20 bytes a fragment, the lists 12).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

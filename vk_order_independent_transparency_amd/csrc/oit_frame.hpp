@@ -244,14 +244,13 @@ constexpr uint32_t kTailWalks = 4;
 
 // One walk of an unordered tail list: the kTailWindow largest values below
 // `bound`, in descending order (0 = none), by an insertion network in
-// registers; returns how many values of the list lie below `bound`, and in
-// `flagged` the number of boundary-flagged values of the whole list. A walk
+// registers; returns how many values of the list lie below `bound`. A walk
 // longer than the arrays hold (a cycle) reports kErrWalk and sets `bad`.
 __device__ __forceinline__ uint32_t tail_window(const TailBuf& tb, uint32_t head, uint32_t vcap, uint32_t bound,
-                                                uint32_t (&w)[kTailWindow], uint32_t& flagged, bool& bad) {
+                                                uint32_t (&w)[kTailWindow], bool& bad) {
 #pragma unroll
   for (int k = 0; k < kTailWindow; ++k) w[k] = 0u;
-  uint32_t n = 0, fl = 0, hops = 0;
+  uint32_t n = 0, hops = 0;
   uint32_t v = head;
   while (v != 0u && v < vcap) {  // a link outside the arrays ends the walk
     if (++hops > tb.cap) {
@@ -260,7 +259,6 @@ __device__ __forceinline__ uint32_t tail_window(const TailBuf& tb, uint32_t head
       break;
     }
     const uint32_t nx = tb.next[tail_index(v)];
-    fl += v & 1u;
     if (v < bound) {
       ++n;
       uint32_t x = v;
@@ -273,7 +271,6 @@ __device__ __forceinline__ uint32_t tail_window(const TailBuf& tb, uint32_t head
     }
     v = nx;
   }
-  flagged = fl;
   return n;
 }
 
@@ -327,31 +324,23 @@ __device__ __forceinline__ uint32_t tail_sort_desc(const TailBuf& tb, uint32_t h
 // background. The list is unordered, so each walk takes the next
 // kTailWindow values in descending order (one walk for most targets, up to
 // kTailWalks) and loads their colours four at a time; a longer tail is
-// sorted in place and folded in one walk. `skip` boundary-flagged entries are in the A-buffer and not blended
-// (Loop64 identical keys, see k_loop64_classify): the flagged ones with the
-// lowest ids (no caller has any since Loop64 finds its tail in the tile path).
+// sorted in place and folded in one walk.
 // tail_fold with the list's head value already loaded (a composite issues
 // that load with its own first loads instead of after them).
-__device__ __forceinline__ float4 tail_fold_from(const TailBuf& tb, uint32_t head, float4 bg, uint32_t skip) {
+__device__ __forceinline__ float4 tail_fold_from(const TailBuf& tb, uint32_t head, float4 bg) {
   const uint32_t vcap = tail_value_cap(tb.cap);
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   if (head == 0u || head >= vcap) return over(acc, bg);
-  uint32_t keep = 0xFFFFFFFFu;  // flagged entries to blend
   uint32_t bound = 0xFFFFFFFFu;
   bool bad = false;
   for (bool first = true;; first = false) {
     uint32_t w[kTailWindow];
-    uint32_t flagged;
-    const uint32_t n = tail_window(tb, head, vcap, bound, w, flagged, bad);
-    if (first && skip > 0u) keep = flagged > skip ? flagged - skip : 0u;
+    const uint32_t n = tail_window(tb, head, vcap, bound, w, bad);
     if (first && !bad && n > (uint32_t)kTailWindow * kTailWalks) {  // a long tail: sorted, then one walk
       for (uint32_t v = tail_sort_desc(tb, head, vcap); v != 0u && v < vcap;) {
         const uint32_t id = tail_index(v);
         const uint32_t nx = tb.next[id];
-        if (!(v & 1u) || keep > 0u) {
-          acc = over(acc, tb.rgba[id]);
-          if (v & 1u) --keep;
-        }
+        acc = over(acc, tb.rgba[id]);
         v = nx;
       }
       break;
@@ -365,10 +354,7 @@ __device__ __forceinline__ float4 tail_fold_from(const TailBuf& tb, uint32_t hea
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t v = w[g + j];
-        if (v != 0u && (!(v & 1u) || keep > 0u)) {
-          acc = over(acc, c[j]);
-          if (v & 1u) --keep;
-        }
+        if (v != 0u) acc = over(acc, c[j]);
       }
     }
     if (bad || n <= (uint32_t)kTailWindow) break;
@@ -377,8 +363,8 @@ __device__ __forceinline__ float4 tail_fold_from(const TailBuf& tb, uint32_t hea
   return over(acc, bg);
 }
 
-__device__ __forceinline__ float4 tail_fold(const TailBuf& tb, uint32_t t, float4 bg, uint32_t skip) {
-  return tail_fold_from(tb, tb.head[t], bg, skip);
+__device__ __forceinline__ float4 tail_fold(const TailBuf& tb, uint32_t t, float4 bg) {
+  return tail_fold_from(tb, tb.head[t], bg);
 }
 
 // Sample shading with spp samples per pixel lays targets out sample-major
@@ -464,8 +450,7 @@ __device__ __forceinline__ float4 tail_fold_cov(const TailBuf& tb, uint32_t t, c
   bool bad = false;
   while (!empty) {  // windows of the unordered list, newest first (tail_fold_from)
     uint32_t w[kTailWindow];
-    uint32_t flagged;
-    const uint32_t n = tail_window(tb, head, vcap, bound, w, flagged, bad);
+    const uint32_t n = tail_window(tb, head, vcap, bound, w, bad);
     if (bound == 0xFFFFFFFFu && !bad && n > (uint32_t)kTailWindow * kTailWalks) {  // a long tail: sorted, one walk
       for (uint32_t v = tail_sort_desc(tb, head, vcap); v != 0u && v < vcap;) {
         const uint32_t id = tail_index(v);

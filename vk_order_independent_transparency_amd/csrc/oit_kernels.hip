@@ -403,7 +403,7 @@ __global__ __launch_bounds__(kBlock, (K == 16 && !kColorTail) ? 6 : 1) void k_ll
     uint32_t cnt;
     const float4 col = ll_walk_reset<K, kTail, kPair>(i, ll, s_dec, s_alpha, a, cnt);
     float4 d = dest_of(c, t);
-    if (kColorTail) d = tail_fold(tb, t, d, 0u);
+    if (kColorTail) d = tail_fold(tb, t, d);
     o.out[t] = over(col, d);
     if (kDebug) write_debug<K>(o, t, a, cnt < (uint32_t)K ? cnt : (uint32_t)K, cnt, true, false);
   }
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(kBlock) void k_ll_resolve_reset_keys(Common c, LLBu
     uint32_t cnt;
     const float4 col = ll_walk_reset_keys<K, kTail, kPair>(i, ll, s_dec, s_alpha, a, cnt);
     float4 d = dest_of(c, t);
-    if (kColorTail) d = tail_fold(tb, t, d, 0u);
+    if (kColorTail) d = tail_fold(tb, t, d);
     o.out[t] = over(col, d);
     if (kDebug) {
       const uint32_t n = cnt < (uint32_t)K ? cnt : (uint32_t)K;
@@ -1319,7 +1319,7 @@ __global__ __launch_bounds__(kBlock) void k_kbuf_resolve(Common c, KBuf kb, Tail
   for (int k = 0; k < K; ++k)
     if ((uint32_t)k < nmax && (uint32_t)k < n) col = over(col, decode_premult_lds(a.col[k], s_dec, s_alpha));
   float4 d = dest_of(c, t);
-  if (kColorTail) d = tail_fold_from(tb, th, d, 0u);
+  if (kColorTail) d = tail_fold_from(tb, th, d);
   o.out[t] = over(col, d);
   if (kDebug) write_debug<K>(o, t, a, n, count, false, false);
 }

@@ -93,7 +93,14 @@ __global__ __launch_bounds__(kBlock) void k_tile_link_batch(BatchArgs b, TileBuf
 // each in id order, by a counting sort. A block's waves take a share of the
 // tile's sorted runs each, count per target, and place their fragments behind
 // the earlier shares'; a fragment's place among its batch's is its rank among
-// the lanes of its target. Leaves each target's number and place in `run` and
+// the lanes of its target. Against a wave per tile that reads the tile once
+// for every 696 fragments' worth of targets, the 24-frame mix (205 M
+// fragments, about 120 M of them in such tiles) went from 10.3 to 5.4 ms, with
+// rows of 16 targets (below) and one queue atomic for 64 tiles to 4.3, with
+// tickets to 3.9: blocks that stepped through the queue were at work half of
+// the time, some tiles holding 36 thousand fragments. Bound by its scattered
+// 8-byte stores and about 230 vector instructions per 64 fragments.
+// Leaves each target's number and place in `run` and
 // the tile's base in the first two words of `more`.
 constexpr uint32_t kBinThreads = 256;
 constexpr uint32_t kBinWaves = kBinThreads / 64u;
