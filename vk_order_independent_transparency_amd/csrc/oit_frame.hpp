@@ -407,6 +407,7 @@ __device__ __forceinline__ uint32_t opaque_visible(const uint64_t* z, uint32_t T
   if (!z) return m;
   if (cov > 1u) {
     // every plane's key in one round trip, whether the sample is covered or not
+    // (1920x1080, 4 samples: frame 446 -> 436 us against a test after each load)
     const uint32_t* const keys = reinterpret_cast<const uint32_t*>(z) + 1;
     uint32_t k[kMaxCoverage];
 #pragma unroll
@@ -417,19 +418,6 @@ __device__ __forceinline__ uint32_t opaque_visible(const uint64_t* z, uint32_t T
     return r & m;
   }
   return key < (uint32_t)(z[t] >> 32) ? m : 0u;
-}
-
-// The opaque depth key of each of a lane's kU targets (kEmpty without a target
-// or an opaque pass), loaded together: tested one after the other, each test
-// would wait for its own load.
-template <int kU>
-__device__ __forceinline__ void opaque_keys(const uint64_t* z, const uint32_t (&t)[kU], uint32_t (&k)[kU]) {
-#pragma unroll
-  for (int u = 0; u < kU; ++u) k[u] = kEmpty;
-  if (!z) return;
-#pragma unroll
-  for (int u = 0; u < kU; ++u)
-    if (t[u] != kEmpty) k[u] = reinterpret_cast<const uint32_t*>(z)[2u * (uint64_t)t[u] + 1u];
 }
 
 // Coverage shading: the ROP blends each tail fragment into the samples of

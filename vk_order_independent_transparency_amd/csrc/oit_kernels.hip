@@ -163,21 +163,16 @@ __device__ __forceinline__ void ll_append_wave(const AppendSrc& f, const float* 
     col[u] = in ? ld_stream(&f.rgba[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
     m[u] = (in && f.mask) ? ld_stream(&f.mask[i]) : 0xFFFFFFFFu;
   }
-  uint32_t behind[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u)
-    if (t[u] >= f.T) t[u] = kEmpty;
-  opaque_keys<kU>(f.cov > 1u ? nullptr : f.opq, t, behind);
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
     const uint64_t i = f.first + (uint64_t)u * 64u + lane;
+    if (t[u] >= f.T) t[u] = kEmpty;
     if (f.mask && t[u] != kEmpty) {
       m[u] &= f.full;
       if (m[u] == 0u) t[u] = kEmpty;  // no sample covered: the shader does not run
     }
     if (f.opq && t[u] != kEmpty) {  // behind the opaque depth in every covered sample: culled
-      if (f.cov > 1u) m[u] = opaque_visible(f.opq, f.T, f.cov, t[u], depth_key(dep[u]), m[u]);
-      else if (depth_key(dep[u]) >= behind[u]) m[u] = 0u;
+      m[u] = opaque_visible(f.opq, f.T, f.cov, t[u], depth_key(dep[u]), m[u]);
       if (m[u] == 0u) t[u] = kEmpty;
     }
     const uint64_t n64 = (uint64_t)f.node0 + i;
