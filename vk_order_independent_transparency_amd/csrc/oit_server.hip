@@ -66,11 +66,12 @@ uint64_t request_bytes(const oit_request& r, uint64_t F) {
   const uint64_t K = r.algorithm == OIT_WEIGHTED ? 1 : r.layers;
   const bool tail = r.tail_blend != 0;
   const uint64_t tails = tail ? 4 * T + 28 * F + 4 * ((F + 1023) / 1024) : 0;
+  const uint64_t tiles = 13 * T + 8 * F;  // run structures per 64 targets, links per fragment
   switch (r.algorithm) {
     case OIT_LINKEDLIST: return 4 * T + 12 * (F + 1) + (tail ? 4 * T : 0);
     case OIT_INTERLOCK: return 4 * T + 28 * (F + 1);
-    case OIT_LOOP: return 12 * K * T + tails;
-    case OIT_LOOP64: return 8 * K * T + 4 * T + 8 * ((F + 63) / 64) + tails;  // more than its tiles' 12.2 T + 8 F
+    case OIT_LOOP: return std::max(12 * K * T + tails, tiles);
+    case OIT_LOOP64: return std::max(8 * K * T + 4 * T + 8 * ((F + 63) / 64) + tails, tiles);
     case OIT_SIMPLE: return 4 * T + 12 * K * T + tails;
     case OIT_SPINLOCK: return 12 * T + 12 * K * T + tails;
     default: return 20 * T;
@@ -348,7 +349,7 @@ int launch(oit_server* s, Slot& sl) {
   if ((rc = oit_clear(pc.ctx, sl.stream))) return rc;
   if ((rc = oit_append(pc.ctx, &f, sl.stream))) return rc;
   if ((rc = oit_resolve(pc.ctx, out, sl.stream))) return rc;
-  if (oit_query_sizes(pc.ctx, &z) == OIT_OK) {  // the resolve may size per-frame buffers (Loop64's and Loop32's run links)
+  if (oit_query_sizes(pc.ctx, &z) == OIT_OK) {  // the resolve may size per-frame buffers (the tiles' run links)
     std::lock_guard<std::mutex> g(s->gmu);
     pc.resident = z.resident_bytes;
     publish_held(s);
