@@ -104,7 +104,6 @@ __global__ __launch_bounds__(kBlock) void k_tile_link_batch(BatchArgs b, TileBuf
 // the tile's base in the first two words of `more`.
 constexpr uint32_t kBinThreads = 256;
 constexpr uint32_t kBinWaves = kBinThreads / 64u;
-constexpr uint32_t kBinRuns = 1024;
 
 struct BinWave {
   uint32_t bits[128];
@@ -172,12 +171,15 @@ __global__ __launch_bounds__(kBinThreads, 8) void k_tile_bin(BinArgs g) {
     const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
     const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
     const uint32_t m = rfl(g.tb.cnt[tile]);
-    if (m > kBinRuns) {  // (the same in every thread)
+    // Left to the deep composite, which like this kernel and the binned
+    // composite tells such a tile by its run count: the entry is read by every
+    // wave of the block and by later kernels, so nothing is written to it. (The
+    // count is the same in every thread: cleared by the composites alone.)
+    if (m > kBinRuns) {
       if (threadIdx.x == 0) {
-        g.tb.deep[g.tb.deep_base + q] = entry | kTileDeepFlag;
         atomicAdd(&g.tb.ctl[g.tb.ctl_index + 1u], 1u);
+        s_next = gridDim.x + turn + kTicketLanes * ticket;
       }
-      if (threadIdx.x == 0) s_next = gridDim.x + turn + kTicketLanes * ticket;
       __syncthreads();
       q = rfl(s_next);
       __syncthreads();

@@ -1447,7 +1447,7 @@ __global__ __launch_bounds__(64) void k_tile_deep(TileArgs args) {
   }
 }
 
-constexpr uint32_t kTileDeepFlag = 1u << 31;  // queue entry of a batch: left to the deep composite
+constexpr uint32_t kBinRuns = 1024;  // a batch's queued tiles of more runs are left to the deep composite
 
 // A batch group's frames: the same composite, each tile with its frame's
 // arrays and size.
@@ -1593,11 +1593,11 @@ __global__ __launch_bounds__(kBlock, K <= 8 ? 8 : (K <= 16 ? 6 : 4)) void k_tile
     uint32_t ticket = 0;
     if (lane == 0u) ticket = draw_ticket(g.tb, g.tb.ticket0 + (kTicketLanes + turn) * 16u);
     const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
-    if (entry & kTileDeepFlag) {  // the deep composite's
+    const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
+    if (rfl(g.tb.cnt[tile]) > kBinRuns) {  // the deep composite's
       q = turn + gridDim.x * kWaves + kTicketLanes * rfl(ticket);
       continue;
     }
-    const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
     const auto fr = (FramePtr)g.frames;
     TileSrc src;
     TileDst dst;
@@ -1660,7 +1660,7 @@ __global__ __launch_bounds__(kBlock, K <= 8 ? 8 : (K <= 16 ? 6 : 4)) void k_tile
 
 template <int K, bool kTail>
 __global__ __launch_bounds__(64) void k_tile_batch_deep(TileBatchArgs args) {
-  if (rfl(ld_relaxed(&args.tb.ctl[args.tb.ctl_index + 1u])) == 0u) return;  // none flagged
+  if (rfl(ld_relaxed(&args.tb.ctl[args.tb.ctl_index + 1u])) == 0u) return;  // none left over
   const uint32_t n = rfl(ld_relaxed(&args.tb.ctl[args.tb.ctl_index]));
   __shared__ float s_dec[256];
   __shared__ float s_alpha[256];
@@ -1673,8 +1673,8 @@ __global__ __launch_bounds__(64) void k_tile_batch_deep(TileBatchArgs args) {
   for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
     const TileBatchArgs& g = fresh_batch_args();
     const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
-    if (!(entry & kTileDeepFlag)) continue;
-    const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry & ~kTileDeepFlag;
+    const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
+    if (rfl(g.tb.cnt[tile]) <= kBinRuns) continue;  // composited: its count is 0
     const auto fr = (FramePtr)g.frames;
     TileSrc src;
     TileDst dst;
