@@ -84,7 +84,8 @@ typedef struct oit_config {
   uint64_t ll_pool_nodes;      /* Linked List capacity in nodes INCLUDING terminator node 0
                                   (SceneData.linkedListAllocatedPerElement for OIT_LINKEDLIST,
                                   oit.cpp:125); 0 = ll_nodes_per_pixel * width * height * samples */
-  uint64_t max_fragments;      /* per-frame fragment capacity of the tail lists; 0 = grow on demand */
+  uint64_t max_fragments;      /* per-frame fragment capacity of the tail lists; 0 = grow on demand. Loop32 and
+                                  Loop64 reserve their links for it with or without tail blending */
   float    background[4];      /* premultiplied RGBA the colour pass starts from (opaque gray 0.5 by default) */
   float    wboit_view_near;    /* WBOIT: view distance = near + depth * span ... */
   float    wboit_view_span;    /* ... stands in for -viewZ (object.vert.glsl:35) */

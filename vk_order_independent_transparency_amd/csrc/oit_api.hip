@@ -385,8 +385,9 @@ oit::TileBuf tiles_of(const oit_ctx* c) {
 
 // Makes the tile path's links hold `need` fragments, keeping this frame's
 // (a stream-ordered copy; the old buffer is freed once the stream has
-// drained). With tail blending, max_fragments bounds a frame as it does for
-// the algorithms that keep tail lists.
+// drained); nothing is allocated where oit_configure reserved enough. With
+// tail blending, max_fragments bounds a frame as it does for the algorithms
+// that keep tail lists.
 int ensure_tile_link(oit_ctx* c, uint64_t need, hipStream_t s) {
   if (need <= c->cap_tile_link) return OIT_OK;
   uint64_t cap = c->cap_tile_link ? c->cap_tile_link : 1024;
@@ -725,9 +726,20 @@ int oit_configure(oit_ctx* c, const oit_config* cfg) {
         if (!rc) rc = reserve(c, &c->tile_deep, &c->cap_tiles, tiles);
       }
       if (!rc) rc = reserve(c, &c->tile_ctl, &c->cap_tile_ctl, oit::kTileCtlAll);
-      if (!rc && cfg->tail_blend && cfg->max_fragments)
-        rc = reserve(c, &c->tile_link, &c->cap_tile_link,
-                     cfg->max_fragments < kMaxFrameFragments ? cfg->max_fragments : kMaxFrameFragments);
+      if (!rc) rc = reserve(c, &c->tile_segs, &c->cap_tile_segs, oit::kSegArgs);
+      // links for a frame of max_fragments, so that its appends allocate
+      // nothing. Only with tail blending does max_fragments bound a frame;
+      // without it the links are grown by the appends where these are not
+      // enough, or could not be had. A Loop32 frame without either gets what
+      // its slot planes would have taken (12 bytes a slot), so that it too
+      // can be captured at once.
+      uint64_t links = cfg->max_fragments;
+      if (!links && !cfg->tail_blend && alg == OIT_LOOP) links = T * K * 12u / sizeof(uint64_t);
+      if (links > kMaxFrameFragments) links = kMaxFrameFragments;
+      if (!rc) {
+        rc = reserve(c, &c->tile_link, &c->cap_tile_link, links);
+        if (rc == OIT_ERR_OOM && !cfg->tail_blend) rc = OIT_OK;
+      }
       c->bytes_abuf = tiles * oit::kTileRuns * 12u;
       c->bytes_aux = tiles * 8u;
       break;

@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "oit.h"
+#include "oit_kernels.hpp"
 #include "oit_scene_gen.hpp"
 
 struct PoolCtx;
@@ -66,7 +67,10 @@ uint64_t request_bytes(const oit_request& r, uint64_t F) {
   const uint64_t K = r.algorithm == OIT_WEIGHTED ? 1 : r.layers;
   const bool tail = r.tail_blend != 0;
   const uint64_t tails = tail ? 4 * T + 28 * F + 4 * ((F + 1023) / 1024) : 0;
-  const uint64_t tiles = 13 * T + 8 * F;  // run structures per 64 targets, links per fragment
+  // Loop32, Loop64: run structures per tile of 64 targets, links per
+  // fragment, counters and a segment table
+  const uint64_t tiles = oit::tile_count(T) * (8 + oit::kTileRuns * 12) + 8 * std::max<uint64_t>(F, 1) +
+                         oit::kTileCtlAll * 4 + oit::kSegArgs * sizeof(oit::TileSeg);
   switch (r.algorithm) {
     case OIT_LINKEDLIST: return 4 * T + 12 * (F + 1) + (tail ? 4 * T : 0);
     case OIT_INTERLOCK: return 4 * T + 28 * (F + 1);
@@ -330,7 +334,10 @@ int launch(oit_server* s, Slot& sl) {
   c.height = r.scene.height;
   c.samples = r.scene.samples;
   c.ll_pool_nodes = (alg == OIT_LINKEDLIST || alg == OIT_INTERLOCK) ? F + 1 : 0;
-  c.max_fragments = (r.tail_blend && alg != OIT_LINKEDLIST && alg != OIT_WEIGHTED) ? (F ? F : 1) : 0;
+  // the tail lists' size, and for Loop32 and Loop64 that of their links, with a tail or without
+  const bool sized_by_fragments = alg == OIT_LOOP || alg == OIT_LOOP64 ||
+                                  (r.tail_blend && alg != OIT_LINKEDLIST && alg != OIT_WEIGHTED);
+  c.max_fragments = sized_by_fragments ? (F ? F : 1) : 0;
   c.background[0] = c.background[1] = c.background[2] = 0.5f;
   c.background[3] = 1.0f;
   c.wboit_view_near = 2.0f;
@@ -349,7 +356,7 @@ int launch(oit_server* s, Slot& sl) {
   if ((rc = oit_clear(pc.ctx, sl.stream))) return rc;
   if ((rc = oit_append(pc.ctx, &f, sl.stream))) return rc;
   if ((rc = oit_resolve(pc.ctx, out, sl.stream))) return rc;
-  if (oit_query_sizes(pc.ctx, &z) == OIT_OK) {  // the resolve may size per-frame buffers (the tiles' run links)
+  if (oit_query_sizes(pc.ctx, &z) == OIT_OK) {  // the append may size per-frame buffers (the interlock's pool)
     std::lock_guard<std::mutex> g(s->gmu);
     pc.resident = z.resident_bytes;
     publish_held(s);
