@@ -56,6 +56,8 @@ enum oit_algorithm {
                                              (always at 32 layers) */
 #define OIT_VARIANT_STORE_CHUNKS_1   0x10u /* accepted, no effect (Loop64 has one schedule) */
 #define OIT_VARIANT_STORE_CHUNKS_4   0x20u /* likewise */
+#define OIT_VARIANT_BATCH_LISTS      0x40u /* oit_batch_tuning only: a list per target even where every other choice is
+                                             the default (a batch composites tiles of 64 targets by default) */
 
 /* Status codes. */
 enum oit_status {
@@ -336,15 +338,20 @@ typedef struct oit_batch_frame {
 enum {
   OIT_BATCH_CONCURRENT = 0x1, /* resolve groups run on forked streams (join before return) */
   OIT_BATCH_GRAPH      = 0x2, /* a run is captured once per frame set and replayed as a hipGraph */
-  OIT_BATCH_FRAME_ORDER = 0x4 /* append frame after frame; by default the frames' fragment slices are
+  OIT_BATCH_FRAME_ORDER = 0x4 /* lists: append frame after frame; by default the frames' fragment slices are
                                  interleaved so that each frame advances in draw order with a share of
-                                 the waves in flight (fewer same-pixel inserts at once, same results) */
+                                 the waves in flight (fewer same-pixel inserts at once, same results).
+                                 Tiles (the default path) are always listed frame after frame */
 };
 
 /* Kernel choices of a batch: append chunks per wave (4 or 8) and, per
  * (K, tail_blend) group, the resolve variant bits (OIT_VARIANT_LL_SINGLE_WALK,
  * OIT_VARIANT_LL_KEYS_ONLY) and a cap on resolve blocks (0 = one block per
- * tile). Index [k][tail] with k = log2(K). */
+ * tile). Index [k][tail] with k = log2(K). These are choices of the paths with
+ * a list or a bucket per target; with the defaults and no
+ * OIT_VARIANT_BATCH_LISTS in any resolve_variant a batch composites tiles of
+ * 64 targets from the fragments themselves (lists where there is no memory
+ * for those, until the tuning is set again). */
 typedef struct oit_batch_tuning {
   uint32_t append_chunks;
   uint32_t resolve_variant[6][2];
@@ -359,7 +366,8 @@ typedef struct oit_batch_tuning {
 typedef struct oit_batch_sizes {
   uint64_t pool_nodes;        /* nodes the frames need, terminator included */
   uint64_t head_entries;      /* padded targets */
-  uint64_t bytes;             /* device bytes for those (nodes 12 B, heads 4 B) */
+  uint64_t bytes;             /* device bytes the tuning's path takes for those: lists 12 B a node and a head, tiles
+                                 20 B a fragment and 776 B per 64 heads */
   uint32_t groups;            /* resolve launches */
   uint32_t frames;
 } oit_batch_sizes;
@@ -369,14 +377,17 @@ int oit_batch_create(oit_batch** out, int device, uint32_t flags);
 int oit_batch_destroy(oit_batch* b);
 /* Pool and head sizes `frames` need (no device work). */
 int oit_batch_query(const oit_batch* b, const oit_batch_frame* frames, uint32_t n, oit_batch_sizes* out);
-/* Grows the resident pool to at least these sizes (never shrinks). */
+/* Grows the resident structures of the tuning's path to at least these sizes
+ * (never shrinks). */
 int oit_batch_reserve(oit_batch* b, uint64_t pool_nodes, uint64_t head_entries);
 /* Appends and resolves every frame on `stream`. Grows the pool when needed
  * (the only allocation). Fragment and output buffers must stay valid until
  * the stream reaches the end of the run. */
 int oit_batch_run(oit_batch* b, const oit_batch_frame* frames, uint32_t n, void* stream);
 /* Times the kernel variants on these frames (synchronous, runs the batch
- * several times) and keeps the fastest per group for later runs. */
+ * several times) and keeps the fastest for later runs: the tiles (the default
+ * tuning) or the lists with the fastest variants per group, named with
+ * OIT_VARIANT_BATCH_LISTS. The other path's memory is given back. */
 int oit_batch_tune(oit_batch* b, const oit_batch_frame* frames, uint32_t n, void* stream);
 int oit_batch_get_tuning(const oit_batch* b, oit_batch_tuning* out);
 int oit_batch_set_tuning(oit_batch* b, const oit_batch_tuning* t);

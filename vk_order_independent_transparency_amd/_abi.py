@@ -46,6 +46,7 @@ VARIANT_LL_APPEND_8 = 0x4
 VARIANT_LL_KEYS_ONLY = 0x8
 VARIANT_STORE_CHUNKS_1 = 0x10
 VARIANT_STORE_CHUNKS_4 = 0x20
+VARIANT_BATCH_LISTS = 0x40  # batch tunings only
 
 BATCH_CONCURRENT = 0x1
 BATCH_GRAPH = 0x2

@@ -20,8 +20,9 @@
 // fragments, 155 to 2810 spheres a frame, a fifth clustered) takes 3.6 ms so
 // and 6.6 ms with lists, whose ordered inserts walk past each other on the
 // clustered pixels. A tuning that asks for anything but the defaults gets the
-// list or bucket kernels it names; so does a batch without memory for the
-// tiles (20 bytes a fragment, the lists 12).
+// list or bucket kernels it names, and one with OIT_VARIANT_BATCH_LISTS the
+// lists in any case; so does a batch without memory for the tiles (20 bytes a
+// fragment, the lists 12).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -220,7 +221,9 @@ bool tuning_valid(const oit_batch_tuning& t) {
   if (!(t.bin_density >= 0.f)) return false;  // NaN too
   for (int k = 0; k < 6; ++k)
     for (int tl = 0; tl < 2; ++tl)
-      if (t.resolve_variant[k][tl] & ~(OIT_VARIANT_LL_SINGLE_WALK | OIT_VARIANT_LL_KEYS_ONLY)) return false;
+      if (t.resolve_variant[k][tl] &
+          ~(OIT_VARIANT_LL_SINGLE_WALK | OIT_VARIANT_LL_KEYS_ONLY | OIT_VARIANT_BATCH_LISTS))
+        return false;
   return true;
 }
 
@@ -246,7 +249,7 @@ struct oit_batch {
   // tile path: run structures per tile of 64 heads, links per fragment
   oit::TileBuf tile;
   uint64_t cap_tile_heads = 0, cap_tile_frags = 0;
-  bool prefer_lists = false;     // the tuner found the lists faster on its frames
+  bool no_tile_memory = false;   // there was none for the tile path under this tuning: lists
   bool dirty = false;            // a run did not complete: re-initialise before the next (lists)
   bool tile_dirty = false;       // likewise (tile path)
   // frame table
@@ -284,16 +287,22 @@ void drop_tiles(oit_batch* b) {
   b->cap_tile_heads = b->cap_tile_frags = 0;
 }
 
+// The lists' structures whose size follows the frames.
+void drop_pool(oit_batch* b) {
+  for (uint32_t** q : {&b->next, &b->head, &b->cursor, &b->deep_q, &b->tile_sum}) {
+    (void)hipFree(*q);
+    *q = nullptr;
+  }
+  (void)hipFree(b->cd);
+  b->cd = nullptr;
+  b->cap_nodes = b->cap_heads = 0;
+}
+
 void release(oit_batch* b) {
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
   (void)hipFree(b->d_tab);
-  (void)hipFree(b->head);
-  (void)hipFree(b->cd);
-  (void)hipFree(b->next);
+  drop_pool(b);
   (void)hipFree(b->counters);
-  (void)hipFree(b->cursor);
-  (void)hipFree(b->deep_q);
-  (void)hipFree(b->tile_sum);
   (void)hipFree(b->deep_n);
   drop_tiles(b);
   (void)hipFree(b->d_table);
@@ -369,7 +378,7 @@ int ensure_pool(oit_batch* b, uint64_t nodes, uint64_t heads, hipStream_t s) {
 
 bool same_tuning(const oit_batch_tuning& a, const oit_batch_tuning& t) { return std::memcmp(&a, &t, sizeof a) == 0; }
 
-bool tile_path(const oit_batch* b) { return !b->prefer_lists && same_tuning(b->tuning, default_tuning()); }
+bool tile_path(const oit_batch* b) { return !b->no_tile_memory && same_tuning(b->tuning, default_tuning()); }
 
 // Bytes of the tile path's structures.
 uint64_t tile_bytes(uint64_t frags, uint64_t heads) {
@@ -641,6 +650,15 @@ int run_graph(oit_batch* b, const Plan& p, hipStream_t s) {
   return st(hipGraphLaunch(b->gexec, s));
 }
 
+// Grows the lists' structures; the tile path's make room for them where they
+// have to (ensure_pool has waited for the device before it allocates).
+int ensure_lists(oit_batch* b, uint64_t nodes, uint64_t heads, hipStream_t s) {
+  const int rc = ensure_pool(b, nodes, heads, s);
+  if (rc != OIT_ERR_OOM || !(b->cap_tile_frags || b->cap_tile_heads)) return rc;
+  drop_tiles(b);
+  return ensure_pool(b, nodes, heads, s);
+}
+
 // Grows what the path in use needs for these pool nodes and heads. The tile
 // path takes 20 bytes a fragment, the lists 12: without memory for the one,
 // the batch goes over to the other.
@@ -649,10 +667,10 @@ int ensure_path(oit_batch* b, uint64_t nodes, uint64_t heads, hipStream_t s) {
     const int rc = ensure_tiles(b, nodes ? nodes - 1u : 0u, heads, s);
     if (rc != OIT_ERR_OOM) return rc;
     drop_tiles(b);
-    b->prefer_lists = true;
+    b->no_tile_memory = true;
     ++b->tuning_version;
   }
-  return ensure_pool(b, nodes, heads, s);
+  return ensure_lists(b, nodes, heads, s);
 }
 
 int prepare(oit_batch* b, const oit_batch_frame* frames, uint32_t n, Plan& p, hipStream_t s) {
@@ -762,10 +780,11 @@ int oit_batch_tune(oit_batch* b, const oit_batch_frame* frames, uint32_t n, void
   int rc = make_plan(frames, n, p, b->tuning.bin_density);
   if (rc) return rc;
   rc = ensure_tiles(b, p.pool_slots, p.heads, s);
-  const bool no_tiles = rc == OIT_ERR_OOM;
-  if (no_tiles) drop_tiles(b);
+  if (rc == OIT_ERR_OOM) drop_tiles(b);
   else if (rc) return rc;
-  if ((rc = ensure_pool(b, p.pool_slots + 1, p.heads, s))) return rc;
+  if ((rc = ensure_lists(b, p.pool_slots + 1, p.heads, s))) return rc;
+  // without memory for both, the lists alone are tuned
+  const bool no_tiles = b->cap_tile_frags < p.pool_slots || b->cap_tile_heads < p.heads;
   if (p.table.empty()) return OIT_OK;
   if ((rc = upload_table(b, p, s))) return rc;
   const size_t G = p.groups.size();
@@ -906,9 +925,24 @@ int oit_batch_tune(oit_batch* b, const oit_batch_frame* frames, uint32_t n, void
     b->dirty = b->tile_dirty = true;
     return rc;
   }
-  b->prefer_lists = no_tiles || lists_ms < tiles_ms;
-  b->tuning = b->prefer_lists ? best : default_tuning();
+  // Tiles are the default tuning; lists are named, so that this choice holds
+  // where it is read and set again. The other path's memory is given back.
+  const bool lists = no_tiles || lists_ms < tiles_ms;
+  b->tuning = lists ? best : default_tuning();
+  b->no_tile_memory = false;
   ++b->tuning_version;
+  if (b->gexec) {  // its launches hold pointers of either path
+    (void)hipGraphExecDestroy(b->gexec);
+    b->gexec = nullptr;
+  }
+  if ((rc = st(hipStreamSynchronize(s)))) return rc;
+  if (lists) {
+    for (auto& k : b->tuning.resolve_variant)
+      for (uint32_t& v : k) v |= OIT_VARIANT_BATCH_LISTS;
+    drop_tiles(b);
+  } else {
+    drop_pool(b);
+  }
   return OIT_OK;
 }
 
@@ -921,7 +955,7 @@ int oit_batch_get_tuning(const oit_batch* b, oit_batch_tuning* out) {
 int oit_batch_set_tuning(oit_batch* b, const oit_batch_tuning* t) {
   if (!b || !t || !tuning_valid(*t)) return OIT_ERR_INVALID_ARG;
   b->tuning = *t;
-  b->prefer_lists = false;
+  b->no_tile_memory = false;
   ++b->tuning_version;
   return OIT_OK;
 }
