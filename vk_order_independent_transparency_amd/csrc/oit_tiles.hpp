@@ -37,6 +37,8 @@
 // here with its own order and tail rule (TileMode).
 #pragma once
 
+#include <cstddef>
+
 #include "oit_frame.hpp"
 
 namespace oit {
@@ -70,8 +72,10 @@ template <>
 struct EntryOf<true> {
   using T = TileEntryId;
 };
+// Aligned for the 64-bit runs that are sorted in the entries' space: a block
+// holds several of these one behind the other.
 template <int C, bool kId>
-struct TileLds {
+struct alignas(16) TileLds {
   static constexpr uint32_t kEntries = C;
   static constexpr bool kHasId = kId;
   static constexpr uint32_t kSize = sizeof(typename EntryOf<kId>::T);
@@ -1366,6 +1370,14 @@ constexpr uint32_t kComputeUnits = 256;
 // bound asks for.
 // (12 or 16 bytes each: about the same LDS.)
 constexpr int tile_entries(bool id) { return id ? 520 : 696; }
+template <bool kId>
+constexpr bool tile_lds_ok() {
+  using Lds = TileLds<tile_entries(kId), kId>;
+  // four blocks of four waves, with the decode tables, in a compute unit's 160 KB
+  return alignof(Lds) % alignof(uint64_t) == 0 && offsetof(Lds, e) == 0 &&
+         4u * (4u * sizeof(Lds) + 2048u) <= 160u * 1024u;
+}
+static_assert(tile_lds_ok<false>() && tile_lds_ok<true>(), "alignment and size of a wave's LDS");
 template <int K>
 constexpr int tile_waves() { return K >= 32 ? 3 : 4; }
 
