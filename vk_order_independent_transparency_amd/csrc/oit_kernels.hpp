@@ -176,9 +176,9 @@ inline uint64_t tile_count(uint64_t targets) { return (targets + 63u) / 64u; }
 
 struct TileBuf {
   uint32_t* cnt = nullptr;   // [tiles] runs of the frame; 0 between frames
-  uint64_t* run = nullptr;   // [tiles][kTileRuns] first id << 32 | length
+  uint64_t* run = nullptr;   // [tiles][kTileRuns] first id << 32 | own fragments << 8 | length
   uint32_t* more = nullptr;  // [tiles][kTileRuns] later runs: first id + 1 of each list's last one, 0 = empty
-  uint64_t* link = nullptr;  // [fragments] of a later run, at its first id: length << 32 | the list's next value
+  uint64_t* link = nullptr;  // [fragments] of a later run, at its first id: own << 40 | length << 32 | the list's next value
   uint32_t* deep = nullptr;  // [tiles] queue of the tiles left to the deep composite
   uint32_t* ctl = nullptr;   // [kTileCtlAll] queue length and ticket per group, tail counters (zeroed by the appends), shares
   uint32_t deep_base = 0;    // the group's part of the queue

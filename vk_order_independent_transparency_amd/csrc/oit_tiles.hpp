@@ -11,10 +11,12 @@
 // lists in LDS and sorts them in registers.
 //
 // Pass 1 (k_tile_link, per append): each wave cuts its 64-fragment chunks
-// into runs of one tile and publishes every run (first id, length) with one
-// returning add on the tile's run count: the first kTileRuns runs go to the
-// tile's own slots, later ones onto kTileRuns unordered lists of the tile
-// (run number mod kTileRuns), so that a wave walks them side by side.
+// into runs of one tile (with short gaps where there are many, join_gaps) and
+// publishes every run (first id, length, the tile's own fragments among
+// those) with one returning add on the tile's run count: the first kTileRuns
+// runs go to the tile's own slots, later ones onto kTileRuns unordered lists
+// of the tile (run number mod kTileRuns), so that a wave walks them side by
+// side.
 // Pass 2 (k_tile_resolve): one wave per tile sorts the runs by first id,
 // takes their fragments 64 at a time, pushes (key, colour) onto the targets'
 // lists in LDS in ascending id, and each lane then walks its own target's
@@ -46,6 +48,12 @@ namespace oit {
 namespace {
 
 constexpr uint32_t kTileTargets = 64;
+
+// A run's word: ids it goes over (1 .. 64) and how many of them are the
+// tile's own.
+__device__ __forceinline__ uint32_t pack_run(uint32_t len, uint32_t own) { return len | own << 8; }
+__device__ __forceinline__ uint32_t run_len(uint32_t w) { return w & 255u; }
+__device__ __forceinline__ uint32_t run_own(uint32_t w) { return w >> 8; }
 
 // Per-wave LDS of a group of fragments: entries in ascending id, 1 ..
 // kEntries, linked per target. A list value is the entry's LDS address, so a
@@ -277,11 +285,13 @@ __device__ __forceinline__ void mark_run(Lds& w, bool on, uint32_t off) {
 // is `part`. The runs have `size` positions in all (at most kMaxPositions),
 // their starts marked in w.bits and the words at LDS address `deltas` giving
 // each one's first id minus first position; id0 is a fragment of theirs.
+// `base` is the list index of the tile's first target: fragments of other
+// tiles, in a run's gaps, are in no part.
 // Returns false (wave-uniform) where the fragments are more than `cap`.
 template <bool kStored, bool kMany, typename Lds>
 __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const CodecTables* tab, uint32_t deltas,
                                             uint32_t id0, uint32_t size, uint32_t shift, uint32_t part, uint32_t cap,
-                                            uint32_t target, bool in) {
+                                            uint32_t base, uint32_t target, bool in) {
   constexpr int kU = 3;  // 64-fragment batches in flight together
   const uint32_t lane = lane_id();
   const uint32_t nb = (size + 63u) >> 6;
@@ -373,7 +383,7 @@ __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const Co
         continue;
       }
       if constexpr (!kStored) {
-        loc[u] = pm_index(loc[u], src.T, src.spp) & 63u;
+        loc[u] = pm_index(loc[u], src.T, src.spp) - base;
         key[u] = depth_key(dv[u]);
         col[u] = encode_color_quick(cv[u], tab);
       }
@@ -817,7 +827,7 @@ __device__ __forceinline__ void exact_composite(TileLane& L, const TileSrc& src,
   }
 }
 
-// Calls f(first id, length, valid) for up to 64 of the tile's m runs at a
+// Calls f(first id, word, valid) for up to 64 of the tile's m runs at a
 // time, every lane of the wave taking part. The lists hold every
 // kTileRuns-th run after the slots', so a walk ends after as many trips.
 template <typename F>
@@ -902,7 +912,7 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
                                           const TileDst& dst, Lds& w, const float* s_dec, const float* s_alpha,
                                           TileQueue* queue) {
   const uint32_t lane = lane_id();
-  const uint32_t a = (tile - dst.tile0) * kTileTargets + lane;  // list index in the frame
+  const uint32_t base = (tile - dst.tile0) * kTileTargets, a = base + lane;  // list indices in the frame
   const bool in = a < dst.T;
   TileLane L;
   L.tile = tile;
@@ -926,7 +936,8 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
     }
     return;
   }
-  uint32_t size, id0, deltas = lds_address(w.delta), cap = Lds::kEntries;
+  // positions of the runs, and the tile's own fragments among them
+  uint32_t size, frags, id0, deltas = lds_address(w.delta), cap = Lds::kEntries;
   if (m <= 64u) {
     uint32_t start = kEmpty, len = 0u;
     uint64_t rec = ahead.rec;
@@ -935,12 +946,14 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
       start = (uint32_t)(rec >> 32);
       len = (uint32_t)rec;
     }
+    frags = __builtin_amdgcn_readlane(wave_scan_u32(run_own(len)), 63);
     if constexpr (kMode == kTileList) {
-      if ((__builtin_amdgcn_readlane(wave_scan_u32(len), 63) >> split) > cap) {  // binned instead
+      if ((frags >> split) > cap) {  // binned instead
         end_share(tb, tile, m, first, split, true, queue);
         return;
       }
     }
+    len = run_len(len);
     // the runs in ascending order of their first ids
     uint32_t rank = 0;
     for (uint32_t j = 0; j < m; ++j) rank += __builtin_amdgcn_readlane(start, j) < start ? 1u : 0u;
@@ -970,10 +983,11 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
     deltas = lds_address(delta);
     id0 = rfl((uint32_t)(run[0] >> 32));
     clear_marks(w);
-    size = 0;
+    size = frags = 0;
     for (uint32_t c = 0; c < got; c += 64u) {
       const uint64_t rec = c + lane < got ? run[c + lane] : 0ull;
-      const uint32_t len = (uint32_t)rec;
+      const uint32_t len = run_len((uint32_t)rec);
+      frags += __builtin_amdgcn_readlane(wave_scan_u32(run_own((uint32_t)rec)), 63);
       const uint32_t incl = wave_scan_u32(len);
       const uint32_t off = size + incl - len;
       size += __builtin_amdgcn_readlane(incl, 63);
@@ -992,11 +1006,11 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
   // part that is still too large is halved
   uint32_t shift = 6u - split;
   if constexpr (kMode != kTileList) {
-    while (shift > 0u && (size >> (6u - shift)) > cap) --shift;
+    while (shift > 0u && (frags >> (6u - shift)) > cap) --shift;
   }
   for (uint32_t t0 = first; t0 < last;) {
     const uint32_t part = t0 >> shift;
-    if (!build_lists<kStored, kGeneral>(w, src, dst.tab, deltas, id0, size, shift, part, cap, L.t, in)) {
+    if (!build_lists<kStored, kGeneral>(w, src, dst.tab, deltas, id0, size, shift, part, cap, base, L.t, in)) {
       wave_lds_sync();
       if (shift == 0u || kMode == kTileList) {  // one target's fragments
         end_share(tb, tile, m, first, split, true, queue);
@@ -1097,7 +1111,7 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
     uint32_t e = load_runs<kDeepRuns>(w.run, tb, tile, m, lo, hi);
     while (e > 0u) {
       // as many of the newest runs as one group holds
-      const uint32_t len0 = lane < e ? (uint32_t)w.run[e - 1u - lane] : 0u;
+      const uint32_t len0 = lane < e ? run_len((uint32_t)w.run[e - 1u - lane]) : 0u;
       const uint32_t sum = wave_scan_u32(len0);
       const uint32_t r = (uint32_t)__builtin_popcountll(__ballot(lane < e && sum <= (uint32_t)kDeepEntries));
       if (r == 0u) break;  // no run is longer than a group
@@ -1106,7 +1120,7 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
       if (lane < r) {
         const uint64_t rec = w.run[first + lane];
         start = (uint32_t)(rec >> 32);
-        len = (uint32_t)rec;
+        len = run_len((uint32_t)rec);
       }
       const uint32_t incl = wave_scan_u32(len);
       const uint32_t N = __builtin_amdgcn_readlane(incl, 63);
@@ -1114,7 +1128,8 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
       mark_run(w.g, lane < r, incl - len);
       w.g.delta[lane] = start - (incl - len);
       wave_lds_sync();
-      (void)build_lists<kStored, true>(w.g, src, dst.tab, lds_address(w.g.delta), rfl(start), N, 6u, 0u, kDeepEntries, t, in);
+      (void)build_lists<kStored, true>(w.g, src, dst.tab, lds_address(w.g.delta), rfl(start), N, 6u, 0u, kDeepEntries,
+                                         (tile - dst.tile0) * kTileTargets, t, in);
       body(first == 0u && lo == 0u);
       ++groups;
       wave_lds_sync();
