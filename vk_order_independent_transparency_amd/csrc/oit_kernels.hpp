@@ -171,11 +171,12 @@ constexpr uint32_t kTileTickets = kTileShares + kBatchMaxGroups * kSharedTiles; 
 constexpr uint32_t kTicketLanes = 8;
 constexpr uint32_t kTicketWords = 2u * kTicketLanes * 16u;
 constexpr uint32_t kTileCtlBatch = kTileTickets + kBatchMaxGroups * kTicketWords;
+constexpr uint32_t kTileUncounted = 1u << 31;  // cnt: the tile's lists hold runs that are not counted too
 constexpr uint32_t kDeepBlocks = 1024;    // waves of the deep composite (tickets hand out its tiles)
 inline uint64_t tile_count(uint64_t targets) { return (targets + 63u) / 64u; }
 
 struct TileBuf {
-  uint32_t* cnt = nullptr;   // [tiles] runs of the frame; 0 between frames
+  uint32_t* cnt = nullptr;   // [tiles] runs of the frame, and kTileUncounted; 0 between frames
   uint64_t* run = nullptr;   // [tiles][kTileRuns] first id << 32 | own fragments << 8 | length
   uint32_t* more = nullptr;  // [tiles][kTileRuns] later runs: first id + 1 of each list's last one, 0 = empty
   uint64_t* link = nullptr;  // [fragments] of a later run, at its first id: own << 40 | length << 32 | the list's next value

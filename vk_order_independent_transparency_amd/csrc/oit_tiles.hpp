@@ -16,7 +16,7 @@
 // those) with one returning add on the tile's run count: the first kTileRuns
 // runs go to the tile's own slots, later ones onto kTileRuns unordered lists
 // of the tile (run number mod kTileRuns), so that a wave walks them side by
-// side.
+// side. Chunks without any order put their runs on the lists directly.
 // Pass 2 (k_tile_resolve): one wave per tile sorts the runs by first id,
 // takes their fragments 64 at a time, pushes (key, colour) onto the targets'
 // lists in LDS in ascending id, and each lane then walks its own target's
@@ -827,48 +827,92 @@ __device__ __forceinline__ void exact_composite(TileLane& L, const TileSrc& src,
   }
 }
 
-// Calls f(first id, word, valid) for up to 64 of the tile's m runs at a
-// time, every lane of the wave taking part. The lists hold every
-// kTileRuns-th run after the slots', so a walk ends after as many trips.
+// Calls f(first id, word, valid) for up to 64 of the tile's runs at a time,
+// every lane of the wave taking part: the slots', and where m is past those
+// (or marked kTileUncounted, which is past any) the lists' to their ends.
 template <typename F>
 __device__ __forceinline__ void each_run(const TileBuf& tb, uint32_t tile, uint32_t m, F&& f) {
   const uint32_t lane = lane_id();
   {
-    const bool on = lane < kTileRuns && lane < m;
+    const bool on = lane < kTileRuns && lane < (m & ~kTileUncounted);
     const uint64_t rec = on ? tb.run[(uint64_t)tile * kTileRuns + lane] : 0ull;
     f((uint32_t)(rec >> 32), (uint32_t)rec, on);
   }
-  uint32_t v = lane < kTileRuns && lane + kTileRuns < m ? tb.more[(uint64_t)tile * kTileRuns + lane] : 0u;
-  for (uint32_t at = kTileRuns; at < m; at += kTileRuns) {
-    const bool on = v != 0u && at + lane < m;
+  uint32_t v = m > kTileRuns ? tb.more[(uint64_t)tile * kTileRuns + lane] : 0u;
+  while (__ballot(v != 0u) != 0ull) {
+    const bool on = v != 0u;
     const uint64_t l = on ? tb.link[v - 1u] : 0ull;
     f(v - 1u, (uint32_t)(l >> 32), on);
     v = on ? (uint32_t)l : 0u;
   }
 }
 
-// Ascending bitonic sort of run[0 .. size) (a power of two) by one wave.
-__device__ __forceinline__ void sort_runs(uint64_t* run, uint32_t size) {
-  for (uint32_t k = 2; k <= size; k <<= 1) {
-    for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-      wave_lds_sync();
-      for (uint32_t i = lane_id(); i < size; i += 64u) {
-        const uint32_t x = i ^ j;
-        if (x > i) {
-          const uint64_t u = run[i], v = run[x];
-          if (((i & k) == 0u) == (u > v)) {
-            run[i] = v;
-            run[x] = u;
-          }
+// Sorts run[0 .. got) ascending, got <= 64 R, by one wave: R runs a lane in
+// registers, sorted in the lane and then merged over 2, 4 .. 64 lanes, each
+// merge by a step against the mirrored lane and halving steps after it
+// (Batcher's bitonic merge with all of its exchanges ascending). A run's 48
+// bits (first id, own, length) are a double in the integers' order, as the
+// sort keys are. Bound by its 21 exchanges between lanes of R values each; in
+// LDS, 512 runs took 45 steps of four exchanges, one waiting for the other
+// (1920x1080 shuffled, about 400 runs a tile: Loop64 4.30 ms so, 3.10 in
+// registers; 256x256: 464 and 272 us).
+template <int R>
+__device__ __forceinline__ void sort_runs(uint64_t* run, uint32_t got) {
+  const uint32_t lane = lane_id();
+  double v[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t i = lane * R + (uint32_t)r;
+    const uint64_t x = i < got ? run[i] : 0ull;
+    const uint32_t first = (uint32_t)(x >> 32);
+    v[r] = i < got ? pack2(first >> 16, first << 16 | (uint32_t)x) : pack2(0x3FFFFFFFu, 0u);
+  }
+  wave_lds_sync();
+  sort_net<R>(v);
+  auto swap_with = [&](uint32_t mask, uint32_t bit, bool mirror) {
+    double o[R];
+    const int from = (int)((lane ^ mask) << 2);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const double x = v[r];
+      o[r] = pack2((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)hi32(x)),
+                   (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)lo32(x)));
+    }
+    const bool low = (lane & bit) == 0u;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const double x = mirror ? o[R - 1 - r] : o[r];
+      v[r] = (x < v[r]) == low ? x : v[r];
+    }
+  };
+#pragma unroll 1
+  for (uint32_t w = 2; w <= 64u; w <<= 1) {
+    swap_with(w - 1u, w >> 1, true);
+#pragma unroll 1
+    for (uint32_t h = w >> 2; h > 0u; h >>= 1) swap_with(h, h, false);
+#pragma unroll
+    for (int j = R / 2; j > 0; j >>= 1) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if ((r & j) == 0) {
+          const double x = v[r], y = v[r + j];
+          v[r] = min_raw(x, y);
+          v[r + j] = max_raw(x, y);
         }
       }
     }
   }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t i = lane * R + (uint32_t)r;
+    if (i < got)
+      run[i] = ((uint64_t)(hi32(v[r]) << 16 | lo32(v[r]) >> 16) << 32) | (lo32(v[r]) & 0xFFFFu);
+  }
   wave_lds_sync();
 }
 
-// The runs of the tile whose first id is in [lo, hi), at most kMost of them
-// (a power of two), sorted, into run[].
+// The runs of the tile whose first id is in [lo, hi), sorted, into run[], and
+// how many they are; where that is over kMost, nothing is in order.
 template <uint32_t kMost>
 __device__ __forceinline__ uint32_t load_runs(uint64_t* run, const TileBuf& tb, uint32_t tile, uint32_t m, uint64_t lo,
                                               uint64_t hi) {
@@ -880,18 +924,18 @@ __device__ __forceinline__ uint32_t load_runs(uint64_t* run, const TileBuf& tb, 
     if (on && at < kMost) run[at] = ((uint64_t)start << 32) | len;
     got += (uint32_t)__builtin_popcountll(mask);
   });
-  if (got > kMost) got = kMost;
-  uint32_t size = 2;
-  while (size < got) size <<= 1;
-  for (uint32_t i = got + lane_id(); i < size; i += 64u) run[i] = kEmpty64;
-  sort_runs(run, size);
+  wave_lds_sync();
+  if (got > kMost) return got;
+  if (got <= 256u) sort_runs<4>(run, got);
+  else if (kMost <= 512u || got <= 512u) sort_runs<8>(run, got);
+  else sort_runs<(int)(kMost / 64u)>(run, got);
   return got;
 }
 
 // What a wave loads of a tile ahead of its turn: the run count and the lanes'
 // runs.
 constexpr uint32_t kAheadRuns = 32;
-constexpr uint32_t kManyRuns = 512;  // runs that the wave's LDS sorts
+constexpr uint32_t kManyRuns = 1024;  // runs that a wave sorts
 struct TileAhead {
   uint32_t m;
   uint64_t rec;
@@ -970,30 +1014,40 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
     end_share(tb, tile, m, first, split, true, queue);
     return;
   } else {
-    // short runs: gathered and sorted in the entries' space, of which their
-    // deltas then take the end
-    if (m > kManyRuns) {
+    // many runs: gathered and sorted in the entries' space, of which their
+    // deltas then take the end, 4 bytes a run
+    if (m > kManyRuns && !(m & kTileUncounted)) {
       end_share(tb, tile, m, first, split, true, queue);
       return;
     }
     uint64_t* const run = reinterpret_cast<uint64_t*>(&w.e[0]);
     const uint32_t got = load_runs<kManyRuns>(run, tb, tile, m, 0u, 1ull << 32);
-    cap = Lds::kEntries - (kManyRuns * 4u + Lds::kSize - 1u) / Lds::kSize;
+    if (got > kManyRuns) {
+      end_share(tb, tile, m, first, split, true, queue);
+      return;
+    }
+    cap = Lds::kEntries - (got * (uint32_t)sizeof(uint32_t) + Lds::kSize - 1u) / Lds::kSize;
+    static_assert(kManyRuns * sizeof(uint64_t) <= sizeof w.e, "the runs fit the entries' space");
     uint32_t* const delta = reinterpret_cast<uint32_t*>(&w.e[cap + 1u]);
     deltas = lds_address(delta);
     id0 = rfl((uint32_t)(run[0] >> 32));
+    // all of the runs are read before the first delta is written: the deltas
+    // lie over the last ones
+    uint64_t rec[kManyRuns / 64u];
+#pragma unroll
+    for (uint32_t c = 0; c < kManyRuns / 64u; ++c) rec[c] = c * 64u + lane < got ? run[c * 64u + lane] : 0ull;
     clear_marks(w);
     size = frags = 0;
-    for (uint32_t c = 0; c < got; c += 64u) {
-      const uint64_t rec = c + lane < got ? run[c + lane] : 0ull;
-      const uint32_t len = run_len((uint32_t)rec);
-      frags += __builtin_amdgcn_readlane(wave_scan_u32(run_own((uint32_t)rec)), 63);
+#pragma unroll
+    for (uint32_t c = 0; c < kManyRuns / 64u; ++c) {
+      const bool on = c * 64u + lane < got;
+      const uint32_t len = run_len((uint32_t)rec[c]);
+      frags += __builtin_amdgcn_readlane(wave_scan_u32(run_own((uint32_t)rec[c])), 63);
       const uint32_t incl = wave_scan_u32(len);
       const uint32_t off = size + incl - len;
       size += __builtin_amdgcn_readlane(incl, 63);
-      if (size > kMaxPositions) break;
-      mark_run(w, c + lane < got, off);
-      if (c + lane < got) delta[c + lane] = (uint32_t)(rec >> 32) - off;
+      if (size <= kMaxPositions) mark_run(w, on, off);
+      if (on) delta[c * 64u + lane] = (uint32_t)(rec[c] >> 32) - off;
     }
     if (size > kMaxPositions) {
       end_share(tb, tile, m, first, split, true, queue);
@@ -1081,7 +1135,7 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
   uint64_t hi = 1ull << 32;
   while (hi > 0u) {
     uint64_t lo = 0;
-    if (m > kDeepRuns) {
+    if (m > kTileRuns) {  // (the lists may hold uncounted runs)
       // a window of at most kDeepRuns runs below hi: first ids differ, so a
       // span of kDeepRuns ids is one; bisected down to a fuller one
       auto count = [&](uint64_t from) {
