@@ -13,12 +13,14 @@ namespace {
 // other tiles in between, which the composite drops. A rasteriser that walks
 // triangles in 2x2 quads alternates between two rows, so that a chunk is two
 // runs so and up to 32 without (1920x1080 in quads, 12.7 M fragments: Loop64
-// K = 8 502 us without, 295 with, 310 with an atomic per fragment; K = 16 518,
-// 307, 247; Loop32 588, 354, 358). The gap is as long as what a quad of four
-// front and four back fragments needs; chunks of few runs, as raster order
-// leaves them, are not looked through (22 us for this pass either way).
-constexpr int kManyStarts = 8;  // runs of a chunk from which gaps are looked for
-constexpr uint32_t kGap = 8;
+// K = 8 502 us without, 286 with, 310 with an atomic per fragment; K = 16 518,
+// 303, 247; Loop32 588, 342, 358). The gap is as long as what a quad of four
+// front and four back fragments needs. Chunks of few runs, as raster order
+// leaves them, are not looked through, and the code is kept small: unrolled
+// over lanes and chunks it took them 23.5 us instead of 22.
+constexpr int kManyStarts = 12;  // runs of a chunk from which gaps are looked for
+constexpr uint32_t kGap = 8;    // (join_gaps' shifts go by it)
+constexpr int kGapTiles = 16;
 // A chunk that is still of more than kDirectRuns runs puts them on the tiles'
 // lists, list by lane, without drawing a place: one atomic a run instead of
 // two, and no scattered record (1920x1080 shuffled, 12.7 M runs: 1.39 ms for
@@ -27,23 +29,72 @@ constexpr uint32_t kGap = 8;
 // a batch, whose binning goes by the run counts.
 constexpr int kDirectRuns = 32;
 __device__ __forceinline__ void join_gaps(uint32_t tile, bool& lead, uint32_t& run) {
+  // the lanes of the lane's tile, for the first kGapTiles tiles of the chunk
+  uint64_t mine = 0ull, left = __ballot(tile != kEmpty);
+#pragma unroll 1
+  for (int n = 0; left != 0ull && n < kGapTiles; ++n) {
+    const uint64_t same = __ballot(tile == (uint32_t)__builtin_amdgcn_readlane(tile, __builtin_ctzll(left)));
+    if ((same >> lane_id()) & 1u) mine = same;
+    left &= ~same;
+  }
+  if (mine == 0ull) return;
   const uint32_t lane = lane_id();
-  uint32_t last = lane;
-  bool joined = false;
-#pragma unroll
-  for (uint32_t g = kGap; g > 0u; --g) {
-    const uint32_t after = __shfl_down(tile, g), before = __shfl_up(tile, g);
-    if (lane + g < 64u && after == tile) last = lane + g;
-    joined = joined || (lane >= g && before == tile);
+  lead = lane == 0u || (mine << (64u - lane)) >> (64u - kGap) == 0ull;
+  // from the lane on: every member and the kGap - 1 lanes after it; the next
+  // gap of that ends the chain
+  const uint64_t from = mine >> lane;
+  uint64_t reach = from | from << 1;
+  reach |= reach << 2;
+  reach |= reach << 4;
+  const uint64_t chain = ~reach ? from & ((1ull << __builtin_ctzll(~reach)) - 1ull) : from;
+  run = pack_run(64u - (uint32_t)__builtin_clzll(chain), (uint32_t)__builtin_popcountll(chain));
+}
+
+// One of a tile's runs of which another `place` came before: into the tile's
+// own slots, or onto its lists.
+__device__ __forceinline__ void put_run(const TileBuf& tb, uint32_t tile, uint32_t place, uint32_t id, uint32_t word) {
+  const uint64_t at = (uint64_t)tile * kTileRuns;
+  if (place < kTileRuns) {
+    tb.run[at + place] = ((uint64_t)id << 32) | word;
+  } else {
+    const uint32_t prev = __hip_atomic_exchange(&tb.more[at + place % kTileRuns], id + 1u, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+    tb.link[id] = ((uint64_t)word << 32) | prev;
   }
-  uint32_t links = last != lane ? 1u : 0u;  // to the chain's end, by pointer doubling
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    links += (uint32_t)__shfl((int)links, (int)last);
-    last = (uint32_t)__shfl((int)last, (int)last);
+}
+
+// The run that starts at the lane, of a chunk whose runs start at `starts`.
+__device__ __forceinline__ uint32_t run_from(uint64_t starts) {
+  const uint64_t above = (starts >> lane_id()) >> 1;
+  const uint32_t len = above ? (uint32_t)__builtin_ctzll(above) + 1u : 64u - lane_id();
+  return pack_run(len, len);
+}
+
+// A chunk of many runs, from its targets on (a wave comes here with all of
+// its chunks, one by one: little code beside the path that raster order takes).
+template <bool kDirect>
+__device__ __forceinline__ void link_scattered(const FragView& f, uint32_t T, uint32_t spp, uint32_t tile0,
+                                               const TileBuf& tb, uint64_t first) {
+  const uint64_t i = first + lane_id();
+  const bool in = i < f.count;
+  const uint32_t t = in ? f.target[i] : kEmpty;
+  const uint32_t tile = t < T ? tile0 + (pm_index(t, T, spp) >> 6) : kEmpty;
+  const uint32_t before = __shfl_up(tile, 1u);
+  const bool start = lane_id() == 0u || before != tile;
+  bool lead = start && tile != kEmpty;
+  uint32_t run = run_from(__ballot(start));
+  // (a fragment without a valid target inside a run could pass for one of its tile's)
+  if (__ballot(in && tile == kEmpty) == 0ull) join_gaps(tile, lead, run);
+  const uint32_t id = f.id_base + (uint32_t)i;
+  if (kDirect && __builtin_popcountll(__ballot(lead)) > kDirectRuns) {
+    if (!lead) return;
+    const uint32_t prev = __hip_atomic_exchange(&tb.more[(uint64_t)tile * kTileRuns + lane_id()], id + 1u,
+                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    tb.link[id] = ((uint64_t)run << 32) | prev;
+    if (prev == 0u) atomicOr(&tb.cnt[tile], kTileUncounted);
+  } else if (lead) {
+    put_run(tb, tile, atomicAdd(&tb.cnt[tile], 1u) & ~kTileUncounted, id, run);
   }
-  lead = !joined && tile != kEmpty;
-  run = pack_run(last - lane + 1u, links + 1u);
 }
 
 // Pass 1 over one source stream: fragments first .. first + 64 kU - 1.
@@ -63,69 +114,37 @@ __device__ __forceinline__ void link_wave(const FragView& f, uint32_t T, uint32_
     t[u] = in ? ld_stream(&f.target[i]) : kEmpty;
   }
   bool lead[kU];
+  uint64_t starts[kU];
+  uint32_t pos[kU];
   int most = 0;  // runs of a chunk
-  uint32_t len[kU], pos[kU];
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
     if (t[u] >= T) t[u] = kEmpty;
     const uint32_t tile = t[u] == kEmpty ? kEmpty : tile0 + (pm_index(t[u], T, spp) >> 6);
     const uint32_t before = __shfl_up(tile, 1u);
     const bool start = lane == 0u || before != tile;
-    const uint64_t starts = __ballot(start);
-    const uint64_t above = (starts >> lane) >> 1;
-    len[u] = above ? (uint32_t)__builtin_ctzll(above) + 1u : 64u - lane;
-    const int runs = __builtin_popcountll(starts);
+    starts[u] = __ballot(start);
+    const int runs = __builtin_popcountll(starts[u]);
     most = most > runs ? most : runs;
     lead[u] = start && tile != kEmpty;
-    len[u] = pack_run(len[u], len[u]);
     t[u] = tile;
     pos[u] = 0u;
     asm volatile("" : "+v"(pos[u]));  // the zeros are written before any atomic goes out
   }
-  bool direct[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) direct[u] = false;
   if (most > kManyStarts) {  // (wave-uniform)
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      // a fragment without a valid target inside a run could pass for one of its tile's
-      const bool in = first + (uint64_t)u * 64u + lane < f.count;
-      if (__ballot(in && t[u] == kEmpty) == 0ull) join_gaps(t[u], lead[u], len[u]);
-      if constexpr (kDirect) direct[u] = __builtin_popcountll(__ballot(lead[u])) > kDirectRuns;
-    }
+#pragma unroll 1
+    for (int u = 0; u < kU; ++u) link_scattered<kDirect>(f, T, spp, tile0, tb, first + (uint64_t)u * 64u);
+    return;
   }
 #pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    if (lead[u]) {
-      if (direct[u]) {
-        const uint32_t id = f.id_base + (uint32_t)(first + (uint64_t)u * 64u + lane);
-        pos[u] = __hip_atomic_exchange(&tb.more[(uint64_t)t[u] * kTileRuns + lane], id + 1u, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-      } else {
-        pos[u] = atomicAdd(&tb.cnt[t[u]], 1u);
-      }
-    }
-  }
+  for (int u = 0; u < kU; ++u)
+    if (lead[u]) pos[u] = atomicAdd(&tb.cnt[t[u]], 1u);
   returns_done();
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
-    if (lead[u]) {
-      const uint32_t id = f.id_base + (uint32_t)(first + (uint64_t)u * 64u + lane);
-      const uint64_t at = (uint64_t)t[u] * kTileRuns;
-      if (direct[u]) {
-        tb.link[id] = ((uint64_t)len[u] << 32) | pos[u];
-        if (pos[u] == 0u) atomicOr(&tb.cnt[t[u]], kTileUncounted);
-        continue;
-      }
-      const uint32_t place = pos[u] & ~kTileUncounted;
-      if (place < kTileRuns) {
-        tb.run[at + place] = ((uint64_t)id << 32) | len[u];
-      } else {
-        const uint32_t prev = __hip_atomic_exchange(&tb.more[at + place % kTileRuns], id + 1u, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT);
-        tb.link[id] = ((uint64_t)len[u] << 32) | prev;
-      }
-    }
+    if (lead[u])
+      put_run(tb, t[u], kDirect ? pos[u] & ~kTileUncounted : pos[u],
+              f.id_base + (uint32_t)(first + (uint64_t)u * 64u + lane), run_from(starts[u]));
   }
 }
 

@@ -870,19 +870,19 @@ __device__ __forceinline__ void sort_runs(uint64_t* run, uint32_t got) {
   wave_lds_sync();
   sort_net<R>(v);
   auto swap_with = [&](uint32_t mask, uint32_t bit, bool mirror) {
-    double o[R];
     const int from = (int)((lane ^ mask) << 2);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const double x = v[r];
-      o[r] = pack2((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)hi32(x)),
+    auto other = [&](double x) {
+      return pack2((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)hi32(x)),
                    (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)lo32(x)));
-    }
+    };
     const bool low = (lane & bit) == 0u;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const double x = mirror ? o[R - 1 - r] : o[r];
-      v[r] = (x < v[r]) == low ? x : v[r];
+    for (int r = 0; r < R / 2; ++r) {
+      const int q = R - 1 - r;
+      const double x = other(v[r]), y = other(v[q]);
+      const double a = mirror ? y : x, b = mirror ? x : y;
+      v[r] = (a < v[r]) == low ? a : v[r];
+      v[q] = (b < v[q]) == low ? b : v[q];
     }
   };
 #pragma unroll 1
@@ -980,7 +980,8 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
     }
     return;
   }
-  // positions of the runs, and the tile's own fragments among them
+  // positions of the runs, and the tile's own fragments among them (or, where
+  // those are no more than cap, any number between)
   uint32_t size, frags, id0, deltas = lds_address(w.delta), cap = Lds::kEntries;
   if (m <= 64u) {
     uint32_t start = kEmpty, len = 0u;
@@ -990,14 +991,15 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
       start = (uint32_t)(rec >> 32);
       len = (uint32_t)rec;
     }
-    frags = __builtin_amdgcn_readlane(wave_scan_u32(run_own(len)), 63);
+    const uint32_t own = run_own(len);
+    len = run_len(len);
     if constexpr (kMode == kTileList) {
-      if ((frags >> split) > cap) {  // binned instead
+      if ((__builtin_amdgcn_readlane(wave_scan_u32(len), 63) >> split) > cap &&
+          (__builtin_amdgcn_readlane(wave_scan_u32(own), 63) >> split) > cap) {  // binned instead
         end_share(tb, tile, m, first, split, true, queue);
         return;
       }
     }
-    len = run_len(len);
     // the runs in ascending order of their first ids
     uint32_t rank = 0;
     for (uint32_t j = 0; j < m; ++j) rank += __builtin_amdgcn_readlane(start, j) < start ? 1u : 0u;
@@ -1005,7 +1007,8 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
     start = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)start);
     len = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)len);
     const uint32_t incl = wave_scan_u32(len);
-    size = __builtin_amdgcn_readlane(incl, 63);
+    size = frags = __builtin_amdgcn_readlane(incl, 63);
+    if (size > cap) frags = __builtin_amdgcn_readlane(wave_scan_u32(own), 63);  // (where it decides)
     id0 = rfl(start);
     clear_marks(w);
     if (size <= kMaxPositions) mark_run(w, lane < m, incl - len);  // 64 runs of at most 64: always
@@ -1027,31 +1030,36 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
       return;
     }
     cap = Lds::kEntries - (got * (uint32_t)sizeof(uint32_t) + Lds::kSize - 1u) / Lds::kSize;
-    static_assert(kManyRuns * sizeof(uint64_t) <= sizeof w.e, "the runs fit the entries' space");
     uint32_t* const delta = reinterpret_cast<uint32_t*>(&w.e[cap + 1u]);
     deltas = lds_address(delta);
     id0 = rfl((uint32_t)(run[0] >> 32));
-    // all of the runs are read before the first delta is written: the deltas
-    // lie over the last ones
-    uint64_t rec[kManyRuns / 64u];
-#pragma unroll
-    for (uint32_t c = 0; c < kManyRuns / 64u; ++c) rec[c] = c * 64u + lane < got ? run[c * 64u + lane] : 0ull;
-    clear_marks(w);
     size = frags = 0;
-#pragma unroll
-    for (uint32_t c = 0; c < kManyRuns / 64u; ++c) {
-      const bool on = c * 64u + lane < got;
-      const uint32_t len = run_len((uint32_t)rec[c]);
-      frags += __builtin_amdgcn_readlane(wave_scan_u32(run_own((uint32_t)rec[c])), 63);
-      const uint32_t incl = wave_scan_u32(len);
-      const uint32_t off = size + incl - len;
-      size += __builtin_amdgcn_readlane(incl, 63);
-      if (size <= kMaxPositions) mark_run(w, on, off);
-      if (on) delta[c * 64u + lane] = (uint32_t)(rec[c] >> 32) - off;
+#pragma unroll 1
+    for (uint32_t c = 0; c < got; c += 64u) {
+      const uint32_t word = c + lane < got ? (uint32_t)run[c + lane] : 0u;
+      size += __builtin_amdgcn_readlane(wave_scan_u32(run_len(word)), 63);
+      frags += __builtin_amdgcn_readlane(wave_scan_u32(run_own(word)), 63);
     }
     if (size > kMaxPositions) {
       end_share(tb, tile, m, first, split, true, queue);
       return;
+    }
+    clear_marks(w);
+    // from the last runs down: the deltas lie over the last ones. They take 4
+    // bytes a run at the end of a space for 8, so that a delta is behind every
+    // run of the batches before its own
+    static_assert(Lds::kEntries * Lds::kSize >= kManyRuns * sizeof(uint64_t), "the runs fit the entries' space");
+    uint32_t at_end = size;
+#pragma unroll 1
+    for (uint32_t c = (got - 1u) & ~63u;; c -= 64u) {
+      const bool on = c + lane < got;
+      const uint64_t rec = on ? run[c + lane] : 0ull;
+      const uint32_t len = run_len((uint32_t)rec), incl = wave_scan_u32(len);
+      at_end -= __builtin_amdgcn_readlane(incl, 63);
+      const uint32_t off = at_end + incl - len;
+      mark_run(w, on, off);
+      if (on) delta[c + lane] = (uint32_t)(rec >> 32) - off;
+      if (c == 0u) break;
     }
   }
   wave_lds_sync();
