@@ -22,9 +22,10 @@
 // lists in LDS in ascending id, and each lane then walks its own target's
 // list, newest fragment first (the walk order of the reference's lists,
 // oitLinkedList.frag.glsl:72,116-143).
-// Tiles with very many runs or fragments go to a queue that k_tile_deep
-// takes: the same, in groups of fragments from the newest to the oldest,
-// with the front K kept in registers. A batch's queue is taken by k_tile_bin
+// Tiles with over 1024 runs, or whose fragments would take more than two
+// passes over them, go to a queue that k_tile_deep takes: the same, in groups
+// of fragments from the newest to the oldest, with the front K kept in
+// registers. A batch's queue is taken by k_tile_bin
 // (oit_tiles.hip) and k_tile_binned: per target in order in memory, then a
 // lane per target. The line between them is what a wave's LDS holds: 696
 // fragments; read in parts beyond it, the batch took 10.3 ms against 3.6.
@@ -1040,7 +1041,13 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
       size += __builtin_amdgcn_readlane(wave_scan_u32(run_len(word)), 63);
       frags += __builtin_amdgcn_readlane(wave_scan_u32(run_own(word)), 63);
     }
-    if (size > kMaxPositions) {
+    // more than two passes over all of these runs are slower than the deep
+    // composite's groups, each fragment once for the front K and once for the
+    // tail (512x512, 2000 spheres, three in ten clustered: Loop64 K = 8 1.60
+    // ms with up to 4096 positions, 1.03 at four passes, 0.91 at three, 0.81
+    // at two; Loop32 2.10, 1.01, 0.93, 0.89). Tiles of few runs stay here at
+    // any number of passes: there are many of them where there are some.
+    if (size > kMaxPositions || frags > 2u * cap) {
       end_share(tb, tile, m, first, split, true, queue);
       return;
     }
@@ -1123,6 +1130,7 @@ struct DeepLds {
   TileLds<kDeepEntries, true> g;
   uint32_t carry[K * 64];   // the front K's colours between groups, [k][lane]
   uint64_t run[kDeepRuns];  // first id << 32 | length, ascending
+  uint32_t delta[kDeepEntries];  // per run of a group
 };
 
 // Calls body(last) for the tile's fragments group by group, the newest
@@ -1140,12 +1148,16 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
     return 1u;
   }
   uint32_t groups = 0;
-  uint64_t hi = 1ull << 32;
-  while (hi > 0u) {
-    uint64_t lo = 0;
+  const uint64_t begin = src.one.id_base;
+  uint64_t hi = begin + src.frags;
+  while (hi > begin) {
+    uint64_t lo = begin;
     if (m > kTileRuns) {  // (the lists may hold uncounted runs)
       // a window of at most kDeepRuns runs below hi: first ids differ, so a
-      // span of kDeepRuns ids is one; bisected down to a fuller one
+      // span of kDeepRuns ids is one; from there to a fuller one, every other
+      // step to where an even spread would have three quarters of kDeepRuns
+      // (halving alone walked the lists up to thirty times for each window:
+      // 1920x1080 shuffled, 21.7 M fragments, Loop64 6.59 ms, 5.44 so)
       auto count = [&](uint64_t from) {
         uint32_t c = 0;
         each_run(tb, tile, m, [&](uint32_t start, uint32_t, bool on) {
@@ -1153,15 +1165,21 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
         });
         return c;
       };
-      uint64_t bad = 0;
-      if (count(0) > kDeepRuns) {
-        uint64_t ok = hi > kDeepRuns ? hi - kDeepRuns : 0u;
+      uint64_t bad = begin;
+      uint32_t c_bad = count(bad);
+      if (c_bad > kDeepRuns) {
+        uint64_t ok = hi - kDeepRuns;  // > bad: more runs than that are between bad and hi
         uint32_t c_ok = 0;
-        while (ok - bad > 1u && c_ok < kDeepRuns / 2u) {
-          const uint64_t mid = bad + (ok - bad) / 2u;
+        for (bool spread = true; ok - bad > 1u && c_ok < kDeepRuns / 2u; spread = !spread) {
+          uint64_t mid = bad + (ok - bad) / 2u;
+          if (spread) {
+            const uint64_t at = hi - (hi - bad) * (kDeepRuns / 4u * 3u) / c_bad;
+            if (at > bad && at < ok) mid = at;
+          }
           const uint32_t c = count(mid);
           if (c > kDeepRuns) {
             bad = mid;
+            c_bad = c;
           } else {
             ok = mid;
             c_ok = c;
@@ -1173,26 +1191,31 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
     uint32_t e = load_runs<kDeepRuns>(w.run, tb, tile, m, lo, hi);
     while (e > 0u) {
       // as many of the newest runs as one group holds
-      const uint32_t len0 = lane < e ? run_len((uint32_t)w.run[e - 1u - lane]) : 0u;
-      const uint32_t sum = wave_scan_u32(len0);
-      const uint32_t r = (uint32_t)__builtin_popcountll(__ballot(lane < e && sum <= (uint32_t)kDeepEntries));
+      uint32_t r = 0, N = 0;
+      while (r < e) {
+        const uint32_t left = e - r, len = lane < left ? run_len((uint32_t)w.run[left - 1u - lane]) : 0u;
+        const uint32_t sum = N + wave_scan_u32(len);
+        const uint32_t k = (uint32_t)__builtin_popcountll(__ballot(lane < left && sum <= (uint32_t)kDeepEntries));
+        if (k > 0u) N = __builtin_amdgcn_readlane(sum, k - 1u);
+        r += k;
+        if (k < 64u) break;
+      }
       if (r == 0u) break;  // no run is longer than a group
       const uint32_t first = e - r;
-      uint32_t start = 0u, len = 0u;
-      if (lane < r) {
-        const uint64_t rec = w.run[first + lane];
-        start = (uint32_t)(rec >> 32);
-        len = run_len((uint32_t)rec);
-      }
-      const uint32_t incl = wave_scan_u32(len);
-      const uint32_t N = __builtin_amdgcn_readlane(incl, 63);
       clear_marks(w.g);
-      mark_run(w.g, lane < r, incl - len);
-      w.g.delta[lane] = start - (incl - len);
+      for (uint32_t c = 0, off = 0; c < r; c += 64u) {
+        const bool on = c + lane < r;
+        const uint64_t rec = on ? w.run[first + c + lane] : 0ull;
+        const uint32_t len = run_len((uint32_t)rec), incl = wave_scan_u32(len), at = off + incl - len;
+        mark_run(w.g, on, at);
+        if (on) w.delta[c + lane] = (uint32_t)(rec >> 32) - at;
+        off += __builtin_amdgcn_readlane(incl, 63);
+      }
+      const uint32_t id0 = rfl((uint32_t)(w.run[first] >> 32));
       wave_lds_sync();
-      (void)build_lists<kStored, true>(w.g, src, dst.tab, lds_address(w.g.delta), rfl(start), N, 6u, 0u, kDeepEntries,
+      (void)build_lists<kStored, true>(w.g, src, dst.tab, lds_address(w.delta), id0, N, 6u, 0u, kDeepEntries,
                                          (tile - dst.tile0) * kTileTargets, t, in);
-      body(first == 0u && lo == 0u);
+      body(first == 0u && lo == begin);
       ++groups;
       wave_lds_sync();
       e = first;
@@ -1565,6 +1588,7 @@ __device__ __forceinline__ void frame_views(FramePtr fr, uint32_t f, const Codec
   src.one.depth = fr[f].depth;
   src.one.rgba = fr[f].rgba;
   src.one.id_base = fr[f].frag_base;
+  src.frags = fr[f].count;
   src.T = dst.T = fr[f].T;
   dst.tile0 = fr[f].target_base / kTileTargets;
   dst.out = fr[f].out;
