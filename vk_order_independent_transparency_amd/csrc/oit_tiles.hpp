@@ -984,7 +984,7 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
   // positions of the runs, and the tile's own fragments among them (or, where
   // those are no more than cap, any number between)
   uint32_t size, frags, id0, deltas = lds_address(w.delta), cap = Lds::kEntries;
-  if (m <= 64u) {
+  if (__builtin_expect(m <= 64u, 1)) {  // (spills go to the other tiles' code: Loop64 K = 8 150 us, 147 so)
     uint32_t start = kEmpty, len = 0u;
     uint64_t rec = ahead.rec;
     if (m > kAheadRuns && lane >= kAheadRuns && lane < m) rec = tb.run[(uint64_t)tile * kTileRuns + lane];
@@ -1108,7 +1108,7 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
     else done = OIT_TILE_SIZE(32);
 #undef OIT_TILE_SIZE
     if constexpr (kMode == kTileLoop64 || kMode == kTileLoop32) {
-      if (!done) exact_composite<K, kMode, kTail, kGeneral>(L, src, dst, s_dec, s_alpha);
+      if (__builtin_expect(!done, 0)) exact_composite<K, kMode, kTail, kGeneral>(L, src, dst, s_dec, s_alpha);
     }
     wave_lds_sync();
   }
