@@ -209,8 +209,6 @@ struct TileSrc {
   uint32_t T = 0, spp = 1;        // targets and samples per pixel of the frame
   uint64_t frags = 0;             // fragments of the frame
   const uint64_t* opq = nullptr;  // opaque depth planes, or null
-  const uint64_t* cd = nullptr;   // stored payloads (depth key << 32 | packed colour) by id, and list index mod 64
-  const uint8_t* loc = nullptr;
 };
 struct TileDst {
   float4* out = nullptr;          // [T]
@@ -226,9 +224,9 @@ struct TileDst {
 // Order and tail of a composite: the Linked List (by depth, then id; evicted
 // colours blended in walk order), Loop64 (by depth, then packed colour; the
 // rest blended in id order with packed colours), Loop32 (one layer per
-// depth, the newest fragment's; the rest with full colours), the Spinlock
-// (by depth, then id; the rest in id order with packed colours).
-enum TileMode { kTileList = 0, kTileLoop64, kTileLoop32, kTileKBuf };
+// depth, the newest fragment's; the rest with full colours). The debug outputs
+// are Loop64's and Loop32's.
+enum TileMode { kTileList = 0, kTileLoop64, kTileLoop32 };
 // Pass 1 of one append.
 hipError_t launch_tile_link(const Common& c, const FragView& f, const TileBuf& tb, hipStream_t s);
 // Writes a segment table to the device (kernel arguments, no copy).

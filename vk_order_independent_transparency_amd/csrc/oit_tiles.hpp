@@ -289,7 +289,7 @@ __device__ __forceinline__ void mark_run(Lds& w, bool on, uint32_t off) {
 // `base` is the list index of the tile's first target: fragments of other
 // tiles, in a run's gaps, are in no part.
 // Returns false (wave-uniform) where the fragments are more than `cap`.
-template <bool kStored, bool kMany, typename Lds>
+template <bool kMany, typename Lds>
 __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const CodecTables* tab, uint32_t deltas,
                                             uint32_t id0, uint32_t size, uint32_t shift, uint32_t part, uint32_t cap,
                                             uint32_t base, uint32_t target, bool in) {
@@ -316,7 +316,7 @@ __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const Co
   uint32_t used = 0;  // entries so far
   // the fields of kU batches; the next kU are loaded while these are listed
   struct Fields {
-    uint32_t id, loc, key, col;
+    uint32_t id, loc;
     float4 cv;
     float dv;
     bool act;
@@ -338,18 +338,11 @@ __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const Co
     }
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
-      if constexpr (kStored) {
-        const uint64_t cd = ld_global_stream(&src.cd[f[u].id]);
-        f[u].key = (uint32_t)(cd >> 32);
-        f[u].col = (uint32_t)cd;
-        f[u].loc = ld_global_stream(&src.loc[f[u].id]);
-      } else {
-        const TileSeg s = seg_of<kMany>(src, f[u].id);
-        const uint32_t i = f[u].id - s.id_base;
-        f[u].loc = ld_global_stream(&s.target[i]);
-        f[u].dv = ld_global_stream(&s.depth[i]);
-        f[u].cv = ld_global_stream(&s.rgba[i]);
-      }
+      const TileSeg s = seg_of<kMany>(src, f[u].id);
+      const uint32_t i = f[u].id - s.id_base;
+      f[u].loc = ld_global_stream(&s.target[i]);
+      f[u].dv = ld_global_stream(&s.depth[i]);
+      f[u].cv = ld_global_stream(&s.rgba[i]);
     }
   };
   Fields ahead[kU];
@@ -364,13 +357,8 @@ __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const Co
       id[u] = ahead[u].id;
       loc[u] = ahead[u].loc;
       act[u] = ahead[u].act;
-      if constexpr (kStored) {
-        key[u] = ahead[u].key;
-        col[u] = ahead[u].col;
-      } else {
-        dv[u] = ahead[u].dv;
-        cv[u] = ahead[u].cv;
-      }
+      dv[u] = ahead[u].dv;
+      cv[u] = ahead[u].cv;
     }
     if (b + kU < nb) load(b + kU, ahead);
     // onto the targets' lists, batch after batch
@@ -383,11 +371,9 @@ __device__ __forceinline__ bool build_lists(Lds& w, const TileSrc& src, const Co
         act[u] = false;
         continue;
       }
-      if constexpr (!kStored) {
-        loc[u] = pm_index(loc[u], src.T, src.spp) - base;
-        key[u] = depth_key(dv[u]);
-        col[u] = encode_color_quick(cv[u], tab);
-      }
+      loc[u] = pm_index(loc[u], src.T, src.spp) - base;
+      key[u] = depth_key(dv[u]);
+      col[u] = encode_color_quick(cv[u], tab);
       act[u] = act[u] && (loc[u] >> shift) == part;
       if (opaque) {
         const uint32_t z = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(loc[u] << 2), (int)front);
@@ -727,14 +713,14 @@ __device__ __forceinline__ bool tile_composite(TileLane& L, const TileSrc& src, 
         if (k < F && (uint32_t)k < n && kMode != kTileLoop32) {
           const uint32_t e = key_value<kMode>(v[k < F ? k : 0]);
           key = key_depth(v[k < F ? k : 0]);
-          val = kMode == kTileLoop64 ? (uint32_t)entry_at(e).col : entry_id(e);
+          val = entry_at(e).col;
         }
         if (kMode != kTileLoop32 || (uint32_t)k >= layers) {
           if (dst.fk_key) dst.fk_key[(uint64_t)L.t * K + k] = key;
           if (dst.fk_val) dst.fk_val[(uint64_t)L.t * K + k] = val;
         }
       }
-      if (dst.counts) dst.counts[L.t] = kMode == kTileLoop32 ? layers : kMode == kTileLoop64 ? n : L.cnt;
+      if (dst.counts) dst.counts[L.t] = kMode == kTileLoop32 ? layers : n;
     }
   }
   return true;
@@ -952,7 +938,7 @@ __device__ __forceinline__ TileAhead load_ahead(const TileBuf& tb, uint32_t tile
 
 // The composite of one tile by one wave (split 0), or of the 64 >> split
 // targets from `first` on: see the head of the file.
-template <int K, int kMode, bool kTail, bool kStored, bool kGeneral, typename Lds>
+template <int K, int kMode, bool kTail, bool kGeneral, typename Lds>
 __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_t split, const TileAhead& ahead, const TileBuf& tb, const TileSrc& src,
                                           const TileDst& dst, Lds& w, const float* s_dec, const float* s_alpha,
                                           TileQueue* queue) {
@@ -1079,7 +1065,7 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
   }
   for (uint32_t t0 = first; t0 < last;) {
     const uint32_t part = t0 >> shift;
-    if (!build_lists<kStored, kGeneral>(w, src, dst.tab, deltas, id0, size, shift, part, cap, base, L.t, in)) {
+    if (!build_lists<kGeneral>(w, src, dst.tab, deltas, id0, size, shift, part, cap, base, L.t, in)) {
       wave_lds_sync();
       if (shift == 0u || kMode == kTileList) {  // one target's fragments
         end_share(tb, tile, m, first, split, true, queue);
@@ -1136,7 +1122,7 @@ struct DeepLds {
 // Calls body(last) for the tile's fragments group by group, the newest
 // first: w.g holds the group's entries (ascending) and the targets' lists.
 // `keep`: the tile has one group and its lists are still in w.g.
-template <bool kStored, typename Lds, typename F>
+template <typename Lds, typename F>
 __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const TileSrc& src, const TileDst& dst,
                                                uint32_t tile, uint32_t m, bool keep, F&& body) {
   const uint32_t list_index = (tile - dst.tile0) * kTileTargets + lane_id();
@@ -1213,7 +1199,7 @@ __device__ __forceinline__ uint32_t each_group(Lds& w, const TileBuf& tb, const 
       }
       const uint32_t id0 = rfl((uint32_t)(w.run[first] >> 32));
       wave_lds_sync();
-      (void)build_lists<kStored, true>(w.g, src, dst.tab, lds_address(w.delta), id0, N, 6u, 0u, kDeepEntries,
+      (void)build_lists<true>(w.g, src, dst.tab, lds_address(w.delta), id0, N, 6u, 0u, kDeepEntries,
                                          (tile - dst.tile0) * kTileTargets, t, in);
       body(first == 0u && lo == begin);
       ++groups;
@@ -1238,7 +1224,7 @@ struct DeepOut {
 // to `carry` and their list values past every entry's (they are newer than
 // all that follows, so they come after at equal depths; first, in Loop32's
 // order). Returns false where equal depths at the K-th need exact_deep.
-template <int K, int kMode, bool kTail, bool kStored>
+template <int K, int kMode, bool kTail>
 __device__ __forceinline__ bool sorted_deep(uint32_t tile, uint32_t m, const TileBuf& tb, const TileSrc& src,
                                             const TileDst& dst, DeepLds<K>& w, const float* s_dec,
                                             const float* s_alpha, DeepOut<K, kMode>& o) {
@@ -1257,7 +1243,7 @@ __device__ __forceinline__ bool sorted_deep(uint32_t tile, uint32_t m, const Til
   double lost = sort_key<kMode>(kEmpty, end);
   uint32_t cnt = 0;
   o.under = zero;
-  const uint32_t groups = each_group<kStored>(w, tb, src, dst, tile, m, false, [&](bool last) {
+  const uint32_t groups = each_group(w, tb, src, dst, tile, m, false, [&](bool last) {
     uint32_t p = w.g.head[lane];
     cnt += w.g.count[lane];
     while (__ballot(p != end) != 0ull) {
@@ -1289,11 +1275,8 @@ __device__ __forceinline__ bool sorted_deep(uint32_t tile, uint32_t m, const Til
   o.deep = cnt > (uint32_t)K;
   if constexpr (kMode != kTileList) {
     bool tie = o.deep && key_depth(lost) == key_depth(v[K - 1]);
-    if constexpr (kMode != kTileKBuf) {
 #pragma unroll
-      for (int k = 1; k < K; ++k)
-        tie = tie || (key_depth(v[k]) == key_depth(v[k - 1]) && key_depth(v[k]) != kEmpty);
-    }
+    for (int k = 1; k < K; ++k) tie = tie || (key_depth(v[k]) == key_depth(v[k - 1]) && key_depth(v[k]) != kEmpty);
     if (__ballot(tie) != 0ull) return false;
   }
   o.col = zero;
@@ -1309,7 +1292,7 @@ __device__ __forceinline__ bool sorted_deep(uint32_t tile, uint32_t m, const Til
       const uint32_t kth = key_depth(v[K - 1]);  // no tail entry has its depth
       float4 acc = zero;
       uint32_t behind = 0;
-      (void)each_group<kStored>(w, tb, src, dst, tile, m, groups == 1u, [&](bool) {
+      (void)each_group(w, tb, src, dst, tile, m, groups == 1u, [&](bool) {
         uint32_t q = o.deep ? w.g.head[lane] : end;
         while (__ballot(q != end) != 0ull) {
           if (q != end) {
@@ -1329,10 +1312,10 @@ __device__ __forceinline__ bool sorted_deep(uint32_t tile, uint32_t m, const Til
   return true;
 }
 
-// The same by 64-bit integer keys with the colours moved along: Loop64 by
-// (depth, colour), the others by (depth, id), Loop32 dropping a depth that it
-// already holds (its newest fragment is met first).
-template <int K, int kMode, bool kTail, bool kStored>
+// The same for Loop64 and Loop32 by 64-bit integer keys with the colours moved
+// along: Loop64 by (depth, colour), Loop32 by (depth, id) and dropping a depth
+// that it already holds (its newest fragment is met first).
+template <int K, int kMode, bool kTail>
 __device__ __forceinline__ void exact_deep(uint32_t tile, uint32_t m, uint32_t t, bool in, const TileBuf& tb,
                                            const TileSrc& src, const TileDst& dst, DeepLds<K>& w, const float* s_dec,
                                            const float* s_alpha, DeepOut<K, kMode>& o) {
@@ -1345,8 +1328,7 @@ __device__ __forceinline__ void exact_deep(uint32_t tile, uint32_t m, uint32_t t
   FrontK<K> f;
   f.init();
   uint32_t cnt = 0, held = 0;
-  o.under = zero;
-  const uint32_t groups = each_group<kStored>(w, tb, src, dst, tile, m, false, [&](bool) {
+  const uint32_t groups = each_group(w, tb, src, dst, tile, m, false, [&](bool) {
     uint32_t p = w.g.head[lane];
     cnt += w.g.count[lane];
     while (__ballot(p != end) != 0ull) {
@@ -1363,9 +1345,6 @@ __device__ __forceinline__ void exact_deep(uint32_t tile, uint32_t m, uint32_t t
       uint64_t ev = x;
       uint32_t evc = c;
       f.insert(x, c, ev, evc);
-      if constexpr (kMode == kTileList && kTail) {
-        if (on && held >= (uint32_t)K) o.under = over(o.under, decode_premult_lds(evc, s_dec, s_alpha));
-      }
       held += put ? 1u : 0u;
     }
   });
@@ -1378,7 +1357,7 @@ __device__ __forceinline__ void exact_deep(uint32_t tile, uint32_t m, uint32_t t
     if ((uint32_t)k < o.n) o.col = over(o.col, decode_premult_lds(f.col[k], s_dec, s_alpha));
   o.tail = zero;
   o.tails = 0;
-  if constexpr (kTail && kMode != kTileList) {
+  if constexpr (kTail) {
     if (__ballot(o.deep) != 0ull) {
       const uint64_t kth = f.sk[K - 1];
       float4 acc = zero;
@@ -1387,7 +1366,7 @@ __device__ __forceinline__ void exact_deep(uint32_t tile, uint32_t m, uint32_t t
         acc = zero;
         behind = 0;
         uint32_t left = keep;
-        (void)each_group<kStored>(w, tb, src, dst, tile, m, groups == 1u, [&](bool) {
+        (void)each_group(w, tb, src, dst, tile, m, groups == 1u, [&](bool) {
           uint32_t q = o.deep ? w.g.head[lane] : end;
           while (__ballot(q != end) != 0ull) {
             if (q != end) {
@@ -1427,13 +1406,12 @@ __device__ __forceinline__ void exact_deep(uint32_t tile, uint32_t m, uint32_t t
       const bool on = (uint32_t)k < o.n;
       if (dst.fk_key) dst.fk_key[(uint64_t)t * K + k] = on ? (uint32_t)(f.sk[k] >> 32) : kEmpty;
       if (dst.fk_val)
-        dst.fk_val[(uint64_t)t * K + k] =
-            !on ? kEmpty : (kMode == kTileLoop32 || kMode == kTileLoop64) ? f.col[k] : (uint32_t)f.sk[k];
+        dst.fk_val[(uint64_t)t * K + k] = on ? f.col[k] : kEmpty;
     }
   }
 }
 
-template <int K, int kMode, bool kTail, bool kStored>
+template <int K, int kMode, bool kTail>
 __device__ __forceinline__ void deep_wave(uint32_t tile, uint32_t shares, uint32_t split, const TileBuf& tb, const TileSrc& src, const TileDst& dst,
                                           DeepLds<K>& w, const float* s_dec, const float* s_alpha) {
   const uint32_t lane = lane_id();
@@ -1442,10 +1420,14 @@ __device__ __forceinline__ void deep_wave(uint32_t tile, uint32_t shares, uint32
   const uint32_t t = in ? pm_target(a, dst.T, dst.spp) : 0u;
   const uint32_t m = rfl(tb.cnt[tile]);
   DeepOut<K, kMode> o;
-  // the sorted front K of a deep tile keeps no ids: asked for them, the integer form runs
-  bool done = false;
-  if (!(dst.fk_key || dst.fk_val)) done = sorted_deep<K, kMode, kTail, kStored>(tile, m, tb, src, dst, w, s_dec, s_alpha, o);
-  if (!done) exact_deep<K, kMode, kTail, kStored>(tile, m, t, in, tb, src, dst, w, s_dec, s_alpha, o);
+  if constexpr (kMode == kTileList) {
+    (void)sorted_deep<K, kMode, kTail>(tile, m, tb, src, dst, w, s_dec, s_alpha, o);
+  } else {
+    // the debug outputs, too, are the integer form's
+    bool done = false;
+    if (!(dst.fk_key || dst.fk_val)) done = sorted_deep<K, kMode, kTail>(tile, m, tb, src, dst, w, s_dec, s_alpha, o);
+    if (!done) exact_deep<K, kMode, kTail>(tile, m, t, in, tb, src, dst, w, s_dec, s_alpha, o);
+  }
   float4 d = dst.background;
   if (dst.rgba && in) d = dst.rgba[t];
   if constexpr (kTail && kMode != kTileList) {
@@ -1457,7 +1439,7 @@ __device__ __forceinline__ void deep_wave(uint32_t tile, uint32_t shares, uint32
   if (!in) return;
   if constexpr (kMode == kTileList) o.col = over(o.col, o.under);
   dst.out[t] = over(o.col, d);
-  if (dst.counts) dst.counts[t] = (kMode == kTileLoop32 || kMode == kTileLoop64) ? o.n : o.cnt;
+  if (dst.counts) dst.counts[t] = o.n;
 }
 
 // ---------------------------------------------------------------------------
@@ -1507,7 +1489,7 @@ __device__ __forceinline__ const TileArgs& fresh_args() {
   return *(const TileArgs*)p;
 }
 
-template <int K, int kMode, bool kTail, bool kStored, bool kGeneral>
+template <int K, int kMode, bool kTail, bool kGeneral>
 __global__ __launch_bounds__(kBlock, tile_waves<K>()) void k_tile_resolve(TileArgs args) {
   constexpr bool kId = kGeneral || kMode == kTileLoop32;
   __shared__ float s_dec[256];
@@ -1527,13 +1509,13 @@ __global__ __launch_bounds__(kBlock, tile_waves<K>()) void k_tile_resolve(TileAr
     const TileArgs& g = fresh_args();
     const TileAhead next = load_ahead(g.tb, (item + stride) >> split, tiles);
     const uint32_t first = (item & ((1u << split) - 1u)) << (6u - split);
-    tile_wave<K, kMode, kTail, kStored, kGeneral>(item >> split, first, split, now, g.tb, g.src, g.dst, s_w[wave],
+    tile_wave<K, kMode, kTail, kGeneral>(item >> split, first, split, now, g.tb, g.src, g.dst, s_w[wave],
                                                   s_dec, s_alpha, nullptr);
     now = next;
   }
 }
 
-template <int K, int kMode, bool kTail, bool kStored>
+template <int K, int kMode, bool kTail>
 __global__ __launch_bounds__(64) void k_tile_deep(TileArgs args) {
   const uint32_t n = rfl(ld_relaxed(&args.tb.ctl[args.tb.ctl_index]));
   if (blockIdx.x >= n) return;
@@ -1554,7 +1536,7 @@ __global__ __launch_bounds__(64) void k_tile_deep(TileArgs args) {
     const uint32_t entry = rfl(g.tb.deep[g.tb.deep_base + q]);
     const uint32_t tile = g.split ? g.tb.tile_first + (entry & 0xFFFFu) : entry;
     const uint32_t shares = g.split ? entry >> 16 : 1u;
-    deep_wave<K, kMode, kTail, kStored>(tile, shares, g.split, g.tb, g.src, g.dst, w, s_dec, s_alpha);
+    deep_wave<K, kMode, kTail>(tile, shares, g.split, g.tb, g.src, g.dst, w, s_dec, s_alpha);
     wave_lds_sync();
   }
 }
@@ -1621,7 +1603,7 @@ __global__ __launch_bounds__(kBlock, tile_waves<K>()) void k_tile_batch(TileBatc
     TileDst dst;
     frame_views(fr, f, g.tab, src, dst);
     const uint32_t first = (item & ((1u << split) - 1u)) << (6u - split);
-    tile_wave<K, kTileList, kTail, false, false>(item >> split, first, split, now, g.tb, src, dst, s_w[wave], s_dec,
+    tile_wave<K, kTileList, kTail, false>(item >> split, first, split, now, g.tb, src, dst, s_w[wave], s_dec,
                                                  s_alpha, &queue);
     now = next;
   }
@@ -1792,7 +1774,7 @@ __global__ __launch_bounds__(64) void k_tile_batch_deep(TileBatchArgs args) {
     TileSrc src;
     TileDst dst;
     frame_views(fr, rfl(find_frame<true>(g.frames, g.f0, g.f1, (uint64_t)tile * kTileTargets)), g.tab, src, dst);
-    deep_wave<K, kTileList, kTail, false>(tile, 1u, 0u, g.tb, src, dst, w, s_dec, s_alpha);
+    deep_wave<K, kTileList, kTail>(tile, 1u, 0u, g.tb, src, dst, w, s_dec, s_alpha);
     wave_lds_sync();
   }
 }
@@ -1852,7 +1834,7 @@ struct TileBatch {
 
 template <int K>
 struct TileResolve {
-  template <int kMode, bool kTail, bool kStored>
+  template <int kMode, bool kTail>
   static hipError_t go(const TileBuf& tb, const TileSrc& src, const TileDst& dst, hipStream_t s) {
     const uint32_t tiles = (dst.T + kTileTargets - 1u) / kTileTargets;
     const uint32_t fit = kComputeUnits * (uint32_t)tile_waves<K>();  // blocks resident at once
@@ -1864,25 +1846,25 @@ struct TileResolve {
     const uint32_t most = 3u * fit;
     const dim3 g(want < most ? want : most), b(kBlock);
     // kGeneral: several segments, or the debug outputs
-    const bool dbg = dst.fk_key || dst.fk_val || dst.counts || (!kStored && src.nseg > 1u);
+    const bool dbg = dst.fk_key || dst.fk_val || dst.counts || src.nseg > 1u;
     const TileArgs args{tb, src, dst, tiles, split};
-    if (dbg) hipLaunchKernelGGL((k_tile_resolve<K, kMode, kTail, kStored, true>), g, b, 0, s, args);
-    else hipLaunchKernelGGL((k_tile_resolve<K, kMode, kTail, kStored, false>), g, b, 0, s, args);
+    if (dbg) hipLaunchKernelGGL((k_tile_resolve<K, kMode, kTail, true>), g, b, 0, s, args);
+    else hipLaunchKernelGGL((k_tile_resolve<K, kMode, kTail, false>), g, b, 0, s, args);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || src.frags == 0u) return e;
     const uint32_t blocks = tiles < kDeepBlocks ? tiles : kDeepBlocks;
-    hipLaunchKernelGGL((k_tile_deep<K, kMode, kTail, kStored>), dim3(blocks), dim3(64), 0, s, args);
+    hipLaunchKernelGGL((k_tile_deep<K, kMode, kTail>), dim3(blocks), dim3(64), 0, s, args);
     return hipGetLastError();
   }
-  template <int kMode, bool kStored>
+  template <int kMode>
   static hipError_t tail_or_not(const TileBuf& tb, const TileSrc& src, const TileDst& dst, bool tail, hipStream_t s) {
-    return tail ? go<kMode, true, kStored>(tb, src, dst, s) : go<kMode, false, kStored>(tb, src, dst, s);
+    return tail ? go<kMode, true>(tb, src, dst, s) : go<kMode, false>(tb, src, dst, s);
   }
   static hipError_t run(const TileBuf& tb, const TileSrc& src, const TileDst& dst, int mode, bool tail,
                         hipStream_t s) {
     switch (mode) {
-      case kTileLoop64: return tail_or_not<kTileLoop64, false>(tb, src, dst, tail, s);
-      case kTileLoop32: return tail_or_not<kTileLoop32, false>(tb, src, dst, tail, s);
+      case kTileLoop64: return tail_or_not<kTileLoop64>(tb, src, dst, tail, s);
+      case kTileLoop32: return tail_or_not<kTileLoop32>(tb, src, dst, tail, s);
       default: return hipErrorInvalidValue;
     }
   }
