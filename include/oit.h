@@ -351,7 +351,12 @@ enum {
  * a list or a bucket per target; with the defaults and no
  * OIT_VARIANT_BATCH_LISTS in any resolve_variant a batch composites tiles of
  * 64 targets from the fragments themselves (lists where there is no memory
- * for those, until the tuning is set again). */
+ * for those, until the tuning is set again). Tiles are the faster where
+ * fragments come in raster order and layers are uneven, lists where the order
+ * is another: three 1920x1080 frames (K = 8, 16, 32) of 12.8 M fragments take
+ * 0.64 ms either way in raster order, 0.88 and 1.31 with three spheres in ten
+ * clustered, 0.84 and 0.69 in blocks of 8x8 pixels, 8.9 and 4.0 shuffled.
+ * oit_batch_tune finds out. */
 typedef struct oit_batch_tuning {
   uint32_t append_chunks;
   uint32_t resolve_variant[6][2];
