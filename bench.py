@@ -149,15 +149,13 @@ ALGORITHM_ROWS = ((1, "linkedlist", 8), (1, "linkedlist", 16), (3, "loop64", 8),
                   (5, "interlock", 16))
 
 
-def bench_algorithms(tg_d, d_d, c_d, F, p, steps, stream, only=None, variant=0, counts=None):
+def bench_algorithms(tg_d, d_d, c_d, F, p, steps, stream, only=None, variant=0):
     """Every algorithm on the same 1920x1080 stream (Linked List pool 1.5F,
     tail blending on): device time per frame, G fragments/s and the
     fraction of the HBM roofline by the algorithm's compulsory bytes.
-    `only`: a set of "name:K" strings to restrict the rows to. `counts`:
-    fragments per target (host), for the slots the composites touch."""
+    `only`: a set of "name:K" strings to restrict the rows to."""
     from vk_order_independent_transparency_amd import DeviceBuffer, Event, FrameConfig, Renderer
     from vk_order_independent_transparency_amd import roofline as rl
-    import numpy as np
 
     P = p.targets
     out = DeviceBuffer((P, 4), "float32")
@@ -181,14 +179,10 @@ def bench_algorithms(tg_d, d_d, c_d, F, p, steps, stream, only=None, variant=0, 
             ms = e0.elapsed_ms(e1) / steps
         if alg == 1:
             nbytes = rl.ll_frame_bytes_reference(F, P)
-        elif alg == 3:
-            occ = None if counts is None else int(np.minimum(counts, K).sum())
-            nbytes = sum(rl.loop64_stage_bytes(F, P, K, occupied=occ).values())
+        elif alg in (2, 3):
+            nbytes = sum(rl.tile_stage_bytes(F, P).values())
         elif alg in (0, 4):
             nbytes = sum(rl.kbuffer_stage_bytes(F, P, K, alg == 4).values())
-        elif alg == 2:
-            occ = None if counts is None else int(np.minimum(counts, K).sum())
-            nbytes = sum(rl.loop32_stage_bytes(F, P, K, occupied=occ).values())
         elif alg == 5:
             nbytes = sum(rl.interlock_stage_bytes(F, P).values())
         else:
@@ -534,9 +528,8 @@ def main():
     st = r.stats(stream)
     r.close()
     only = {x.strip() for x in args.only_algorithms.split(",") if x.strip()}
-    counts = np.bincount(tg[tg < P].astype(np.int64), minlength=P)  # fragments per target
     algorithms = None if args.no_algorithms else bench_algorithms(tg_d, d_d, c_d, F, p, args.algorithm_steps, stream,
-                                                                  only, args.variant, counts)
+                                                                  only, args.variant)
 
     frames_4k = None if args.no_4k else bench_4k_4x(10, args.variant)
     batch = None if args.no_batch else bench_batch(1, args.batch_frames)
