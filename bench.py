@@ -252,7 +252,7 @@ def bench_batch(seed, frames_n, resolutions=(256, 512, 1024, 2048)):
     import numpy as np
 
     from vk_order_independent_transparency_amd import (Batch, BatchFrame, DeviceBuffer, Event, FrameConfig,
-                                                       OIT_LINKEDLIST, Renderer, Stream, scene)
+                                                       OIT_LINKEDLIST, Renderer, Stream, _abi, scene)
 
     work = scene.batch_workload(seed, frames_n, resolutions)
     st = Stream()
@@ -315,16 +315,21 @@ def bench_batch(seed, frames_n, resolutions=(256, 512, 1024, 2048)):
         b.close()
         return min(runs), ok, t
 
-    order_ms, order_ok, _ = timed(True)
     bat_ms, exact, t = timed(False)
-    exact = exact and order_ok
-    log(f"batch frame after frame: {order_ms:.3f} ms, interleaved: {bat_ms:.3f} ms")
+    # the append schedules differ where the tuner has taken lists
+    lists = any(v & _abi.VARIANT_BATCH_LISTS for k in t.resolve_variant for v in k)
+    order_ms = None
+    if lists:
+        order_ms, order_ok, _ = timed(True)
+        exact = exact and order_ok
+        log(f"batch frame after frame: {order_ms:.3f} ms, interleaved: {bat_ms:.3f} ms")
     log(f"batch: sequential {seq_ms:.3f} ms, batched {bat_ms:.3f} ms, {seq_ms / bat_ms:.2f}x, bit-exact {exact}")
     sizes = "" if tuple(resolutions) == (256, 512, 1024, 2048) else "_" + "_".join(str(r) for r in resolutions)
     return {"workload": f"batch_{len(frames)}_frames_seed{seed}{sizes}", "frames": len(frames), "fragments": total,
             "sequential_ms": round(seq_ms, 4), "batched_ms": round(bat_ms, 4),
             "speedup": round(seq_ms / bat_ms, 3), "G_fragments_per_s": round(total / bat_ms / 1e6, 3),
-            "frame_order_ms": round(order_ms, 4),
+            "path": "lists" if lists else "tiles",
+            "frame_order_ms": None if order_ms is None else round(order_ms, 4),
             "bit_exact_vs_sequential": bool(exact), "append_chunks": int(t.append_chunks),
             "bin_density": float(t.bin_density),
             "binned_frames": sum(1 for f in frames if f.count >= t.bin_density * f.width * f.height * f.samples
