@@ -138,7 +138,7 @@ struct oit_ctx {
   bool resolved = false;
   uint64_t frame_frags = 0;
   uint64_t appends = 0;
-  std::vector<oit::FragView> segments;
+  std::vector<oit::TileSeg> segments;  // Loop32, Loop64: the appends of the frame
   // sizes
   uint64_t bytes_abuf = 0, bytes_aux = 0;
   // allocated elements of each frame buffer: a reconfiguration reuses a
@@ -1049,9 +1049,13 @@ int oit_append(oit_ctx* c, const oit_fragments* f, void* stream) {
         rc = reserve(c, &c->tile_segs, &c->cap_tile_segs, want);
       }
       if (rc) return rc;
+      try {
+        c->segments.push_back({v.target, v.depth, v.rgba, v.id_base, 0u});
+      } catch (const std::bad_alloc&) {
+        return OIT_ERR_OOM;
+      }
       c->tile_clean = false;
       e = staged(c, kStStore, s, [&] { return oit::launch_tile_link(k, v, tiles_of(c), s); });
-      c->segments.push_back(v);
       break;
     }
     case OIT_SIMPLE: {
@@ -1156,8 +1160,7 @@ int oit_resolve_debug(oit_ctx* c, float* out_rgba, uint32_t* fk_key, uint32_t* f
       src.spp = k.spp;
       src.frags = c->frame_frags;
       src.opq = k.opq_z;
-      std::vector<oit::TileSeg> segs;
-      for (const auto& v : c->segments) segs.push_back({v.target, v.depth, v.rgba, v.id_base, 0u});
+      const std::vector<oit::TileSeg>& segs = c->segments;
       if (!segs.empty()) src.one = segs[0];
       if (segs.size() > 1) {
         src.nseg = (uint32_t)segs.size();
