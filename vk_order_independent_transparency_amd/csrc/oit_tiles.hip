@@ -18,7 +18,7 @@ namespace {
 // front and four back fragments needs. Chunks of few runs, as raster order
 // leaves them, are not looked through, and the code is kept small: unrolled
 // over lanes and chunks it took them 23.5 us instead of 22.
-constexpr int kManyStarts = 12;  // runs of a chunk from which gaps are looked for
+constexpr int kManyStarts = 15;  // runs of a chunk past which gaps are looked for: spheres of a pixel or two make up to 14
 constexpr uint32_t kGap = 8;    // (join_gaps' shifts go by it)
 constexpr int kGapTiles = 16;
 // A chunk that is still of more than kDirectRuns runs puts them on the tiles'

@@ -1027,13 +1027,17 @@ __device__ __forceinline__ void tile_wave(uint32_t tile, uint32_t first, uint32_
       size += __builtin_amdgcn_readlane(wave_scan_u32(run_len(word)), 63);
       frags += __builtin_amdgcn_readlane(wave_scan_u32(run_own(word)), 63);
     }
-    // more than two passes over all of these runs are slower than the deep
-    // composite's groups, each fragment once for the front K and once for the
-    // tail (512x512, 2000 spheres, three in ten clustered: Loop64 K = 8 1.60
-    // ms with up to 4096 positions, 1.03 at four passes, 0.91 at three, 0.81
-    // at two; Loop32 2.10, 1.01, 0.93, 0.89). Tiles of few runs stay here at
-    // any number of passes: there are many of them where there are some.
-    if (size > kMaxPositions || frags > 2u * cap) {
+    // Many passes over all of these runs are slower than the deep composite's
+    // groups, each fragment once for the front K and once for the tail
+    // (512x512, 2000 spheres, three in ten clustered, a tile for two waves:
+    // Loop64 K = 8 1.60 ms with up to 4096 positions here, 1.03 with up to four
+    // times what the LDS holds, 0.92 with three times; Loop32 2.10, 1.02 at
+    // four; 1920x1080 in blocks of 8x8 pixels, a tile for a wave: Loop32 0.31
+    // at three times, 0.37 at two). Where four or eight waves share a tile
+    // there are few tiles, and one wave's groups are the longer way (181x89,
+    // 718 spheres: Loop64 K = 8 61 us so, 118 with groups).
+    const uint32_t most = split + (kMode == kTileLoop32 ? 3u : 2u);
+    if (size > kMaxPositions || (split < 2u && frags > most * cap)) {
       end_share(tb, tile, m, first, split, true, queue);
       return;
     }
