@@ -842,9 +842,11 @@ __device__ __forceinline__ void each_run(const TileBuf& tb, uint32_t tile, uint3
 // sort keys are. Bound by its 21 exchanges between lanes of R values each; in
 // LDS, 512 runs took 45 steps of four exchanges, one waiting for the other
 // (1920x1080 shuffled, about 400 runs a tile: Loop64 4.30 ms so, 3.10 in
-// registers; 256x256: 464 and 272 us).
+// registers; 256x256: 464 and 272 us). A function of its own: inlined, its
+// registers and code cost the composite of the common tiles two per cent
+// (1368x978, Loop64 K = 16: 44.5 us, 43.7 so).
 template <int R>
-__device__ __forceinline__ void sort_runs(uint64_t* run, uint32_t got) {
+__device__ __attribute__((noinline)) void sort_runs(uint64_t* run, uint32_t got) {
   const uint32_t lane = lane_id();
   double v[R];
 #pragma unroll
