@@ -354,8 +354,9 @@ enum {
  * for those, until the tuning is set again). Tiles are the faster where
  * fragments come in raster order and layers are uneven, lists where the order
  * is another: three 1920x1080 frames (K = 8, 16, 32) of 12.8 M fragments take
- * 0.64 ms either way in raster order, 0.88 and 1.31 with three spheres in ten
- * clustered, 0.84 and 0.69 in blocks of 8x8 pixels, 8.9 and 4.0 shuffled.
+ * 0.60 ms with tiles and 0.64 with lists in raster order, 0.87 and 1.31 with
+ * three spheres in ten clustered, 0.79 and 0.69 in blocks of 8x8 pixels, 8.6
+ * and 4.0 shuffled.
  * oit_batch_tune finds out. */
 typedef struct oit_batch_tuning {
   uint32_t append_chunks;

@@ -13,8 +13,8 @@ namespace {
 // other tiles in between, which the composite drops. A rasteriser that walks
 // triangles in 2x2 quads alternates between two rows, so that a chunk is two
 // runs so and up to 32 without (1920x1080 in quads, 12.7 M fragments: Loop64
-// K = 8 502 us without, 286 with, 310 with an atomic per fragment; K = 16 518,
-// 303, 247; Loop32 588, 342, 358). The gap is as long as what a quad of four
+// K = 8 502 us without, 276 with, 310 with an atomic per fragment; K = 16 518,
+// 290, 247; Loop32 588, 336, 358). The gap is as long as what a quad of four
 // front and four back fragments needs. Chunks of few runs, as raster order
 // leaves them, are not looked through, and the code is kept small: unrolled
 // over lanes and chunks it took them 23.5 us instead of 22.

@@ -30,7 +30,7 @@
 // lane per target. The line between them is what a wave's LDS holds: 696
 // fragments; read in parts beyond it, the batch took 10.3 ms against 3.6.
 //
-// Measured (composite alone): 1920x1080 Loop64 K = 8, 12.7 M fragments, 143
+// Measured (composite alone): 1920x1080 Loop64 K = 8, 12.7 M fragments, 147
 // us, where counting, storing, classifying and compositing per target took
 // 290; 1600x900 Loop32 K = 16, 8.8 M, 175 us against 290. While resident, the
 // waves keep the vector units about 80 % busy; the rest is uneven tiles.
