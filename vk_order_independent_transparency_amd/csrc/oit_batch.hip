@@ -931,14 +931,15 @@ int oit_batch_tune(oit_batch* b, const oit_batch_frame* frames, uint32_t n, void
   b->tuning = lists ? best : default_tuning();
   b->no_tile_memory = false;
   ++b->tuning_version;
+  if (lists)
+    for (auto& k : b->tuning.resolve_variant)
+      for (uint32_t& v : k) v |= OIT_VARIANT_BATCH_LISTS;
+  if ((rc = st(hipDeviceSynchronize()))) return rc;  // earlier runs, on any stream, have ended
   if (b->gexec) {  // its launches hold pointers of either path
     (void)hipGraphExecDestroy(b->gexec);
     b->gexec = nullptr;
   }
-  if ((rc = st(hipStreamSynchronize(s)))) return rc;
   if (lists) {
-    for (auto& k : b->tuning.resolve_variant)
-      for (uint32_t& v : k) v |= OIT_VARIANT_BATCH_LISTS;
     drop_tiles(b);
   } else {
     drop_pool(b);

@@ -22,12 +22,11 @@
 // lists in LDS in ascending id, and each lane then walks its own target's
 // list, newest fragment first (the walk order of the reference's lists,
 // oitLinkedList.frag.glsl:72,116-143).
-// Tiles with over 1024 runs, or whose fragments would take more than two
-// passes over them, go to a queue that k_tile_deep takes: the same, in groups
-// of fragments from the newest to the oldest, with the front K kept in
-// registers. A batch's queue is taken by k_tile_bin
-// (oit_tiles.hip) and k_tile_binned: per target in order in memory, then a
-// lane per target. The line between them is what a wave's LDS holds: 696
+// Tiles with over 1024 runs, or of many runs that would be read more often
+// than pays, go to a queue that k_tile_deep takes: the same, in groups of
+// fragments from the newest to the oldest, with the front K kept in
+// registers. A batch's queue is taken by k_tile_bin (oit_tiles.hip) and
+// k_tile_binned: per target in order in memory, then a lane per target. The line between them is what a wave's LDS holds: 696
 // fragments; read in parts beyond it, the batch took 10.3 ms against 3.6.
 //
 // Measured (composite alone): 1920x1080 Loop64 K = 8, 12.7 M fragments, 147
