@@ -30,17 +30,18 @@ def test_queue_entries_are_written_once():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("layers,tail", [(4, 1), (16, 1), (32, 0)])
-def test_many_deep_tiles_of_an_unshared_group(oracle, layers, tail):
-    """Over 8192 tiles in the group, so that a wave takes whole tiles and an
-    entry is a tile's number; 400 of them have 30 to 1400 runs of one fragment,
-    on both sides of what the binning sorts (1024). Bit-exact: the image is a
-    function of integer keys and of the oracle's float expressions."""
+@pytest.mark.parametrize("W,H,tiles", [(800, 680, 300), (160, 136, 60)], ids=["unshared", "shared"])
+def test_many_deep_tiles(oracle, W, H, tiles, layers, tail):
+    """8500 tiles in the group, where a wave takes whole tiles and an entry is
+    a tile's number, and 340, which several waves share, where it also
+    holds the shares that were left; some of them have 30 to 2500 runs of one
+    fragment, on both sides of what the binning sorts (2048). Bit-exact: the
+    image is a function of integer keys and of the oracle's float expressions."""
     from vk_order_independent_transparency_amd import Batch, BatchFrame, DeviceBuffer, Stream
 
     rng = np.random.default_rng(layers)
-    W, H, tiles = 800, 680, 400  # 8500 tiles
-    runs = rng.choice([30, 300, 700, 1023, 1024, 1025, 1200, 1400], tiles)
-    which = rng.permutation(8500)[:tiles]
+    runs = rng.choice([30, 300, 1023, 1025, 1400, 2047, 2048, 2049, 2500], tiles)
+    which = rng.permutation(W * H // 64)[:tiles]
     # round r: one fragment on every tile that still has one, so each is a run of its own
     tile = np.concatenate([which[runs > r] for r in range(int(runs.max()))])
     assert (tile[1:] != tile[:-1]).all()
